@@ -546,8 +546,15 @@ __global__ void __launch_bounds__(kBlock) k_gnn_heads_bwd(int nV, const int* __r
     dh[id] = acc;
 }
 
-// per-workgroup records of the head weight gradients [W_o (4x80), b_o, W_d (3x32), b_d]
-__global__ void __launch_bounds__(512) k_gnn_heads_wgrad(int E, int nV, const int* __restrict__ eu,
+// Per-workgroup records of the head weight gradients [W_o (4x80), b_o, W_d (3x32), b_d]: thread j owns entry j
+// and sums it over the workgroup's tiles of 64 edges, then of 64 vertices. Bound by the latency of the gathers (each
+// edge's two h rows and its features), so a tile's rows are staged in LDS by all threads at once and the products
+// run from there (gradient entry broadcast, input columns consecutive: no bank conflicts). 15 workgroups whose
+// threads walked 2,000 edges one after another took 513 us at 10k faces (30k edges); one tile per workgroup, up to
+// kGnnMaxGrid, takes 14 us.
+constexpr int kHeadTile = 64, kHeadThreads = 512;
+constexpr int kHeadIn = 2 * kGnnH + kGnnNEs;  // staged inputs of an edge: h_u | h_w | features (the rest are zero)
+__global__ void __launch_bounds__(kHeadThreads) k_gnn_heads_wgrad(int E, int nV, const int* __restrict__ eu,
                                                          const int* __restrict__ ew, const float* __restrict__ ef,
                                                          const float* __restrict__ h,
                                                          const unsigned char* __restrict__ fixed,
@@ -555,41 +562,73 @@ __global__ void __launch_bounds__(512) k_gnn_heads_wgrad(int E, int nV, const in
                                                          const float4* __restrict__ dGd,
                                                          const float4* __restrict__ dGo, float* part)
 {
+    __shared__ float X[kHeadTile][kHeadIn + 1];
+    __shared__ float D[4][kHeadTile];
     const int j = threadIdx.x;
-    if (j >= kWStrideHead) return;
     float acc = 0.0f;
-    if (j < 4 * kGnnKM + 4) {
-        long e0, e1;
-        chunk(E, e0, e1);
-        const int i = j < 4 * kGnnKM ? j / kGnnKM : j - 4 * kGnnKM;
-        const int k = j < 4 * kGnnKM ? j % kGnnKM : -1;
-        for (long e = e0; e < e1; ++e) {
-            const int u = eu[e], w = ew[e];
-            if (w > u) continue;
-            const float4 d = dGo[e];
-            const float di = i == 0 ? d.x : (i == 1 ? d.y : (i == 2 ? d.z : d.w));
-            float x = 1.0f;
-            if (k >= 0)
-                x = k < kGnnH ? h[(size_t)u * kGnnH + k]
-                              : (k < 2 * kGnnH ? h[(size_t)w * kGnnH + k - kGnnH]
-                                               : (k < 2 * kGnnH + kGnnNEs ? ef[(size_t)e * kGnnNEs + k - 2 * kGnnH]
-                                                                          : 0.0f));
-            acc += di * x;
-        }
-    } else {
-        long u0, u1;
-        chunk(nV, u0, u1);
-        const int jj = j - (4 * kGnnKM + 4);
-        const int i = jj < 3 * kGnnH ? jj / kGnnH : jj - 3 * kGnnH;
-        const int k = jj < 3 * kGnnH ? jj % kGnnH : -1;
-        for (long u = u0; u < u1; ++u) {
-            if (fixed[u]) continue;
-            const float4 g = Gd[u], dg = dGd[u];
-            const float dd = i == 0 ? dg.x * g.x : (i == 1 ? dg.z : dg.w * g.w);
-            acc += dd * (k >= 0 ? h[(size_t)u * kGnnH + k] : 1.0f);
+    {
+        const int i = j < 4 * kGnnKM ? j / kGnnKM : (j - 4 * kGnnKM) & 3;
+        const int k = j < 4 * kGnnKM ? j % kGnnKM : kHeadIn;  // column kHeadIn holds 1 (the bias)
+        const bool mine = j < 4 * kGnnKM + 4 && (k <= kHeadIn);
+        for (long base = (long)blockIdx.x * kHeadTile; base < E; base += (long)gridDim.x * kHeadTile) {
+            __syncthreads();
+            // unrolled, so that a thread's gathers are in flight together
+#pragma unroll
+            for (int t = 0; t < (kHeadTile * (kHeadIn + 1) + kHeadThreads - 1) / kHeadThreads; ++t) {
+                const int q = j + t * kHeadThreads, r = q / (kHeadIn + 1), c = q % (kHeadIn + 1);
+                if (r >= kHeadTile) break;
+                const long e = base + r;
+                float x = 0.0f;
+                if (e < E)
+                    x = c < kGnnH ? h[(size_t)eu[e] * kGnnH + c]
+                                  : (c < 2 * kGnnH ? h[(size_t)ew[e] * kGnnH + c - kGnnH]
+                                                   : (c < kHeadIn ? ef[(size_t)e * kGnnNEs + c - 2 * kGnnH] : 1.0f));
+                X[r][c] = x;
+            }
+            if (j < kHeadTile) {
+                const long e = base + j;
+                const float4 d = e < E && ew[e] < eu[e] ? dGo[e] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                D[0][j] = d.x;
+                D[1][j] = d.y;
+                D[2][j] = d.z;
+                D[3][j] = d.w;
+            }
+            __syncthreads();
+            // inputs kHeadIn.. of W_o are zero: their entries stay 0 (k == kHeadIn is b_o's column of ones)
+            if (mine && (j >= 4 * kGnnKM || k < kHeadIn))
+#pragma unroll 8
+                for (int r = 0; r < kHeadTile; ++r) acc += D[i][r] * X[r][k];
         }
     }
-    part[(size_t)blockIdx.x * kWStrideHead + j] = acc;
+    {
+        const int jj = j - (4 * kGnnKM + 4);
+        const int i = jj < 3 * kGnnH ? jj / kGnnH : jj - 3 * kGnnH;
+        const int k = jj < 3 * kGnnH ? jj % kGnnH : kGnnH;
+        for (long base = (long)blockIdx.x * kHeadTile; base < nV; base += (long)gridDim.x * kHeadTile) {
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < (kHeadTile * (kGnnH + 1) + kHeadThreads - 1) / kHeadThreads; ++t) {
+                const int q = j + t * kHeadThreads, r = q / (kGnnH + 1), c = q % (kGnnH + 1);
+                if (r >= kHeadTile) break;
+                const long u = base + r;
+                X[r][c] = u < nV ? (c < kGnnH ? h[(size_t)u * kGnnH + c] : 1.0f) : 0.0f;
+            }
+            if (j < kHeadTile) {
+                const long u = base + j;
+                const bool on = u < nV && !fixed[u];
+                const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                const float4 g = on ? Gd[u] : zero, dg = on ? dGd[u] : zero;
+                D[0][j] = dg.x * g.x;
+                D[1][j] = dg.z;
+                D[2][j] = dg.w * g.w;
+            }
+            __syncthreads();
+            if (jj >= 0 && j < kWStrideHead)
+#pragma unroll 8
+                for (int r = 0; r < kHeadTile; ++r) acc += D[i][r] * X[r][k];
+        }
+    }
+    if (j < kWStrideHead) part[(size_t)blockIdx.x * kWStrideHead + j] = acc;
 }
 
 // Update-layer backward on 32-vertex tiles: dZ = dh * [R > 0];
@@ -793,36 +832,64 @@ __global__ void __launch_bounds__(kBlock) k_gnn_scatter_dh(int nV, const int* __
     dh[id] += acc;
 }
 
-// records of the encoder gradients [W_enc (32x4), b_enc]
+// Records of the encoder gradients [W_enc (32x4), b_enc], tiles of 64 vertices staged in LDS as in
+// k_gnn_heads_wgrad (6 workgroups walking 900 vertices each took 474 us at 10k faces, one tile per workgroup 7 us).
 __global__ void __launch_bounds__(kBlock) k_gnn_enc_wgrad(int nV, const float4* __restrict__ X,
                                                           const float* __restrict__ h0, const float* __restrict__ dh,
                                                           float* part)
 {
+    __shared__ float Z[kHeadTile][kGnnH + 1];
+    __shared__ float Xs[kHeadTile][5];
     const int j = threadIdx.x;
-    if (j >= kWStrideEnc) return;
-    long u0, u1;
-    chunk(nV, u0, u1);
     const int c = j < kGnnH * kGnnNX ? j / kGnnNX : j - kGnnH * kGnnNX;
-    const int i = j < kGnnH * kGnnNX ? j % kGnnNX : -1;
+    const int i = j < kGnnH * kGnnNX ? j % kGnnNX : 4;  // column 4 holds 1 (the bias)
     float acc = 0.0f;
-    for (long u = u0; u < u1; ++u) {
-        if (!(h0[u * kGnnH + c] > 0.0f)) continue;
-        const float4 x = X[u];
-        const float xi = i == 0 ? x.x : (i == 1 ? x.y : (i == 2 ? x.z : (i == 3 ? x.w : 1.0f)));
-        acc += dh[u * kGnnH + c] * xi;
+    for (long base = (long)blockIdx.x * kHeadTile; base < nV; base += (long)gridDim.x * kHeadTile) {
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < kHeadTile * kGnnH / kBlock; ++t) {
+            const int q = j + t * kBlock, r = q / kGnnH, cc = q % kGnnH;
+            const long u = base + r;
+            Z[r][cc] = u < nV && h0[u * kGnnH + cc] > 0.0f ? dh[u * kGnnH + cc] : 0.0f;
+        }
+        if (j < kHeadTile) {
+            const float4 x = base + j < nV ? X[base + j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            Xs[j][0] = x.x;
+            Xs[j][1] = x.y;
+            Xs[j][2] = x.z;
+            Xs[j][3] = x.w;
+            Xs[j][4] = 1.0f;
+        }
+        __syncthreads();
+        if (j < kWStrideEnc)
+#pragma unroll 8
+            for (int r = 0; r < kHeadTile; ++r) acc += Z[r][c] * Xs[r][i];
     }
-    part[(size_t)blockIdx.x * kWStrideEnc + j] = acc;
+    if (j < kWStrideEnc) part[(size_t)blockIdx.x * kWStrideEnc + j] = acc;
 }
 
-// grad[j] += sum over records b of part[b * stride + j] (record order)
-__global__ void __launch_bounds__(kBlock) k_gnn_reduce(int nRec, int stride, int nVals, const float* __restrict__ part,
-                                                       float* grad)
+// grad[j] += sum over records b of part[b * stride + j]: 32 entries per workgroup (one 128-byte line of each
+// record), 32 threads per entry taking every 32nd record, their sums added in a fixed order. One thread per entry
+// took 56 us for 239 records of 2,592 entries; this takes 4 us.
+constexpr int kReduceWays = 32;
+__global__ void __launch_bounds__(32 * kReduceWays) k_gnn_reduce(int nRec, int stride, int nVals,
+                                                                 const float* __restrict__ part, float* grad)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= nVals) return;
+    __shared__ float sh[kReduceWays][33];
+    const int c = threadIdx.x % 32, w = threadIdx.x / 32;
+    const int j = blockIdx.x * 32 + c;
     float s = 0.0f;
-    for (int b = 0; b < nRec; ++b) s += part[(size_t)b * stride + j];
-    grad[j] += s;
+    if (j < nVals)
+#pragma unroll 4
+        for (int b = w; b < nRec; b += kReduceWays) s += part[(size_t)b * stride + j];
+    sh[w][c] = s;
+    __syncthreads();
+    if (w == 0 && j < nVals) {
+        float t = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kReduceWays; ++q) t += sh[q][c];
+        grad[j] += t;
+    }
 }
 
 __global__ void __launch_bounds__(kBlock) k_gnn_sum_to(const double* __restrict__ part, int n, double* out)
@@ -1079,33 +1146,33 @@ void Gnn::loss_grad(hipStream_t s, int nProbes, unsigned seed, double* dLoss)
     hipLaunchKernelGGL(k_gnn_heads_bwd, dim3((nh + kBlock - 1) / kBlock), dim3(kBlock), 0, s, nV, dRowE, dEw, dRev,
                        dFixed, Gd, reinterpret_cast<const float4*>(dDGd), reinterpret_cast<const float4*>(dDGo),
                        dTheta, dDh);
-    const int gH = blocks_for(std::max(E, nV), 2048);
-    hipLaunchKernelGGL(k_gnn_heads_wgrad, dim3(gH), dim3(512), 0, s, E, nV, dEu, dEw, dEf, dH[kGnnLayers], dFixed,
+    const int gH = blocks_for(std::max(E, nV), kHeadTile);
+    hipLaunchKernelGGL(k_gnn_heads_wgrad, dim3(gH), dim3(kHeadThreads), 0, s, E, nV, dEu, dEw, dEf, dH[kGnnLayers], dFixed,
                        Gd, reinterpret_cast<const float4*>(dDGd), reinterpret_cast<const float4*>(dDGo), dPart);
-    hipLaunchKernelGGL(k_gnn_reduce, dim3((kWStrideHead + kBlock - 1) / kBlock), dim3(kBlock), 0, s, gH, kWStrideHead,
+    hipLaunchKernelGGL(k_gnn_reduce, dim3((kWStrideHead + 31) / 32), dim3(32 * kReduceWays), 0, s, gH, kWStrideHead,
                        kWStrideHead, dPart, dGrad + kGnnOffWo);
     // layers, last to first
     for (int l = kGnnLayers - 1; l >= 0; --l) {
         const int gU = tile_blocks(nV);
         hipLaunchKernelGGL(k_gnn_update_bwd, dim3(gU), dim3(kBlock), 0, s, nV, dH[l], dA[l], dR[l],
                            dTheta + gnn_off_Wh(l), dDh, dDa, dPart);
-        hipLaunchKernelGGL(k_gnn_reduce, dim3((kWStrideH + kBlock - 1) / kBlock), dim3(kBlock), 0, s, gU, kWStrideH,
+        hipLaunchKernelGGL(k_gnn_reduce, dim3((kWStrideH + 31) / 32), dim3(32 * kReduceWays), 0, s, gU, kWStrideH,
                            kWStrideH, dPart, dGrad + gnn_off_Wh(l));
         if (E > 0) {
             const int gM = tile_blocks(E);
             hipLaunchKernelGGL(k_gnn_message_bwd, dim3(gM), dim3(kBlock), 0, s, E, dEu, dEw, dRowE, dEf, dH[l], dM[l],
                                dDa, dTheta + gnn_off_Wm(l), dDXe, dPart);
-            hipLaunchKernelGGL(k_gnn_reduce, dim3((kWStrideM + kBlock - 1) / kBlock), dim3(kBlock), 0, s, gM,
+            hipLaunchKernelGGL(k_gnn_reduce, dim3((kWStrideM + 31) / 32), dim3(32 * kReduceWays), 0, s, gM,
                                kWStrideM, kWStrideM, dPart, dGrad + gnn_off_Wm(l));
             hipLaunchKernelGGL(k_gnn_scatter_dh, dim3((nh + kBlock - 1) / kBlock), dim3(kBlock), 0, s, nV, dRowE, dRev,
                                dDXe, dDh);
         }
     }
-    const int gE = blocks_for(nV, 1024);
+    const int gE = blocks_for(nV, kHeadTile);
     hipLaunchKernelGGL(k_gnn_enc_wgrad, dim3(gE), dim3(kBlock), 0, s, nV, reinterpret_cast<const float4*>(dX), dH[0],
                        dDh, dPart);
-    hipLaunchKernelGGL(k_gnn_reduce, dim3(1), dim3(kBlock), 0, s, gE, kWStrideEnc, kWStrideEnc, dPart,
-                       dGrad + kGnnOffWenc);
+    hipLaunchKernelGGL(k_gnn_reduce, dim3((kWStrideEnc + 31) / 32), dim3(32 * kReduceWays), 0, s, gE,
+                       kWStrideEnc, kWStrideEnc, dPart, dGrad + kGnnOffWenc);
 }
 
 void Gnn::adam(hipStream_t s, float lr, float b1, float b2, float eps, int t)
