@@ -62,8 +62,8 @@ def assembly_bytes(nF, nV, nnzb, nub):
 def cheb_bytes(n, blocks, bs, word=8):
     """Algorithmic bytes of one V-cycle Chebyshev step (k_cheb_step) on a level of n rows and `blocks` stored
     bs x bs blocks: the blocks and their column indices, row pointers, per row the inverse diagonal block, the
-    gathered direction (read once), the residual and the iterate read and written, the new direction written."""
-    return blocks * (bs * bs * word + 4) + 4 * (n + 1) + n * (bs * bs * word + 6 * bs * word)
+    gathered direction (read once) and the iterate read and written."""
+    return blocks * (bs * bs * word + 4) + 4 * (n + 1) + n * (bs * bs * word + 3 * bs * word)
 
 
 def cheb_levels(ctx, reps=50):

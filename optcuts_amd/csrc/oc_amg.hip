@@ -986,11 +986,19 @@ __global__ void __launch_bounds__(256) k_dense_inverse(int nn, int bs, const int
 // bound by memory, and FP64 arithmetic keeps the FP32-stored V-cycle as close
 // to a fixed symmetric operator as its storage allows.
 //
-// pre-smoothing, first Chebyshev step from x = 0: r = D^-1 b, d = r/theta, x = d
-template <typename T, int BS, typename BIN>
-__global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ stop, int n, const BIN* __restrict__ bin, T* b,
-                                                      const T* __restrict__ Dinv, const double* __restrict__ lam,
-                                                      T* x, T* r, T* d)
+// Each smoothing is two Chebyshev steps for D^-1 A, before the coarse
+// correction from x = 0 and after it from x. The first step's direction d =
+// D^-1 (b - A x) / theta is the only vector it leaves: the residual of the
+// preconditioned system it came from is theta d, the pre-smoothing iterate is
+// d itself, and the second step's new residual and direction have no reader.
+// (Keeping residual, direction and iterate as vectors of their own moved 64
+// to 96 more bytes per fine row and step beside the ~300 of the row's blocks.)
+//
+// pre-smoothing, first step from x = 0: d = D^-1 b / theta
+template <typename T, int BS>
+__global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ stop, int n,
+                                                      const double* __restrict__ b, const T* __restrict__ Dinv,
+                                                      const double* __restrict__ lam, T* d)
 {
     if (stop && *stop) return;
     const ChebP cp = cheb_params(*lam);
@@ -998,39 +1006,31 @@ __global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ st
     chunk_rows(n, r0, r1);
     for (int u = r0 + threadIdx.x; u < r1; u += blockDim.x) {
         double bu[BS], Dm[BS * BS];
-        ld_vec<BS>(bin, u, bu);
+        ld_vec<BS>(b, u, bu);
         ld_block<BS>(Dinv + (size_t)u * BS * BS, Dm);
-        if ((const void*)bin != (const void*)b) {
-            T bt[BS];
-#pragma unroll
-            for (int i = 0; i < BS; ++i) bt[i] = (T)bu[i];
-            st_vec<BS>(b, u, bt);
-        }
-        T rt[BS], dt[BS];
+        T dt[BS];
 #pragma unroll
         for (int i = 0; i < BS; ++i) {
             double t = 0.0;
 #pragma unroll
             for (int j = 0; j < BS; ++j) t += Dm[i * BS + j] * bu[j];
-            rt[i] = (T)t;
             dt[i] = (T)(t / cp.theta);
         }
-        st_vec<BS>(r, u, rt);
         st_vec<BS>(d, u, dt);
-        st_vec<BS>(x, u, dt);
     }
 }
 
-// Chebyshev step k (k = 0 after pre1/post1): w = A d; r -= D^-1 w;
-// d' = rho1 rho0 d + 2 rho1/delta r; x += d'. d is read for the neighbours,
-// so the new d goes to dout. FINAL: z = x (FP64) and partial records of
-// rFinal.z per workgroup. Launch with row_grid workgroups.
-template <typename T, int BS, bool FINAL>
+// Second Chebyshev step, d the first step's direction: r = theta d - D^-1 A d,
+// d' = rho1 rho0 d + 2 rho1/delta r; KIND 0 (pre-smoothing): x = d + d'; 1
+// (post-smoothing): x += d + d'; 2 (the finest level's last step): z = x + d +
+// d' in FP64 and partial records of rFinal.z per workgroup. d is read for the
+// neighbours and not written. Launch with row_grid workgroups.
+template <typename T, int BS, int KIND>
 __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
                                                const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                const T* __restrict__ Dinv, const double* __restrict__ lam,
-                                               const T* __restrict__ din, T* dout, T* r, T* x,
-                                               const double* __restrict__ rFinal, double* zFinal, double* rzPart)
+                                               const T* __restrict__ d, T* x, const double* __restrict__ rFinal,
+                                               double* zFinal, double* rzPart)
 {
     constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
     const ChebP cp = cheb_params(*lam);
@@ -1042,71 +1042,66 @@ __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int*
     double acc[1] = {0.0};
     for (int p = 0; p < rc.passes; ++p) {
         RowPass<T, BS, UNROLL> rp;
-        rp.load(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr, colIdx, vals, din, lane);
-        double Dm[UNROLL][BS * BS], ro[UNROLL][BS], dd[UNROLL][BS], xo[UNROLL][BS], rf[UNROLL][BS];
+        rp.load(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr, colIdx, vals, d, lane);
+        double Dm[UNROLL][BS * BS], dd[UNROLL][BS], xo[UNROLL][BS], rf[UNROLL][BS];
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q)
             if (lane == 0 && rp.u[q] < rc.r1) {
                 ld_block<BS>(Dinv + (size_t)rp.u[q] * BS * BS, Dm[q]);
-                ld_vec<BS>(r, rp.u[q], ro[q]);
-                ld_vec<BS>(din, rp.u[q], dd[q]);
-                ld_vec<BS>(x, rp.u[q], xo[q]);
-                if (FINAL) ld_vec<BS>(rFinal, rp.u[q], rf[q]);
+                ld_vec<BS>(d, rp.u[q], dd[q]);
+                if (KIND >= 1) ld_vec<BS>(x, rp.u[q], xo[q]);
+                if (KIND == 2) ld_vec<BS>(rFinal, rp.u[q], rf[q]);
             }
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q) {
             double w[BS];
-            rp.mv(q, colIdx, vals, din, lane, w);
+            rp.mv(q, colIdx, vals, d, lane, w);
             if (lane == 0 && rp.u[q] < rc.r1) {
                 double xn[BS];
-                T rt[BS], dt[BS], xt[BS];
 #pragma unroll
                 for (int i = 0; i < BS; ++i) {
                     double dw = 0.0;
 #pragma unroll
                     for (int j = 0; j < BS; ++j) dw += Dm[q][i * BS + j] * w[j];
-                    const double rn = ro[q][i] - dw;
+                    const double rn = cp.theta * dd[q][i] - dw;
                     const double dn = c1 * dd[q][i] + c2 * rn;
-                    xn[i] = xo[q][i] + dn;
-                    rt[i] = (T)rn;
-                    dt[i] = (T)dn;
-                    xt[i] = (T)xn[i];
+                    xn[i] = (KIND >= 1 ? xo[q][i] + dd[q][i] : dd[q][i]) + dn;
                 }
-                st_vec<BS>(r, rp.u[q], rt);
-                st_vec<BS>(dout, rp.u[q], dt);
-                st_vec<BS>(x, rp.u[q], xt);
-                if (FINAL) {
+                if (KIND == 2) {
 #pragma unroll
                     for (int i = 0; i < BS; ++i) acc[0] += rf[q][i] * xn[i];
                     st_vec<BS>(zFinal, rp.u[q], xn);
+                } else {
+                    T xt[BS];
+#pragma unroll
+                    for (int i = 0; i < BS; ++i) xt[i] = (T)xn[i];
+                    st_vec<BS>(x, rp.u[q], xt);
                 }
             }
         }
     }
-    if (FINAL) {
+    if (KIND == 2) {
         block_sum<1>(acc);
         if (threadIdx.x == 0) rzPart[blk] = acc[0];
     }
 }
 
-template <typename T, int BS, bool FINAL>
+template <typename T, int BS, int KIND>
 __global__ void __launch_bounds__(kBlock) k_cheb_step(const int* __restrict__ stop, int n, const int* __restrict__ rowPtr,
                                                       const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                       const T* __restrict__ Dinv, const double* __restrict__ lam,
-                                                      const T* __restrict__ din, T* dout, T* r, T* x,
-                                                      const double* __restrict__ rFinal, double* zFinal,
-                                                      double* rzPart)
+                                                      const T* __restrict__ d, T* x, const double* __restrict__ rFinal,
+                                                      double* zFinal, double* rzPart)
 {
     if (stop && *stop) return;
-    cheb_step_rows<T, BS, FINAL>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, din, dout, r, x, rFinal,
-                                 zFinal, rzPart);
+    cheb_step_rows<T, BS, KIND>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, d, x, rFinal, zFinal, rzPart);
 }
 
-// residual res = b - A x (row_grid workgroups)
-template <typename T, int BS>
+// residual res = b - A x (row_grid workgroups); b is the FP64 right-hand side itself on the finest level
+template <typename T, int BS, typename B>
 __device__ __forceinline__ void residual_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
                                               const int* __restrict__ colIdx, const T* __restrict__ vals,
-                                              const T* __restrict__ b, const T* __restrict__ x, T* res)
+                                              const B* __restrict__ b, const T* __restrict__ x, T* res)
 {
     constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
     const RowChunk rc = row_chunk<BS>(n, blk, G);
@@ -1132,23 +1127,21 @@ __device__ __forceinline__ void residual_rows(int blk, int G, int n, const int* 
     }
 }
 
-template <typename T, int BS>
+template <typename T, int BS, typename B>
 __global__ void __launch_bounds__(kBlock) k_residual(const int* __restrict__ stop, int n, const int* __restrict__ rowPtr,
                                                      const int* __restrict__ colIdx, const T* __restrict__ vals,
-                                                     const T* __restrict__ b, const T* __restrict__ x, T* res)
+                                                     const B* __restrict__ b, const T* __restrict__ x, T* res)
 {
     if (stop && *stop) return;
-    residual_rows<T, BS>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, b, x, res);
+    residual_rows<T, BS, B>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, b, x, res);
 }
 
-// post-smoothing first step from the prolongated x: r = D^-1 (b - A x); d = r/theta;
-// xout = x + d (row_grid workgroups)
-template <typename T, int BS>
+// post-smoothing, first step from the prolongated x: d = D^-1 (b - A x) / theta (row_grid workgroups)
+template <typename T, int BS, typename B>
 __device__ __forceinline__ void cheb_post1_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
                                                 const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                 const T* __restrict__ Dinv, const double* __restrict__ lam,
-                                                const T* __restrict__ b, const T* __restrict__ xin, T* xout, T* r,
-                                                T* d)
+                                                const B* __restrict__ b, const T* __restrict__ x, T* d)
 {
     constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
     const ChebP cp = cheb_params(*lam);
@@ -1156,22 +1149,21 @@ __device__ __forceinline__ void cheb_post1_rows(int blk, int G, int n, const int
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
     for (int p = 0; p < rc.passes; ++p) {
         RowPass<T, BS, UNROLL> rp;
-        rp.load(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr, colIdx, vals, xin, lane);
-        double Dm[UNROLL][BS * BS], bo[UNROLL][BS], xo[UNROLL][BS];
+        rp.load(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr, colIdx, vals, x, lane);
+        double Dm[UNROLL][BS * BS], bo[UNROLL][BS];
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q)
             if (lane == 0 && rp.u[q] < rc.r1) {
                 ld_block<BS>(Dinv + (size_t)rp.u[q] * BS * BS, Dm[q]);
                 ld_vec<BS>(b, rp.u[q], bo[q]);
-                ld_vec<BS>(xin, rp.u[q], xo[q]);
             }
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q) {
             double y[BS];
-            rp.mv(q, colIdx, vals, xin, lane, y);
+            rp.mv(q, colIdx, vals, x, lane, y);
             if (lane == 0 && rp.u[q] < rc.r1) {
                 double res[BS];
-                T ru[BS], dv[BS], xv[BS];
+                T dt[BS];
 #pragma unroll
                 for (int i = 0; i < BS; ++i) res[i] = bo[q][i] - y[i];
 #pragma unroll
@@ -1179,42 +1171,34 @@ __device__ __forceinline__ void cheb_post1_rows(int blk, int G, int n, const int
                     double t = 0.0;
 #pragma unroll
                     for (int j = 0; j < BS; ++j) t += Dm[q][i * BS + j] * res[j];
-                    const double dvi = t / cp.theta;
-                    ru[i] = (T)t;
-                    dv[i] = (T)dvi;
-                    xv[i] = (T)(xo[q][i] + dvi);
+                    dt[i] = (T)(t / cp.theta);
                 }
-                st_vec<BS>(r, rp.u[q], ru);
-                st_vec<BS>(d, rp.u[q], dv);
-                st_vec<BS>(xout, rp.u[q], xv);
+                st_vec<BS>(d, rp.u[q], dt);
             }
         }
     }
 }
 
-template <typename T, int BS>
+template <typename T, int BS, typename B>
 __global__ void __launch_bounds__(kBlock) k_cheb_post1(const int* __restrict__ stop, int n, const int* __restrict__ rowPtr,
                                                        const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                        const T* __restrict__ Dinv, const double* __restrict__ lam,
-                                                       const T* __restrict__ b, const T* __restrict__ xin,
-                                                       T* xout, T* r, T* d)
+                                                       const B* __restrict__ b, const T* __restrict__ x, T* d)
 {
     if (stop && *stop) return;
-    cheb_post1_rows<T, BS>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, b, xin, xout, r, d);
+    cheb_post1_rows<T, BS, B>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, b, x, d);
 }
 
 // bc_c = sum over P blocks (u,c) of P^T res_u, LN lanes per coarse node (the launcher picks LN from the mean
 // length of the restriction lists: on the small coarse levels a node gathers ~100 P blocks, and with few nodes
 // the kernel is one latency chain per lane, so the lanes per node grow with the list).
-// PRE1: the next level's first pre-smoothing step (k_cheb_pre1 from x = 0:
-// r = D^-1 b, d = r/theta, x = d) is row-local, so it runs here on each
-// restricted row instead of in a launch of its own.
+// PRE1: the next level's first pre-smoothing step (k_cheb_pre1) is row-local,
+// so it runs here on each restricted row instead of in a launch of its own.
 template <typename T, int BS, bool PRE1, int LN>
 __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int* __restrict__ rPtr,
                                               const int* __restrict__ rP, const int* __restrict__ pRow,
                                               const T* __restrict__ P, const T* __restrict__ res, T* bc,
-                                              const T* __restrict__ DinvN, const double* __restrict__ lamN, T* xN,
-                                              T* rN, T* dN)
+                                              const T* __restrict__ DinvN, const double* __restrict__ lamN, T* dN)
 {
     const int cc = (nc + G - 1) / G;
     const int c0 = blk * cc, c1 = min(nc, c0 + cc);
@@ -1244,18 +1228,15 @@ __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int*
                 const double theta = cheb_params(*lamN).theta;
                 double Dm[NS * NS];
                 ld_block<NS>(DinvN + (size_t)c * NS * NS, Dm);
-                T rt[NS], dt[NS];
+                T dt[NS];
 #pragma unroll
                 for (int i = 0; i < NS; ++i) {
                     double t = 0.0;
 #pragma unroll
                     for (int j = 0; j < NS; ++j) t += Dm[i * NS + j] * (double)bt[j];
-                    rt[i] = (T)t;
                     dt[i] = (T)(t / theta);
                 }
-                st_vec<NS>(rN, c, rt);
                 st_vec<NS>(dN, c, dt);
-                st_vec<NS>(xN, c, dt);
             }
         }
     }
@@ -1266,10 +1247,10 @@ __global__ void __launch_bounds__(kBlock) k_restrict(const int* __restrict__ sto
                                                      const int* __restrict__ rP, const int* __restrict__ pRow,
                                                      const T* __restrict__ P, const T* __restrict__ res, T* bc,
                                                      const T* __restrict__ DinvN, const double* __restrict__ lamN,
-                                                     T* xN, T* rN, T* dN)
+                                                     T* dN)
 {
     if (stop && *stop) return;
-    restrict_rows<T, BS, PRE1, LN>(blockIdx.x, gridDim.x, nc, rPtr, rP, pRow, P, res, bc, DinvN, lamN, xN, rN, dN);
+    restrict_rows<T, BS, PRE1, LN>(blockIdx.x, gridDim.x, nc, rPtr, rP, pRow, P, res, bc, DinvN, lamN, dN);
 }
 
 // x_u += sum over P blocks (u,c) of P xc_c, kProlongLanes lanes per fine row (one P block each per pass, the
@@ -1376,7 +1357,7 @@ struct Amg<T>::Level : AmgHostLevel {
         *dTcP = nullptr, *dAcPtr = nullptr, *dAcP = nullptr, *dAcT = nullptr;
     unsigned char* dPIsTent = nullptr;
     T *vals = nullptr, *Dinv = nullptr, *Pt = nullptr, *P = nullptr, *Tv = nullptr;
-    T *b = nullptr, *x = nullptr, *x2 = nullptr, *r = nullptr, *d = nullptr, *d2 = nullptr;
+    T *b = nullptr, *x = nullptr, *r = nullptr, *d = nullptr;  // right-hand side, iterate, residual, direction
     double *Bnext = nullptr, *lz = nullptr, *lam = nullptr;  // lz: 6 Lanczos vectors, then alpha/beta/count
     // hand every buffer back to the owner's pool
     void give_back(Pool& pool)
@@ -1385,7 +1366,7 @@ struct Amg<T>::Level : AmgHostLevel {
                         (void*)dPCol, (void*)dPRow, (void*)dPsPtr, (void*)dPsA, (void*)dRPtr, (void*)dRP,
                         (void*)dTcPtr, (void*)dTcA, (void*)dTcP, (void*)dAcPtr, (void*)dAcP, (void*)dAcT,
                         (void*)dPIsTent, (void*)vals, (void*)Dinv, (void*)Pt, (void*)P, (void*)Tv, (void*)b,
-                        (void*)x, (void*)x2, (void*)r, (void*)d, (void*)d2, (void*)Bnext, (void*)lz, (void*)lam})
+                        (void*)x, (void*)r, (void*)d, (void*)Bnext, (void*)lz, (void*)lam})
             if (p) pool.put(p);
     }
 };
@@ -1498,11 +1479,11 @@ void Amg<T>::cheb_step_level(hipStream_t s, int l)
 {
     Level& A = *L[l];
     if (A.bs == 2)
-        hipLaunchKernelGGL((k_cheb_step<T, 2, false>), dim3(row_grid(A.n, 2)), dim3(kBlock), 0, s, nullptr, A.n,
-                           A.dRowPtr, A.dColIdx, A.vals, A.Dinv, A.lam, A.d, A.d2, A.r, A.x, nullptr, nullptr, nullptr);
+        hipLaunchKernelGGL((k_cheb_step<T, 2, 1>), dim3(row_grid(A.n, 2)), dim3(kBlock), 0, s, nullptr, A.n,
+                           A.dRowPtr, A.dColIdx, A.vals, A.Dinv, A.lam, A.d, A.x, nullptr, nullptr, nullptr);
     else
-        hipLaunchKernelGGL((k_cheb_step<T, 3, false>), dim3(row_grid(A.n, 3)), dim3(kBlock), 0, s, nullptr, A.n,
-                           A.dRowPtr, A.dColIdx, A.vals, A.Dinv, A.lam, A.d, A.d2, A.r, A.x, nullptr, nullptr, nullptr);
+        hipLaunchKernelGGL((k_cheb_step<T, 3, 1>), dim3(row_grid(A.n, 3)), dim3(kBlock), 0, s, nullptr, A.n,
+                           A.dRowPtr, A.dColIdx, A.vals, A.Dinv, A.lam, A.d, A.x, nullptr, nullptr, nullptr);
 }
 
 template <typename T>
@@ -1551,10 +1532,8 @@ int Amg<T>::setup(hipStream_t s, int nV, const std::vector<int>& rowPtr, const s
         dalloc(pool_, A.Dinv, (size_t)A.n * bs * bs);
         dalloc(pool_, A.b, (size_t)A.n * bs);
         dalloc(pool_, A.x, (size_t)A.n * bs);
-        dalloc(pool_, A.x2, (size_t)A.n * bs);
         dalloc(pool_, A.r, (size_t)A.n * bs);
         dalloc(pool_, A.d, (size_t)A.n * bs);
-        dalloc(pool_, A.d2, (size_t)A.n * bs);
         dalloc(pool_, A.lam, 2);
         dalloc(pool_, A.lz, (size_t)6 * A.n * bs + 2 * kLanczosSteps + 1);
         if (l + 1 < L.size()) {
@@ -1736,7 +1715,7 @@ struct TailArgs {
     const int *rowPtr, *colIdx, *rPtr, *rP, *pRow, *pPtr, *pCol;
     const void *vals, *Dinv, *P;
     const double* lam;
-    void *b, *x, *x2, *r, *d, *d2;
+    void *b, *x, *r, *d;
     // coarsest level
     int nc, cbs, dense;
     const void* DinvC;
@@ -1751,16 +1730,13 @@ __global__ void __launch_bounds__(kBlock) k_vcycle_tail(const int* __restrict__ 
     const T* vals = static_cast<const T*>(a.vals);
     const T* Dinv = static_cast<const T*>(a.Dinv);
     const T* P = static_cast<const T*>(a.P);
-    T *b = static_cast<T*>(a.b), *x = static_cast<T*>(a.x), *x2 = static_cast<T*>(a.x2);
-    T *r = static_cast<T*>(a.r), *d = static_cast<T*>(a.d), *d2 = static_cast<T*>(a.d2);
+    T *b = static_cast<T*>(a.b), *x = static_cast<T*>(a.x), *r = static_cast<T*>(a.r), *d = static_cast<T*>(a.d);
     T *bC = static_cast<T*>(a.bC), *xC = static_cast<T*>(a.xC);
-    cheb_step_rows<T, 3, false>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, d2, r, x, nullptr, nullptr,
-                                nullptr);
+    cheb_step_rows<T, 3, 0>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, x, nullptr, nullptr, nullptr);
     __syncthreads();
-    residual_rows<T, 3>(0, 1, a.n, a.rowPtr, a.colIdx, vals, b, x, r);
+    residual_rows<T, 3, T>(0, 1, a.n, a.rowPtr, a.colIdx, vals, b, x, r);
     __syncthreads();
-    restrict_rows<T, 3, false, LN>(0, 1, a.nc, a.rPtr, a.rP, a.pRow, P, r, bC, nullptr, nullptr, nullptr, nullptr,
-                                   nullptr);
+    restrict_rows<T, 3, false, LN>(0, 1, a.nc, a.rPtr, a.rP, a.pRow, P, r, bC, nullptr, nullptr, nullptr);
     __syncthreads();
     if (a.dense) {
         dense_apply_rows<T>(a.nc * a.cbs, a.Inv, bC, xC);
@@ -1774,10 +1750,9 @@ __global__ void __launch_bounds__(kBlock) k_vcycle_tail(const int* __restrict__ 
     __syncthreads();
     for (int blk = 0; blk * kBlock < a.n * kProlongLanes; ++blk) prolong_rows<T, 3>(blk, a.n, a.pPtr, a.pCol, P, xC, x);
     __syncthreads();
-    cheb_post1_rows<T, 3>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, b, x, x2, r, d);
+    cheb_post1_rows<T, 3, T>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, b, x, d);
     __syncthreads();
-    cheb_step_rows<T, 3, false>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, d2, r, x2, nullptr, nullptr,
-                                nullptr);
+    cheb_step_rows<T, 3, 1>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, x, nullptr, nullptr, nullptr);
 }
 
 template <typename T>
@@ -1808,10 +1783,10 @@ void Amg<T>::restrict_to(hipStream_t s, int l, const int* stop)
     const auto launch = [&](auto kern) {
         if (fuse)
             hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, s, stop, A.nc, A.dRPtr, A.dRP, A.dPRow, A.P, A.r, N.b, N.Dinv,
-                               N.lam, N.x, N.r, N.d);
+                               N.lam, N.d);
         else
             hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, s, stop, A.nc, A.dRPtr, A.dRP, A.dPRow, A.P, A.r, N.b,
-                               nullptr, nullptr, nullptr, nullptr, nullptr);
+                               nullptr, nullptr, nullptr);
     };
 #define OC_RESTRICT(BS_, F_)                                                      \
     (ln == 64 ? launch(k_restrict<T, BS_, F_, 64>)                                \
@@ -1846,10 +1821,8 @@ void Amg<T>::vcycle_tail(hipStream_t s, int l, const int* stop)
     a.lam = A.lam;
     a.b = A.b;
     a.x = A.x;
-    a.x2 = A.x2;
     a.r = A.r;
     a.d = A.d;
-    a.d2 = A.d2;
     a.nc = C.n;
     a.cbs = C.bs;
     a.dense = coarseDiag ? 0 : 1;
@@ -1865,6 +1838,8 @@ void Amg<T>::vcycle_tail(hipStream_t s, int l, const int* stop)
     else hipLaunchKernelGGL((k_vcycle_tail<T, 16>), dim3(1), dim3(kBlock), 0, s, stop, a);
 }
 
+// One smoothed level of the V-cycle below the finest (or the coarsest solve): from N.b and the direction that the
+// restriction left in N.d to N.x.
 template <typename T>
 void Amg<T>::vcycle(hipStream_t s, int l, const int* stop)
 {
@@ -1873,45 +1848,24 @@ void Amg<T>::vcycle(hipStream_t s, int l, const int* stop)
         coarse_solve(s, stop);
         return;
     }
-    Level& N = *L[l + 1];
-    const int gUp = rows_grid(A.n, kBlock);
-    if (A.bs == 2) {
-        const int g = row_grid(A.n, 2);
-        (void)gUp;  // level 0 starts from k_cheb_pre1 in apply(); lower levels from the fused restriction
-        hipLaunchKernelGGL((k_cheb_step<T, 2, false>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
-                           A.vals, A.Dinv, A.lam, A.d, A.d2, A.r, A.x, nullptr, nullptr, nullptr);
-        hipLaunchKernelGGL((k_residual<T, 2>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
-                           A.b, A.x, A.r);
-        restrict_to(s, l, stop);
-        vcycle(s, l + 1, stop);
-        hipLaunchKernelGGL((k_prolong<T, 2>), dim3(grid_for((long)A.n * kProlongLanes)), dim3(kBlock), 0, s, stop, A.n, A.dPPtr, A.dPCol, A.P,
-                           N.x, A.x);
-        hipLaunchKernelGGL((k_cheb_post1<T, 2>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
-                           A.Dinv, A.lam, A.b, A.x, A.x2, A.r, A.d);
-    } else {
-        const int g = row_grid(A.n, 3);
-        if (l == 0)  // levels below the finest start from the restriction's fused first step
-            hipLaunchKernelGGL((k_cheb_pre1<T, 3, T>), dim3(gUp), dim3(kBlock), 0, s, stop, A.n, A.b, A.b, A.Dinv, A.lam,
-                               A.x, A.r, A.d);
-        if (l + 2 == (int)L.size() && A.n <= (tailMax_ < 0 ? kTailMaxNodes : tailMax_)) {
-            vcycle_tail(s, l, stop);
-            std::swap(A.x, A.x2);
-            return;
-        }
-        hipLaunchKernelGGL((k_cheb_step<T, 3, false>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
-                           A.vals, A.Dinv, A.lam, A.d, A.d2, A.r, A.x, nullptr, nullptr, nullptr);
-        hipLaunchKernelGGL((k_residual<T, 3>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
-                           A.b, A.x, A.r);
-        restrict_to(s, l, stop);
-        vcycle(s, l + 1, stop);
-        hipLaunchKernelGGL((k_prolong<T, 3>), dim3(grid_for((long)A.n * kProlongLanes)), dim3(kBlock), 0, s, stop, A.n, A.dPPtr, A.dPCol, A.P,
-                           N.x, A.x);
-        hipLaunchKernelGGL((k_cheb_post1<T, 3>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
-                           A.Dinv, A.lam, A.b, A.x, A.x2, A.r, A.d);
-        hipLaunchKernelGGL((k_cheb_step<T, 3, false>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
-                           A.vals, A.Dinv, A.lam, A.d, A.d2, A.r, A.x2, nullptr, nullptr, nullptr);
-        std::swap(A.x, A.x2);
+    if (l + 2 == (int)L.size() && A.n <= (tailMax_ < 0 ? kTailMaxNodes : tailMax_)) {
+        vcycle_tail(s, l, stop);
+        return;
     }
+    Level& N = *L[l + 1];
+    const int g = row_grid(A.n, 3);
+    hipLaunchKernelGGL((k_cheb_step<T, 3, 0>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
+                       A.Dinv, A.lam, A.d, A.x, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((k_residual<T, 3, T>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
+                       A.b, A.x, A.r);
+    restrict_to(s, l, stop);
+    vcycle(s, l + 1, stop);
+    hipLaunchKernelGGL((k_prolong<T, 3>), dim3(grid_for((long)A.n * kProlongLanes)), dim3(kBlock), 0, s, stop, A.n,
+                       A.dPPtr, A.dPCol, A.P, N.x, A.x);
+    hipLaunchKernelGGL((k_cheb_post1<T, 3, T>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
+                       A.Dinv, A.lam, A.b, A.x, A.d);
+    hipLaunchKernelGGL((k_cheb_step<T, 3, 1>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
+                       A.Dinv, A.lam, A.d, A.x, nullptr, nullptr, nullptr);
 }
 
 template <typename T>
@@ -1926,13 +1880,22 @@ void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, co
         hipLaunchKernelGGL(k_finish_z<T>, dim3(g), dim3(kBlock), 0, s, stop, A.n * 2, A.x, r, z, rzPart);
         return;
     }
-    // level 0 pre-smoothing reads the FP64 residual and keeps a T copy in A.b
-    hipLaunchKernelGGL((k_cheb_pre1<T, 2, double>), dim3(rows_grid(A.n, kBlock)), dim3(kBlock), 0, s, stop, A.n, r, A.b,
-                       A.Dinv, A.lam, A.x, A.r, A.d);
-    vcycle(s, 0, stop);
-    // final post-smoothing step writes z (FP64) and the r.z partial records
-    hipLaunchKernelGGL((k_cheb_step<T, 2, true>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
-                       A.Dinv, A.lam, A.d, A.d2, A.r, A.x2, r, z, rzPart);
+    // the finest level reads the FP64 residual in place; its last step writes z (FP64) and the r.z records
+    Level& N = *L[1];
+    hipLaunchKernelGGL((k_cheb_pre1<T, 2>), dim3(rows_grid(A.n, kBlock)), dim3(kBlock), 0, s, stop, A.n, r, A.Dinv,
+                       A.lam, A.d);
+    hipLaunchKernelGGL((k_cheb_step<T, 2, 0>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
+                       A.Dinv, A.lam, A.d, A.x, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((k_residual<T, 2, double>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
+                       A.vals, r, A.x, A.r);
+    restrict_to(s, 0, stop);
+    vcycle(s, 1, stop);
+    hipLaunchKernelGGL((k_prolong<T, 2>), dim3(grid_for((long)A.n * kProlongLanes)), dim3(kBlock), 0, s, stop, A.n,
+                       A.dPPtr, A.dPCol, A.P, N.x, A.x);
+    hipLaunchKernelGGL((k_cheb_post1<T, 2, double>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
+                       A.vals, A.Dinv, A.lam, r, A.x, A.d);
+    hipLaunchKernelGGL((k_cheb_step<T, 2, 2>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
+                       A.Dinv, A.lam, A.d, A.x, r, z, rzPart);
 }
 
 template class Amg<float>;
