@@ -275,6 +275,24 @@ __device__ __forceinline__ void ld_block(const T* __restrict__ p, R (&a)[BS * BS
     }
 }
 
+// N consecutive values, in 16-byte loads where they are an even number of doubles (the caller's blocks are then
+// 16-byte aligned)
+template <int N, typename T>
+__device__ __forceinline__ void ld_blk(const T* __restrict__ p, T (&a)[N])
+{
+    if constexpr (std::is_same<T, double>::value && N % 2 == 0) {
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i) {
+            const double2 t = reinterpret_cast<const double2*>(p)[i];
+            a[2 * i] = t.x;
+            a[2 * i + 1] = t.y;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) a[i] = p[i];
+    }
+}
+
 template <int BS, typename T, typename R>
 __device__ __forceinline__ void ld_vec(const T* __restrict__ p, size_t u, R (&x)[BS])
 {
@@ -823,7 +841,8 @@ __global__ void __launch_bounds__(kBlock) k_smooth_p(int nP, const int* __restri
                                                      const int* __restrict__ psPtr, const int* __restrict__ psA,
                                                      const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                      const T* __restrict__ Dinv, const T* __restrict__ Pt,
-                                                     const double* __restrict__ lam, T* P)
+                                                     const double* __restrict__ lam, const int* __restrict__ rPos,
+                                                     T* P, T* R)
 {
     constexpr int LANES = kSetupLanes;
     const int j = (blockIdx.x * blockDim.x + threadIdx.x) / LANES, lane = threadIdx.x % LANES;
@@ -848,6 +867,7 @@ __global__ void __launch_bounds__(kBlock) k_smooth_p(int nP, const int* __restri
     const T* ptu = Pt + (size_t)u * BS * NS;
     const bool tent = pIsTent[j] != 0;
     T* o = P + (size_t)j * BS * NS;
+    T* ro = R + (size_t)rPos[j] * BS * NS;
 #pragma unroll
     for (int i = 0; i < BS; ++i)
 #pragma unroll
@@ -855,8 +875,21 @@ __global__ void __launch_bounds__(kBlock) k_smooth_p(int nP, const int* __restri
             double s = 0.0;
 #pragma unroll
             for (int l = 0; l < BS; ++l) s += (double)D[i * BS + l] * S[l * NS + c];
-            o[i * NS + c] = (T)((tent ? (double)ptu[i * NS + c] : 0.0) - omega * s);
+            const T v = (T)((tent ? (double)ptu[i * NS + c] : 0.0) - omega * s);
+            o[i * NS + c] = v;
+            ro[i * NS + c] = v;
         }
+}
+
+// Restriction order of the P blocks: entry q of the lists is block rP[q]; its fine row and each block's place.
+__global__ void __launch_bounds__(kBlock) k_restrict_maps(int nP, const int* __restrict__ rP,
+                                                          const int* __restrict__ pRow, int* rRow, int* rPos)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nP) return;
+    const int j = rP[q];
+    rRow[q] = pRow[j];
+    rPos[j] = q;
 }
 
 // T block = sum over (A block, P block) pairs of A_k P_j (BS x NS); kSetupLanes lanes per block
@@ -1191,25 +1224,29 @@ __global__ void __launch_bounds__(kBlock) k_cheb_post1(const int* __restrict__ s
 
 // bc_c = sum over P blocks (u,c) of P^T res_u, LN lanes per coarse node (the launcher picks LN from the mean
 // length of the restriction lists: on the small coarse levels a node gathers ~100 P blocks, and with few nodes
-// the kernel is one latency chain per lane, so the lanes per node grow with the list).
+// the kernel is one latency chain per lane, so the lanes per node grow with the list). R holds the P blocks in
+// list order (k_smooth_p writes both), so a node's blocks are one contiguous run and the fine rows are read
+// without passing through the block index; with the XCD chunk order the residual rows of neighbouring nodes stay
+// in one L2. Gathering 48-byte P blocks from workgroups dealt round robin ran at 2 TB/s (1M faces, finest level:
+// 38 us, now 24; 200k faces 9.9, now 6.0).
 // PRE1: the next level's first pre-smoothing step (k_cheb_pre1) is row-local,
 // so it runs here on each restricted row instead of in a launch of its own.
 template <typename T, int BS, bool PRE1, int LN>
 __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int* __restrict__ rPtr,
-                                              const int* __restrict__ rP, const int* __restrict__ pRow,
-                                              const T* __restrict__ P, const T* __restrict__ res, T* bc,
+                                              const int* __restrict__ rRow, const T* __restrict__ R,
+                                              const T* __restrict__ res, T* bc,
                                               const T* __restrict__ DinvN, const double* __restrict__ lamN, T* dN)
 {
     const int cc = (nc + G - 1) / G;
-    const int c0 = blk * cc, c1 = min(nc, c0 + cc);
+    const int c0 = xcd_chunk(blk, G) * cc, c1 = min(nc, c0 + cc);
     constexpr int RPP = kBlock / LN;
     const int sub = threadIdx.x / LN, lane = threadIdx.x % LN;
     for (int c = c0 + sub; c < c1; c += RPP) {
         double s[NS] = {};
         for (int q = rPtr[c] + lane; q < rPtr[c + 1]; q += LN) {
-            const int j = rP[q];
-            const T* p = P + (size_t)j * BS * NS;
-            const T* ru = res + (size_t)pRow[j] * BS;
+            T p[BS * NS], ru[BS];
+            ld_blk<BS * NS>(R + (size_t)q * BS * NS, p);
+            ld_vec<BS>(res, rRow[q], ru);
 #pragma unroll
             for (int l = 0; l < BS; ++l)
 #pragma unroll
@@ -1244,13 +1281,13 @@ __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int*
 
 template <typename T, int BS, bool PRE1, int LN>
 __global__ void __launch_bounds__(kBlock) k_restrict(const int* __restrict__ stop, int nc, const int* __restrict__ rPtr,
-                                                     const int* __restrict__ rP, const int* __restrict__ pRow,
-                                                     const T* __restrict__ P, const T* __restrict__ res, T* bc,
+                                                     const int* __restrict__ rRow, const T* __restrict__ R,
+                                                     const T* __restrict__ res, T* bc,
                                                      const T* __restrict__ DinvN, const double* __restrict__ lamN,
                                                      T* dN)
 {
     if (stop && *stop) return;
-    restrict_rows<T, BS, PRE1, LN>(blockIdx.x, gridDim.x, nc, rPtr, rP, pRow, P, res, bc, DinvN, lamN, dN);
+    restrict_rows<T, BS, PRE1, LN>(blockIdx.x, gridDim.x, nc, rPtr, rRow, R, res, bc, DinvN, lamN, dN);
 }
 
 // x_u += sum over P blocks (u,c) of P xc_c, kProlongLanes lanes per fine row (one P block each per pass, the
@@ -1353,19 +1390,19 @@ struct Amg<T>::Level : AmgHostLevel {
     // device
     int *dRowPtr = nullptr, *dColIdx = nullptr, *dDiagPos = nullptr;
     int *dAggPtr = nullptr, *dAggMem = nullptr, *dPPtr = nullptr, *dPCol = nullptr, *dPRow = nullptr,
-        *dPsPtr = nullptr, *dPsA = nullptr, *dRPtr = nullptr, *dRP = nullptr, *dTcPtr = nullptr, *dTcA = nullptr,
+        *dPsPtr = nullptr, *dPsA = nullptr, *dRPtr = nullptr, *dRRow = nullptr, *dRPos = nullptr, *dTcPtr = nullptr, *dTcA = nullptr,
         *dTcP = nullptr, *dAcPtr = nullptr, *dAcP = nullptr, *dAcT = nullptr;
     unsigned char* dPIsTent = nullptr;
-    T *vals = nullptr, *Dinv = nullptr, *Pt = nullptr, *P = nullptr, *Tv = nullptr;
+    T *vals = nullptr, *Dinv = nullptr, *Pt = nullptr, *P = nullptr, *R = nullptr, *Tv = nullptr;
     T *b = nullptr, *x = nullptr, *r = nullptr, *d = nullptr;  // right-hand side, iterate, residual, direction
     double *Bnext = nullptr, *lz = nullptr, *lam = nullptr;  // lz: 6 Lanczos vectors, then alpha/beta/count
     // hand every buffer back to the owner's pool
     void give_back(Pool& pool)
     {
         for (void* p : {(void*)dRowPtr, (void*)dColIdx, (void*)dDiagPos, (void*)dAggPtr, (void*)dAggMem, (void*)dPPtr,
-                        (void*)dPCol, (void*)dPRow, (void*)dPsPtr, (void*)dPsA, (void*)dRPtr, (void*)dRP,
+                        (void*)dPCol, (void*)dPRow, (void*)dPsPtr, (void*)dPsA, (void*)dRPtr, (void*)dRRow, (void*)dRPos,
                         (void*)dTcPtr, (void*)dTcA, (void*)dTcP, (void*)dAcPtr, (void*)dAcP, (void*)dAcT,
-                        (void*)dPIsTent, (void*)vals, (void*)Dinv, (void*)Pt, (void*)P, (void*)Tv, (void*)b,
+                        (void*)dPIsTent, (void*)vals, (void*)Dinv, (void*)Pt, (void*)P, (void*)R, (void*)Tv, (void*)b,
                         (void*)x, (void*)r, (void*)d, (void*)Bnext, (void*)lz, (void*)lam})
             if (p) pool.put(p);
     }
@@ -1545,7 +1582,14 @@ int Amg<T>::setup(hipStream_t s, int nV, const std::vector<int>& rowPtr, const s
             up(pool_, s, A.dPsPtr, A.psPtr);
             up(pool_, s, A.dPsA, A.psA);
             up(pool_, s, A.dRPtr, A.rPtr);
-            up(pool_, s, A.dRP, A.rP);
+            int* rP = nullptr;  // read by the next kernel only; the pool hands it out again in stream order
+            up(pool_, s, rP, A.rP);
+            dalloc(pool_, A.dRRow, A.rP.size());
+            dalloc(pool_, A.dRPos, A.rP.size());
+            if (rP && A.dRRow && A.dRPos && !A.rP.empty())
+                hipLaunchKernelGGL(k_restrict_maps, dim3(grid_for((long)A.rP.size())), dim3(kBlock), 0, s,
+                                   (int)A.rP.size(), rP, A.dPRow, A.dRRow, A.dRPos);
+            if (rP) pool_.put(rP);
             up(pool_, s, A.dTcPtr, A.tcPtr);
             up(pool_, s, A.dTcA, A.tcA);
             up(pool_, s, A.dTcP, A.tcP);
@@ -1558,6 +1602,7 @@ int Amg<T>::setup(hipStream_t s, int nV, const std::vector<int>& rowPtr, const s
             dalloc(pool_, A.Pt, (size_t)A.n * bs * NS);
             (void)hipMemsetAsync(A.Pt, 0, sizeof(T) * (size_t)A.n * bs * NS, s);
             dalloc(pool_, A.P, A.pCol.size() * bs * NS);
+            dalloc(pool_, A.R, A.pCol.size() * bs * NS);
             dalloc(pool_, A.Tv, A.tCol.size() * bs * NS);
             dalloc(pool_, A.Bnext, (size_t)A.nc * NS * NS);
         }
@@ -1648,7 +1693,7 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
             hipLaunchKernelGGL((k_tentative<T, 2>), dim3(setup_grid(A.nc, kSetupLanes)), dim3(kBlock), 0, s, A.nc, A.dAggPtr,
                                A.dAggMem, reinterpret_cast<const double2*>(UV), Bin, A.Pt, A.Bnext);
             hipLaunchKernelGGL((k_smooth_p<T, 2>), dim3(setup_grid(nP, kSetupLanes)), dim3(kBlock), 0, s, nP, A.dPRow, A.dPIsTent,
-                               A.dPsPtr, A.dPsA, A.dColIdx, A.vals, A.Dinv, A.Pt, A.lam, A.P);
+                               A.dPsPtr, A.dPsA, A.dColIdx, A.vals, A.Dinv, A.Pt, A.lam, A.dRPos, A.P, A.R);
             hipLaunchKernelGGL((k_ap<T, 2>), dim3(setup_grid(nT, kSetupLanes)), dim3(kBlock), 0, s, nT, A.dTcPtr, A.dTcA, A.dTcP,
                                A.vals, A.P, A.Tv);
             hipLaunchKernelGGL((k_ptap<T, 2>), dim3(setup_grid(nAc, kSetupLanes)), dim3(kBlock), 0, s, nAc, A.dAcPtr, A.dAcP,
@@ -1657,7 +1702,7 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
             hipLaunchKernelGGL((k_tentative<T, 3>), dim3(setup_grid(A.nc, kSetupLanes)), dim3(kBlock), 0, s, A.nc, A.dAggPtr,
                                A.dAggMem, reinterpret_cast<const double2*>(UV), Bin, A.Pt, A.Bnext);
             hipLaunchKernelGGL((k_smooth_p<T, 3>), dim3(setup_grid(nP, kSetupLanes)), dim3(kBlock), 0, s, nP, A.dPRow, A.dPIsTent,
-                               A.dPsPtr, A.dPsA, A.dColIdx, A.vals, A.Dinv, A.Pt, A.lam, A.P);
+                               A.dPsPtr, A.dPsA, A.dColIdx, A.vals, A.Dinv, A.Pt, A.lam, A.dRPos, A.P, A.R);
             hipLaunchKernelGGL((k_ap<T, 3>), dim3(setup_grid(nT, kSetupLanes)), dim3(kBlock), 0, s, nT, A.dTcPtr, A.dTcA, A.dTcP,
                                A.vals, A.P, A.Tv);
             hipLaunchKernelGGL((k_ptap<T, 3>), dim3(setup_grid(nAc, kSetupLanes)), dim3(kBlock), 0, s, nAc, A.dAcPtr, A.dAcP,
@@ -1712,8 +1757,8 @@ constexpr int kTailMaxNodes = OC_TAIL_MAX_NODES;  // largest last smoothed level
 struct TailArgs {
     // smoothed level (3x3 blocks)
     int n;
-    const int *rowPtr, *colIdx, *rPtr, *rP, *pRow, *pPtr, *pCol;
-    const void *vals, *Dinv, *P;
+    const int *rowPtr, *colIdx, *rPtr, *rRow, *pPtr, *pCol;
+    const void *vals, *Dinv, *P, *R;
     const double* lam;
     void *b, *x, *r, *d;
     // coarsest level
@@ -1736,7 +1781,8 @@ __global__ void __launch_bounds__(kBlock) k_vcycle_tail(const int* __restrict__ 
     __syncthreads();
     residual_rows<T, 3, T>(0, 1, a.n, a.rowPtr, a.colIdx, vals, b, x, r);
     __syncthreads();
-    restrict_rows<T, 3, false, LN>(0, 1, a.nc, a.rPtr, a.rP, a.pRow, P, r, bC, nullptr, nullptr, nullptr);
+    restrict_rows<T, 3, false, LN>(0, 1, a.nc, a.rPtr, a.rRow, static_cast<const T*>(a.R), r, bC, nullptr, nullptr,
+                                   nullptr);
     __syncthreads();
     if (a.dense) {
         dense_apply_rows<T>(a.nc * a.cbs, a.Inv, bC, xC);
@@ -1779,13 +1825,13 @@ void Amg<T>::restrict_to(hipStream_t s, int l, const int* stop)
     // lanes per coarse node: the power of two nearest the mean restriction-list length, 16 to 64
     const long meanLen = A.nc > 0 ? (long)A.rP.size() / A.nc : 0;
     const int ln = meanLen >= 48 ? 64 : (meanLen >= 24 ? 32 : 16);
-    const dim3 g(rows_grid(A.nc, kBlock / ln));
+    const dim3 g((rows_grid(A.nc, kBlock / ln) + 7) & ~7);  // XCD chunk order
     const auto launch = [&](auto kern) {
         if (fuse)
-            hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, s, stop, A.nc, A.dRPtr, A.dRP, A.dPRow, A.P, A.r, N.b, N.Dinv,
+            hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, s, stop, A.nc, A.dRPtr, A.dRRow, A.R, A.r, N.b, N.Dinv,
                                N.lam, N.d);
         else
-            hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, s, stop, A.nc, A.dRPtr, A.dRP, A.dPRow, A.P, A.r, N.b,
+            hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, s, stop, A.nc, A.dRPtr, A.dRRow, A.R, A.r, N.b,
                                nullptr, nullptr, nullptr);
     };
 #define OC_RESTRICT(BS_, F_)                                                      \
@@ -1811,8 +1857,8 @@ void Amg<T>::vcycle_tail(hipStream_t s, int l, const int* stop)
     a.rowPtr = A.dRowPtr;
     a.colIdx = A.dColIdx;
     a.rPtr = A.dRPtr;
-    a.rP = A.dRP;
-    a.pRow = A.dPRow;
+    a.rRow = A.dRRow;
+    a.R = A.R;
     a.pPtr = A.dPPtr;
     a.pCol = A.dPCol;
     a.vals = A.vals;
