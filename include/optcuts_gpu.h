@@ -233,7 +233,7 @@ int oc_solver_apply_precond(oc_ctx* ctx, const double* r, double* z);
  * counterpart. */
 int oc_ic0_set_sweeps(oc_ctx* ctx, int factorSweeps, int applySweeps);
 /* Largest last smoothed multigrid level (nodes) whose part of the V-cycle (its smoothing, residual, transfers and
- * the coarsest solve) runs as one single-workgroup launch instead of seven launches; the result is bit-identical
+ * the coarsest solve) runs as one single-workgroup launch instead of six launches; the result is bit-identical
  * either way. 0 turns it off, -1 restores the built-in limit (128). Takes effect when a multigrid structure is
  * next built (oc_newton_init, a re-mesh that rebuilds it, oc_solver_set_pattern + oc_solver_factorize). No
  * reference counterpart (diagnostics and tests). */

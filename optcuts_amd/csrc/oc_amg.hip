@@ -1171,14 +1171,15 @@ __global__ void __launch_bounds__(kBlock) k_residual(const int* __restrict__ sto
 
 // post-smoothing, first step from the prolongated x: d = D^-1 (b - A x) / theta (row_grid workgroups)
 template <typename T, int BS, typename B>
-__device__ __forceinline__ void cheb_post1_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
-                                                const int* __restrict__ colIdx, const T* __restrict__ vals,
-                                                const T* __restrict__ Dinv, const double* __restrict__ lam,
-                                                const B* __restrict__ b, const T* __restrict__ x, T* d)
+__global__ void __launch_bounds__(kBlock) k_cheb_post1(const int* __restrict__ stop, int n, const int* __restrict__ rowPtr,
+                                                       const int* __restrict__ colIdx, const T* __restrict__ vals,
+                                                       const T* __restrict__ Dinv, const double* __restrict__ lam,
+                                                       const B* __restrict__ b, const T* __restrict__ x, T* d)
 {
+    if (stop && *stop) return;
     constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
     const ChebP cp = cheb_params(*lam);
-    const RowChunk rc = row_chunk<BS>(n, blk, G);
+    const RowChunk rc = row_chunk<BS>(n, blockIdx.x, gridDim.x);
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
     for (int p = 0; p < rc.passes; ++p) {
         RowPass<T, BS, UNROLL> rp;
@@ -1210,16 +1211,6 @@ __device__ __forceinline__ void cheb_post1_rows(int blk, int G, int n, const int
             }
         }
     }
-}
-
-template <typename T, int BS, typename B>
-__global__ void __launch_bounds__(kBlock) k_cheb_post1(const int* __restrict__ stop, int n, const int* __restrict__ rowPtr,
-                                                       const int* __restrict__ colIdx, const T* __restrict__ vals,
-                                                       const T* __restrict__ Dinv, const double* __restrict__ lam,
-                                                       const B* __restrict__ b, const T* __restrict__ x, T* d)
-{
-    if (stop && *stop) return;
-    cheb_post1_rows<T, BS, B>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, b, x, d);
 }
 
 // bc_c = sum over P blocks (u,c) of P^T res_u, LN lanes per coarse node (the launcher picks LN from the mean
@@ -1294,12 +1285,13 @@ __global__ void __launch_bounds__(kBlock) k_restrict(const int* __restrict__ sto
 // partial sums combined by shuffles): the few blocks of a row are loaded together instead of one after another
 constexpr int kProlongLanes = 4;
 template <typename T, int BS>
-__device__ __forceinline__ void prolong_rows(int blk, int n, const int* __restrict__ pPtr,
-                                             const int* __restrict__ pCol, const T* __restrict__ P,
-                                             const T* __restrict__ xc, T* x)
+__global__ void __launch_bounds__(kBlock) k_prolong(const int* __restrict__ stop, int n, const int* __restrict__ pPtr,
+                                                    const int* __restrict__ pCol, const T* __restrict__ P,
+                                                    const T* __restrict__ xc, T* x)
 {
+    if (stop && *stop) return;
     constexpr int LN = kProlongLanes;
-    const int t = blk * kBlock + threadIdx.x;
+    const int t = blockIdx.x * kBlock + threadIdx.x;
     const int u = t / LN, lane = t % LN;
     double s[BS] = {};
     if (u < n) {
@@ -1322,12 +1314,83 @@ __device__ __forceinline__ void prolong_rows(int blk, int n, const int* __restri
     }
 }
 
+// Coarse correction and the first post-smoothing step in one pass: x += P xc and d = D^-1 (b - A x) / theta, where
+// the residual after the correction is res - (A P) xc with res the residual that was restricted and T = A P the
+// product the set-up formed for the Galerkin operator. T's rows hold the columns of P's and a few more, both read
+// the short coarse vector, and the fine x is neither written in between nor gathered: one launch less, and on the
+// coarse levels fewer bytes (6 blocks a row in T against 13 in A; 1M faces, level 1: 21.3 -> 15.0 us, 200k faces
+// 8.8 -> 5.4). On the finest level T is as large as A (273 against 256 bytes a row) and evicts it from the caches
+// between the smoothing steps that do read A, so only the saved launch counts there: up to kCorrectMaxFine rows.
+// Whole Newton step, this pass against prolongation + product: 25k rows 1546 / 1565 us, 51k 2020 / 2043, 100k 2988 /
+// 3016, 203k 4953 / 4809, 501k 9084 / 8977. kCorrectLanes lanes per fine row.
+constexpr int kCorrectLanes = 8;
+constexpr int kCorrectMaxFine = 131072;
 template <typename T, int BS>
-__global__ void __launch_bounds__(kBlock) k_prolong(const int* __restrict__ stop, int n, const int* __restrict__ pPtr, const int* __restrict__ pCol,
-                                                    const T* __restrict__ P, const T* __restrict__ xc, T* x)
+__device__ __forceinline__ void correct_rows(int blk, int G, int n, const int* __restrict__ pPtr,
+                                             const int* __restrict__ pCol, const T* __restrict__ P,
+                                             const int* __restrict__ tPtr, const int* __restrict__ tCol,
+                                             const T* __restrict__ Tv, const T* __restrict__ Dinv,
+                                             const double* __restrict__ lam, const T* __restrict__ xc,
+                                             const T* __restrict__ res, T* x, T* d)
+{
+    constexpr int LN = kCorrectLanes, RPP = kBlock / LN;
+    const double theta = cheb_params(*lam).theta;
+    const int c = (n + G - 1) / G;
+    const int r0 = xcd_chunk(blk, G) * c, r1 = min(n, r0 + c);
+    const int sub = threadIdx.x / LN, lane = threadIdx.x % LN;
+    for (int u = r0 + sub; u < r1; u += RPP) {
+        const int j0 = pPtr[u], j1 = pPtr[u + 1], t0 = tPtr[u], t1 = tPtr[u + 1];
+        double Dm[BS * BS], ro[BS], xo[BS], s[2 * BS] = {};  // (A P) xc, then P xc
+        if (lane == 0) {
+            ld_block<BS>(Dinv + (size_t)u * BS * BS, Dm);
+            ld_vec<BS>(res, u, ro);
+            ld_vec<BS>(x, u, xo);
+        }
+        for (int t = t0 + lane; t < t1; t += LN) {
+            T a[BS * NS], v[NS];
+            ld_blk<BS * NS>(Tv + (size_t)t * BS * NS, a);
+            ld_blk<NS>(xc + (size_t)tCol[t] * NS, v);
+#pragma unroll
+            for (int i = 0; i < BS; ++i)
+#pragma unroll
+                for (int k = 0; k < NS; ++k) s[i] += (double)a[i * NS + k] * (double)v[k];
+        }
+        for (int j = j0 + lane; j < j1; j += LN) {
+            T a[BS * NS], v[NS];
+            ld_blk<BS * NS>(P + (size_t)j * BS * NS, a);
+            ld_blk<NS>(xc + (size_t)pCol[j] * NS, v);
+#pragma unroll
+            for (int i = 0; i < BS; ++i)
+#pragma unroll
+                for (int k = 0; k < NS; ++k) s[BS + i] += (double)a[i * NS + k] * (double)v[k];
+        }
+        group_sum<LN, 2 * BS>(s);
+        if (lane == 0) {
+            T dt[BS], xt[BS];
+#pragma unroll
+            for (int i = 0; i < BS; ++i) {
+                double t = 0.0;
+#pragma unroll
+                for (int k = 0; k < BS; ++k) t += Dm[i * BS + k] * (ro[k] - s[k]);
+                dt[i] = (T)(t / theta);
+                xt[i] = (T)(xo[i] + s[BS + i]);
+            }
+            st_vec<BS>(d, u, dt);
+            st_vec<BS>(x, u, xt);
+        }
+    }
+}
+
+template <typename T, int BS>
+__global__ void __launch_bounds__(kBlock) k_correct(const int* __restrict__ stop, int n, const int* __restrict__ pPtr,
+                                                    const int* __restrict__ pCol, const T* __restrict__ P,
+                                                    const int* __restrict__ tPtr, const int* __restrict__ tCol,
+                                                    const T* __restrict__ Tv, const T* __restrict__ Dinv,
+                                                    const double* __restrict__ lam, const T* __restrict__ xc,
+                                                    const T* __restrict__ res, T* x, T* d)
 {
     if (stop && *stop) return;
-    prolong_rows<T, BS>(blockIdx.x, n, pPtr, pCol, P, xc, x);
+    correct_rows<T, BS>(blockIdx.x, gridDim.x, n, pPtr, pCol, P, tPtr, tCol, Tv, Dinv, lam, xc, res, x, d);
 }
 
 template <typename T>
@@ -1390,7 +1453,7 @@ struct Amg<T>::Level : AmgHostLevel {
     // device
     int *dRowPtr = nullptr, *dColIdx = nullptr, *dDiagPos = nullptr;
     int *dAggPtr = nullptr, *dAggMem = nullptr, *dPPtr = nullptr, *dPCol = nullptr, *dPRow = nullptr,
-        *dPsPtr = nullptr, *dPsA = nullptr, *dRPtr = nullptr, *dRRow = nullptr, *dRPos = nullptr, *dTcPtr = nullptr, *dTcA = nullptr,
+        *dPsPtr = nullptr, *dPsA = nullptr, *dRPtr = nullptr, *dRRow = nullptr, *dRPos = nullptr, *dTPtr = nullptr, *dTCol = nullptr, *dTcPtr = nullptr, *dTcA = nullptr,
         *dTcP = nullptr, *dAcPtr = nullptr, *dAcP = nullptr, *dAcT = nullptr;
     unsigned char* dPIsTent = nullptr;
     T *vals = nullptr, *Dinv = nullptr, *Pt = nullptr, *P = nullptr, *R = nullptr, *Tv = nullptr;
@@ -1400,7 +1463,7 @@ struct Amg<T>::Level : AmgHostLevel {
     void give_back(Pool& pool)
     {
         for (void* p : {(void*)dRowPtr, (void*)dColIdx, (void*)dDiagPos, (void*)dAggPtr, (void*)dAggMem, (void*)dPPtr,
-                        (void*)dPCol, (void*)dPRow, (void*)dPsPtr, (void*)dPsA, (void*)dRPtr, (void*)dRRow, (void*)dRPos,
+                        (void*)dPCol, (void*)dPRow, (void*)dPsPtr, (void*)dPsA, (void*)dRPtr, (void*)dRRow, (void*)dRPos, (void*)dTPtr, (void*)dTCol,
                         (void*)dTcPtr, (void*)dTcA, (void*)dTcP, (void*)dAcPtr, (void*)dAcP, (void*)dAcT,
                         (void*)dPIsTent, (void*)vals, (void*)Dinv, (void*)Pt, (void*)P, (void*)R, (void*)Tv, (void*)b,
                         (void*)x, (void*)r, (void*)d, (void*)Bnext, (void*)lz, (void*)lam})
@@ -1590,6 +1653,8 @@ int Amg<T>::setup(hipStream_t s, int nV, const std::vector<int>& rowPtr, const s
                 hipLaunchKernelGGL(k_restrict_maps, dim3(grid_for((long)A.rP.size())), dim3(kBlock), 0, s,
                                    (int)A.rP.size(), rP, A.dPRow, A.dRRow, A.dRPos);
             if (rP) pool_.put(rP);
+            up(pool_, s, A.dTPtr, A.tPtr);
+            up(pool_, s, A.dTCol, A.tCol);
             up(pool_, s, A.dTcPtr, A.tcPtr);
             up(pool_, s, A.dTcA, A.tcA);
             up(pool_, s, A.dTcP, A.tcP);
@@ -1757,8 +1822,8 @@ constexpr int kTailMaxNodes = OC_TAIL_MAX_NODES;  // largest last smoothed level
 struct TailArgs {
     // smoothed level (3x3 blocks)
     int n;
-    const int *rowPtr, *colIdx, *rPtr, *rRow, *pPtr, *pCol;
-    const void *vals, *Dinv, *P, *R;
+    const int *rowPtr, *colIdx, *rPtr, *rRow, *pPtr, *pCol, *tPtr, *tCol;
+    const void *vals, *Dinv, *P, *R, *Tv;
     const double* lam;
     void *b, *x, *r, *d;
     // coarsest level
@@ -1794,12 +1859,12 @@ __global__ void __launch_bounds__(kBlock) k_vcycle_tail(const int* __restrict__ 
         }
     }
     __syncthreads();
-    for (int blk = 0; blk * kBlock < a.n * kProlongLanes; ++blk) prolong_rows<T, 3>(blk, a.n, a.pPtr, a.pCol, P, xC, x);
-    __syncthreads();
-    cheb_post1_rows<T, 3, T>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, b, x, d);
+    correct_rows<T, 3>(0, 1, a.n, a.pPtr, a.pCol, P, a.tPtr, a.tCol, static_cast<const T*>(a.Tv), Dinv, a.lam, xC, r, x, d);
     __syncthreads();
     cheb_step_rows<T, 3, 1>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, x, nullptr, nullptr, nullptr);
 }
+
+int correct_grid(int n) { return (rows_grid(n, kBlock / kCorrectLanes) + 7) & ~7; }
 
 template <typename T>
 void Amg<T>::coarse_solve(hipStream_t s, const int* stop)
@@ -1859,6 +1924,9 @@ void Amg<T>::vcycle_tail(hipStream_t s, int l, const int* stop)
     a.rPtr = A.dRPtr;
     a.rRow = A.dRRow;
     a.R = A.R;
+    a.tPtr = A.dTPtr;
+    a.tCol = A.dTCol;
+    a.Tv = A.Tv;
     a.pPtr = A.dPPtr;
     a.pCol = A.dPCol;
     a.vals = A.vals;
@@ -1906,10 +1974,8 @@ void Amg<T>::vcycle(hipStream_t s, int l, const int* stop)
                        A.b, A.x, A.r);
     restrict_to(s, l, stop);
     vcycle(s, l + 1, stop);
-    hipLaunchKernelGGL((k_prolong<T, 3>), dim3(grid_for((long)A.n * kProlongLanes)), dim3(kBlock), 0, s, stop, A.n,
-                       A.dPPtr, A.dPCol, A.P, N.x, A.x);
-    hipLaunchKernelGGL((k_cheb_post1<T, 3, T>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
-                       A.Dinv, A.lam, A.b, A.x, A.d);
+    hipLaunchKernelGGL((k_correct<T, 3>), dim3(correct_grid(A.n)), dim3(kBlock), 0, s, stop, A.n, A.dPPtr, A.dPCol,
+                       A.P, A.dTPtr, A.dTCol, A.Tv, A.Dinv, A.lam, N.x, A.r, A.x, A.d);
     hipLaunchKernelGGL((k_cheb_step<T, 3, 1>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
                        A.Dinv, A.lam, A.d, A.x, nullptr, nullptr, nullptr);
 }
@@ -1936,10 +2002,15 @@ void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, co
                        A.vals, r, A.x, A.r);
     restrict_to(s, 0, stop);
     vcycle(s, 1, stop);
-    hipLaunchKernelGGL((k_prolong<T, 2>), dim3(grid_for((long)A.n * kProlongLanes)), dim3(kBlock), 0, s, stop, A.n,
-                       A.dPPtr, A.dPCol, A.P, N.x, A.x);
-    hipLaunchKernelGGL((k_cheb_post1<T, 2, double>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
-                       A.vals, A.Dinv, A.lam, r, A.x, A.d);
+    if (A.n <= kCorrectMaxFine) {
+        hipLaunchKernelGGL((k_correct<T, 2>), dim3(correct_grid(A.n)), dim3(kBlock), 0, s, stop, A.n, A.dPPtr, A.dPCol,
+                           A.P, A.dTPtr, A.dTCol, A.Tv, A.Dinv, A.lam, N.x, A.r, A.x, A.d);
+    } else {
+        hipLaunchKernelGGL((k_prolong<T, 2>), dim3(grid_for((long)A.n * kProlongLanes)), dim3(kBlock), 0, s, stop, A.n,
+                           A.dPPtr, A.dPCol, A.P, N.x, A.x);
+        hipLaunchKernelGGL((k_cheb_post1<T, 2, double>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
+                           A.vals, A.Dinv, A.lam, r, A.x, A.d);
+    }
     hipLaunchKernelGGL((k_cheb_step<T, 2, 2>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
                        A.Dinv, A.lam, A.d, A.x, r, z, rzPart);
 }
