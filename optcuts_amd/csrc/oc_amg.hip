@@ -64,20 +64,6 @@ __device__ __forceinline__ void row_mv(const int* __restrict__ rowPtr, const int
         for (int i = 0; i < BS; ++i) y[i] += __shfl_xor(y[i], off, LANES);
 }
 
-// Chebyshev parameters on [lmax/30, lmax], lmax = 1.1 * lambda estimate
-struct ChebP {
-    double theta, delta, sigma;
-};
-__device__ __forceinline__ ChebP cheb_params(double lam)
-{
-    const double lmax = 1.1 * lam, lmin = lmax / 30.0;
-    ChebP p;
-    p.theta = 0.5 * (lmax + lmin);
-    p.delta = 0.5 * (lmax - lmin);
-    p.sigma = p.theta / p.delta;
-    return p;
-}
-
 // ---------------------------------------------------------------------------- numeric set-up kernels
 template <typename TI, typename T>
 __global__ void __launch_bounds__(kBlock) k_cvt(long n, const TI* __restrict__ in, T* out)
@@ -1027,7 +1013,7 @@ __global__ void __launch_bounds__(256) k_dense_inverse(int nn, int bs, const int
 // (Keeping residual, direction and iterate as vectors of their own moved 64
 // to 96 more bytes per fine row and step beside the ~300 of the row's blocks.)
 //
-// pre-smoothing, first step from x = 0: d = D^-1 b / theta
+// pre-smoothing, first step from x = 0: d = D^-1 b / theta (for callers other than the PCG, whose kernels do it)
 template <typename T, int BS>
 __global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ stop, int n,
                                                       const double* __restrict__ b, const T* __restrict__ Dinv,
@@ -1058,12 +1044,36 @@ __global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ st
 // (post-smoothing): x += d + d'; 2 (the finest level's last step): z = x + d +
 // d' in FP64 and partial records of rFinal.z per workgroup. d is read for the
 // neighbours and not written. Launch with row_grid workgroups.
-template <typename T, int BS, int KIND>
+// Whether the PCG's residual is within its tolerance (then its control record is set as k_pcg_spmv sets it): every
+// workgroup sums the r.r records itself, in the same order. bb, the right-hand side's norm, is what the first
+// residual's records hold; k_pcg_spmv keeps it from then on.
+__device__ __forceinline__ bool pcg_converged(const PcgStage& st)
+{
+    double acc[1] = {0.0};
+    for (int b = threadIdx.x; b < st.nRr; b += blockDim.x) acc[0] += st.partRr[(size_t)b * st.sRr];
+    const int it = st.ctrl->itNext;
+    const double bbKept = st.ctrl->bb, tol2 = st.ctrl->tol2;
+    block_sum<1>(acc);
+    __shared__ double sh;
+    if (threadIdx.x == 0) sh = acc[0];
+    __syncthreads();
+    const double rr = sh, bb = it == 0 ? rr : bbKept;
+    if (bb != 0.0 && !(rr <= tol2 * bb)) return false;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (it == 0) st.ctrl->bb = bb;
+        st.ctrl->rr = rr;
+        st.ctrl->iter = it;
+        st.ctrl->done = 1;
+    }
+    return true;
+}
+
+template <typename T, int BS, int KIND, bool CHECK = false>
 __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
                                                const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                const T* __restrict__ Dinv, const double* __restrict__ lam,
                                                const T* __restrict__ d, T* x, const double* __restrict__ rFinal,
-                                               double* zFinal, double* rzPart)
+                                               double* zFinal, double* rzPart, const PcgStage& st = {})
 {
     constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
     const ChebP cp = cheb_params(*lam);
@@ -1085,6 +1095,7 @@ __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int*
                 if (KIND >= 1) ld_vec<BS>(x, rp.u[q], xo[q]);
                 if (KIND == 2) ld_vec<BS>(rFinal, rp.u[q], rf[q]);
             }
+        if (CHECK && p == 0 && pcg_converged(st)) return;
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q) {
             double w[BS];
@@ -1128,6 +1139,19 @@ __global__ void __launch_bounds__(kBlock) k_cheb_step(const int* __restrict__ st
 {
     if (stop && *stop) return;
     cheb_step_rows<T, BS, KIND>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, d, x, rFinal, zFinal, rzPart);
+}
+
+// The finest level's first kernel of a V-cycle inside a PCG: the pre-smoothing step behind the convergence test of the
+// residual it smooths, whose record sums overlap the row loads.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_cheb_first(int n, const int* __restrict__ rowPtr,
+                                                       const int* __restrict__ colIdx, const T* __restrict__ vals,
+                                                       const T* __restrict__ Dinv, const double* __restrict__ lam,
+                                                       const T* __restrict__ d, T* x, PcgStage st)
+{
+    if (st.ctrl->done) return;
+    cheb_step_rows<T, 2, 0, true>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, d, x, nullptr, nullptr,
+                                  nullptr, st);
 }
 
 // residual res = b - A x (row_grid workgroups); b is the FP64 right-hand side itself on the finest level
@@ -1981,7 +2005,7 @@ void Amg<T>::vcycle(hipStream_t s, int l, const int* stop)
 }
 
 template <typename T>
-void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop)
+void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop, const PcgStage* pcg)
 {
     Level& A = *L[0];
     const int g = row_grid(A.n, 2);
@@ -1994,10 +2018,15 @@ void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, co
     }
     // the finest level reads the FP64 residual in place; its last step writes z (FP64) and the r.z records
     Level& N = *L[1];
-    hipLaunchKernelGGL((k_cheb_pre1<T, 2>), dim3(rows_grid(A.n, kBlock)), dim3(kBlock), 0, s, stop, A.n, r, A.Dinv,
-                       A.lam, A.d);
-    hipLaunchKernelGGL((k_cheb_step<T, 2, 0>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
-                       A.Dinv, A.lam, A.d, A.x, nullptr, nullptr, nullptr);
+    if (pcg) {
+        hipLaunchKernelGGL(k_cheb_first<T>, dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.dColIdx, A.vals, A.Dinv,
+                           A.lam, A.d, A.x, *pcg);
+    } else {
+        hipLaunchKernelGGL((k_cheb_pre1<T, 2>), dim3(rows_grid(A.n, kBlock)), dim3(kBlock), 0, s, stop, A.n, r, A.Dinv,
+                           A.lam, A.d);
+        hipLaunchKernelGGL((k_cheb_step<T, 2, 0>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
+                           A.vals, A.Dinv, A.lam, A.d, A.x, nullptr, nullptr, nullptr);
+    }
     hipLaunchKernelGGL((k_residual<T, 2, double>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx,
                        A.vals, r, A.x, A.r);
     restrict_to(s, 0, stop);
@@ -2013,6 +2042,13 @@ void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, co
     }
     hipLaunchKernelGGL((k_cheb_step<T, 2, 2>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
                        A.Dinv, A.lam, A.d, A.x, r, z, rzPart);
+}
+
+template <typename T>
+FirstStep Amg<T>::first_step() const
+{
+    if (L.size() < 2) return {};  // a single level is solved, not smoothed
+    return FirstStep{L[0]->Dinv, L[0]->lam, L[0]->d, std::is_same<T, float>::value ? 1 : 0};
 }
 
 template class Amg<float>;

@@ -89,7 +89,9 @@ public:
     // z = M r (one V-cycle) for FP64 vectors of 2*nV; writes per-workgroup
     // partial records of r.z into rzPart (rz_records() of them). Every
     // kernel returns at once while *stop is nonzero (a converged PCG).
-    void apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop) override;
+    void apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop,
+               const PcgStage* pcg = nullptr) override;
+    FirstStep first_step() const override;
 
     int rz_records() const override;
     int levels() const override { return (int)L.size(); }

@@ -444,9 +444,16 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
     double* partS = c->dPcgPart.as<double>() + 4 * (size_t)GU;
     double* partRZ = partS + GS;
     const double* Minv = amg ? nullptr : P.dMinv.as<double>();
+    // A multigrid's first smoothing step runs in the kernels that write the residual, and its first kernel stops the
+    // iteration when that residual is within the tolerance (the V-cycle on a converged residual has no use).
+    const oc::FirstStep first = amg ? amg->first_step() : oc::FirstStep{};
+    const auto precondition = [&](const double* pu) {
+        const oc::PcgStage stage{pu + 1, GU, 2, ctrl};
+        amg->apply(c->stream, c->dR.as<double>(), c->dZ.as<double>(), partRZ, &ctrl->done, first.d ? &stage : nullptr);
+    };
     oc::launch_pcg_init(c->stream, nV, b, Minv, c->dX.as<double>(), c->dR.as<double>(), c->dZ.as<double>(), partU[0],
-                        ctrl);
-    if (amg) amg->apply(c->stream, c->dR.as<double>(), c->dZ.as<double>(), partRZ, &ctrl->done);
+                        ctrl, first);
+    if (amg) precondition(partU[0]);
     double* pbuf[2] = {c->dP0.as<double>(), c->dP1.as<double>()};
     // One iteration's launches. The kernels take the iteration number from
     // the control record, so the launches depend only on its parity (which
@@ -464,8 +471,8 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
                                 c->dZ.as<double>(), pOld, pNew, c->dQ.as<double>(), pu, GU, 2, pu + 1, GU, 2, partS,
                                 ctrl);
         oc::launch_pcg_update(c->stream, nV, pNew, c->dQ.as<double>(), Minv, c->dX.as<double>(), c->dR.as<double>(),
-                              c->dZ.as<double>(), partS, partU[par ^ 1], ctrl);
-        if (amg) amg->apply(c->stream, c->dR.as<double>(), c->dZ.as<double>(), partRZ, &ctrl->done);
+                              c->dZ.as<double>(), partS, partU[par ^ 1], ctrl, first);
+        if (amg) precondition(partU[par ^ 1]);
     };
     // Graphs: 0 an even iteration, 1 an odd one, 2 an even+odd pair, 3 a run
     // of kChain pairs. They name these buffers and sizes; anything else
@@ -527,8 +534,9 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
     // Iterations are queued in batches and the control record read back after
     // each. Queued iterations past convergence still launch (and return at
     // once), so the first batch is sized by the caller's hint (the previous
-    // solve's iteration count, +1 for the converging check), then grows.
-    int batch = hint > 0 ? hint + 1 : (amg ? 8 : 32);
+    // solve's iteration count, +1 for the converging check unless the preconditioner makes it at the end of the
+    // iteration), then grows.
+    int batch = hint > 0 ? hint + (first.d ? 0 : 1) : (amg ? 8 : 32);
     int next = amg ? 2 : 32;
     const int maxBatch = amg ? 32 : 512;
     for (;;) {

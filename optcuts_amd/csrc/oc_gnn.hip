@@ -1090,7 +1090,7 @@ void Gnn::forward(hipStream_t s, const void* vals, int vals32)
 
 int Gnn::rz_records() const { return blocks_for(nV, kBlock); }
 
-void Gnn::apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop)
+void Gnn::apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop, const PcgStage*)
 {
     const int g = blocks_for(nV, kBlock);
     const float4* Ci = reinterpret_cast<const float4*>(dCinv);

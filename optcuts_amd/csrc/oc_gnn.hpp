@@ -75,7 +75,8 @@ public:
     void forward(hipStream_t s, const void* vals, int vals32);
     // z = M^-1 r for FP64 vectors of 2 nV; per-workgroup records of r.z in
     // rzPart (rz_records() of them). Returns at once while *stop != 0.
-    void apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop) override;
+    void apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop,
+               const PcgStage* pcg = nullptr) override;
     int rz_records() const override;
 
     // Training (after forward): adds dL/dtheta to grads(), *dLoss (device) += L.

@@ -278,7 +278,7 @@ void Ic0::numeric(hipStream_t s, const double* vals)
 
 int Ic0::rz_records() const { return row_grid(nV_); }
 
-void Ic0::apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop)
+void Ic0::apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop, const PcgStage*)
 {
     const int n = nV_, g = row_grid(n), m = applySweeps_;
     const double4* L = reinterpret_cast<const double4*>(dL_[factorSweeps_ & 1]);

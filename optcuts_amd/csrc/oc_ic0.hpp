@@ -45,7 +45,8 @@ public:
     bool ready() const { return nV_ > 0; }
     // Factor of the FP64 block values (double4 per block of the pattern) on the stream.
     void numeric(hipStream_t s, const double* vals);
-    void apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop) override;
+    void apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop,
+               const PcgStage* pcg = nullptr) override;
     int rz_records() const override;
     // Diagonal blocks that took the diagonal-part fallback in the last numeric() (synchronises the stream).
     int breakdowns(hipStream_t s);

@@ -792,7 +792,8 @@ void launch_ls_decide_commit(hipStream_t s, const double* cand, const unsigned l
 //              r -= alpha q; z = M r; partials of r.z and r.r.
 // With an external preconditioner (Minv == nullptr) init/update leave z
 // alone and the caller applies M between update(i) and spmv(i+1), handing
-// its own r.z partial records to spmv.
+// its own r.z partial records to spmv; a multigrid's row-local first step is
+// computed where the residual is written (FirstStep).
 // Scalars shared across kernels (rz_i, bb, done) are written by block 0 only,
 // into slots that no other block of the same kernel reads. No atomics and no
 // device-scope fences: kernel boundaries order everything.
@@ -844,11 +845,32 @@ __device__ __forceinline__ void row_chunk(int nV, int& r0, int& r1)
     r1 = min(nV, r0 + chunk);
 }
 
-template <bool APPLY_M>
-__global__ void __launch_bounds__(kBlock) k_pcg_init(int nV, const double2* __restrict__ b,
-                                                     const double* __restrict__ Minv, double2* x, double2* r,
-                                                     double2* z, double* partU, PcgCtrl* ctrl)
+// What init and update do with the residual they write: nothing more (an external preconditioner), z = M r, or the
+// external preconditioner's first step d = Dinv r / theta in double or float.
+enum { kPcgExternal = 0, kPcgApplyM = 1, kPcgFirst64 = 2, kPcgFirst32 = 3 };
+
+template <int MODE>
+__device__ __forceinline__ void pcg_first(const FirstStep& f, double theta, int v, double2 r)
 {
+    if constexpr (MODE == kPcgFirst64) {
+        const double4 m = reinterpret_cast<const double4*>(f.Dinv)[v];
+        reinterpret_cast<double2*>(f.d)[v] =
+            make_double2((m.x * r.x + m.y * r.y) / theta, (m.z * r.x + m.w * r.y) / theta);
+    } else if constexpr (MODE == kPcgFirst32) {
+        const float4 m = reinterpret_cast<const float4*>(f.Dinv)[v];
+        reinterpret_cast<float2*>(f.d)[v] =
+            make_float2((float)(((double)m.x * r.x + (double)m.y * r.y) / theta),
+                        (float)(((double)m.z * r.x + (double)m.w * r.y) / theta));
+    }
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(kBlock) k_pcg_init(int nV, const double2* __restrict__ b,
+                                                     const double* __restrict__ Minv, FirstStep first, double2* x,
+                                                     double2* r, double2* z, double* partU, PcgCtrl* ctrl)
+{
+    constexpr bool APPLY_M = MODE == kPcgApplyM;
+    const double theta = MODE >= kPcgFirst64 ? cheb_params(*first.lam).theta : 0.0;
     int r0, r1;
     row_chunk(nV, r0, r1);
     double acc[2] = {0.0, 0.0};
@@ -861,6 +883,7 @@ __global__ void __launch_bounds__(kBlock) k_pcg_init(int nV, const double2* __re
             z[v] = zv;
             acc[0] += bv.x * zv.x + bv.y * zv.y;
         }
+        pcg_first<MODE>(first, theta, v, bv);
         acc[1] += bv.x * bv.x + bv.y * bv.y;
     }
     block_sum<2>(acc);
@@ -887,16 +910,17 @@ int pcg_grid_spmv(int nV)
 }
 
 void launch_pcg_init(hipStream_t s, int nV, const double* b, const double* Minv, double* x, double* r, double* z,
-                     double* partU, PcgCtrl* ctrl)
+                     double* partU, PcgCtrl* ctrl, const FirstStep& first)
 {
-    if (Minv)
-        hipLaunchKernelGGL(k_pcg_init<true>, dim3(pcg_grid_update(nV)), dim3(kBlock), 0, s, nV,
-                           reinterpret_cast<const double2*>(b), Minv, reinterpret_cast<double2*>(x),
+    const auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(pcg_grid_update(nV)), dim3(kBlock), 0, s, nV,
+                           reinterpret_cast<const double2*>(b), Minv, first, reinterpret_cast<double2*>(x),
                            reinterpret_cast<double2*>(r), reinterpret_cast<double2*>(z), partU, ctrl);
-    else
-        hipLaunchKernelGGL(k_pcg_init<false>, dim3(pcg_grid_update(nV)), dim3(kBlock), 0, s, nV,
-                           reinterpret_cast<const double2*>(b), Minv, reinterpret_cast<double2*>(x),
-                           reinterpret_cast<double2*>(r), reinterpret_cast<double2*>(z), partU, ctrl);
+    };
+    if (Minv) launch(k_pcg_init<kPcgApplyM>);
+    else if (!first.d) launch(k_pcg_init<kPcgExternal>);
+    else if (first.f32) launch(k_pcg_init<kPcgFirst32>);
+    else launch(k_pcg_init<kPcgFirst64>);
 }
 
 // q_v = sum_k A_vk (z_w + beta p_w) over the row's blocks, kSpmvLanes lanes per row.
@@ -1062,14 +1086,17 @@ void launch_pcg_spmv(hipStream_t s, int nV, const int* rowPtr, const int* colIdx
                            reinterpret_cast<double2*>(q), partRz, nRz, sRz, partRr, nRr, sRr, partS, ctrl);
 }
 
-template <bool APPLY_M>
+template <int MODE>
 __global__ void __launch_bounds__(kBlock) k_pcg_update(int nV, const double2* __restrict__ p,
                                                        const double2* __restrict__ q,
-                                                       const double* __restrict__ Minv, double2* x, double2* r,
+                                                       const double* __restrict__ Minv, FirstStep first, double2* x,
+                                                       double2* r,
                                                        double2* z, const double* __restrict__ partS, int nPartS,
                                                        double* partUout, PcgCtrl* ctrl)
 {
+    constexpr bool APPLY_M = MODE == kPcgApplyM;
     if (ctrl->done) return;
+    const double theta = MODE >= kPcgFirst64 ? cheb_params(*first.lam).theta : 0.0;
     double pq[1];
     reduce_partials<1>(partS, nPartS, pq);
     if (!(pq[0] > 0.0)) {  // breakdown: A not positive definite along p
@@ -1096,6 +1123,7 @@ __global__ void __launch_bounds__(kBlock) k_pcg_update(int nV, const double2* __
             z[v] = zv;
             acc[0] += rv.x * zv.x + rv.y * zv.y;
         }
+        pcg_first<MODE>(first, theta, v, rv);
         acc[1] += rv.x * rv.x + rv.y * rv.y;
     }
     block_sum<2>(acc);
@@ -1106,18 +1134,19 @@ __global__ void __launch_bounds__(kBlock) k_pcg_update(int nV, const double2* __
 }
 
 void launch_pcg_update(hipStream_t s, int nV, const double* pNew, const double* q, const double* Minv,
-                       double* x, double* r, double* z, const double* partS, double* partUout, PcgCtrl* ctrl)
+                       double* x, double* r, double* z, const double* partS, double* partUout, PcgCtrl* ctrl,
+                       const FirstStep& first)
 {
-    if (Minv)
-        hipLaunchKernelGGL(k_pcg_update<true>, dim3(pcg_grid_update(nV)), dim3(kBlock), 0, s, nV,
-                           reinterpret_cast<const double2*>(pNew), reinterpret_cast<const double2*>(q), Minv,
+    const auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(pcg_grid_update(nV)), dim3(kBlock), 0, s, nV,
+                           reinterpret_cast<const double2*>(pNew), reinterpret_cast<const double2*>(q), Minv, first,
                            reinterpret_cast<double2*>(x), reinterpret_cast<double2*>(r),
                            reinterpret_cast<double2*>(z), partS, pcg_grid_spmv(nV), partUout, ctrl);
-    else
-        hipLaunchKernelGGL(k_pcg_update<false>, dim3(pcg_grid_update(nV)), dim3(kBlock), 0, s, nV,
-                           reinterpret_cast<const double2*>(pNew), reinterpret_cast<const double2*>(q), Minv,
-                           reinterpret_cast<double2*>(x), reinterpret_cast<double2*>(r),
-                           reinterpret_cast<double2*>(z), partS, pcg_grid_spmv(nV), partUout, ctrl);
+    };
+    if (Minv) launch(k_pcg_update<kPcgApplyM>);
+    else if (!first.d) launch(k_pcg_update<kPcgExternal>);
+    else if (first.f32) launch(k_pcg_update<kPcgFirst32>);
+    else launch(k_pcg_update<kPcgFirst64>);
 }
 
 // ----------------------------------------------------------------------------

@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "oc_precond.hpp"
+
 namespace oc {
 
 // Triangle set of one system, SoA in HBM. Triangles [0, nFmesh) are mesh
@@ -126,18 +128,6 @@ constexpr int kPcgLanes = 4;      // lanes per block-row in the PCG product
 constexpr int kPcgRows = 2;       // block rows per lane group and pass in the PCG product
 constexpr int kPcgMaxGrid = 1024;  // workgroups of the PCG kernels (bounds the partial records)
 
-// The iteration number lives here, not in launch arguments, so that every
-// iteration of one parity launches identical arguments (graph replay):
-// k_pcg_init sets itNext = 0; k_pcg_spmv reads itNext and records it in itCur
-// (and iter); k_pcg_update reads itCur and sets itNext = itCur + 1. Each field
-// is written by one kernel and read only by the next.
-struct PcgCtrl {
-    double bb, tol2, rr, pad0;
-    double rzSlot[2];
-    int iter, maxit, done, itNext;
-    int itCur, pad1, pad2, pad3;
-};
-
 // Workgroups of the update/init kernels and of the SpMV kernel for nV rows.
 int pcg_grid_update(int nV);
 int pcg_grid_spmv(int nV);
@@ -146,14 +136,17 @@ int pcg_grid_spmv(int nV);
 // when Minv is given: the block-Jacobi M is applied inline); partS: per-block
 // p.q records of spmv(i) read by update(i). spmv(i) sums r.z over nRz
 // records of stride sRz and r.r over nRr records of stride sRr.
+// first (without Minv): the external preconditioner's first step, computed
+// by init / update(i) from the residual they write.
 void launch_pcg_init(hipStream_t s, int nV, const double* b, const double* Minv, double* x, double* r, double* z,
-                     double* partU, PcgCtrl* ctrl);
+                     double* partU, PcgCtrl* ctrl, const FirstStep& first = {});
 // vals: double4 blocks, or float4 blocks when vals32 (FP64 arithmetic either way).
 void launch_pcg_spmv(hipStream_t s, int nV, const int* rowPtr, const int* colIdx, const void* vals,
                      int vals32, const double* z, const double* pOld, double* pNew, double* q, const double* partRz,
                      int nRz, int sRz, const double* partRr, int nRr, int sRr, double* partS, PcgCtrl* ctrl);
 void launch_pcg_update(hipStream_t s, int nV, const double* pNew, const double* q, const double* Minv,
-                       double* x, double* r, double* z, const double* partS, double* partUout, PcgCtrl* ctrl);
+                       double* x, double* r, double* z, const double* partS, double* partUout, PcgCtrl* ctrl,
+                       const FirstStep& first = {});
 
 // y = A x (2x2-block CSR; float blocks when vals32).
 void launch_spmv(hipStream_t s, int nV, const int* rowPtr, const int* colIdx, const void* vals, int vals32,
