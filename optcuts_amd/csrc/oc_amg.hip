@@ -171,6 +171,15 @@ __device__ __forceinline__ double hash_unit(unsigned int i)
     return (double)(i & 0xffffff) / (double)0x800000 - 1.0;
 }
 
+template <int LANES, int NV>
+__device__ __forceinline__ void group_sum(double (&v)[NV])
+{
+#pragma unroll
+    for (int off = LANES / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) v[i] += __shfl_xor(v[i], off, LANES);
+}
+
 // lambda_max(D^-1 A) by Lanczos in the D inner product (D^-1 A is self-adjoint
 // there; D is the block diagonal with zero diagonal entries set to 1, as in
 // k_blockinv). Ritz values approach the extreme eigenvalues far faster than
@@ -558,33 +567,36 @@ __global__ void __launch_bounds__(kBlock) k_lanczos(int j, int nsteps, int n, co
 // then needs many more steps); weighting the start by g_u^4 puts its mass
 // where those vectors live. h = hash * g^4, W_{-1} = D^-1 h, partial records
 // of h^T D^-1 h = |W_{-1}|_D^2 and of max g (gPart).
+// One lane group per row as in the row kernels (a thread per row walked a coarse row's 10-30 blocks one after
+// another: 13-15 us on every coarse level, now 4-5).
 template <typename T, int BS>
 __global__ void __launch_bounds__(kBlock) k_lanczos_start(int n, const int* __restrict__ rowPtr,
                                                           const T* __restrict__ vals, const T* __restrict__ Dinv,
                                                           double* W, double* partOut, double* gPart, double* coef,
                                                           int nsteps)
 {
-    int r0, r1;
-    chunk_rows(n, r0, r1);
+    constexpr int LN = RowShape<BS>::lanes, RPP = kBlock / LN;
+    const RowChunk rc = row_chunk<BS>(n, blockIdx.x, gridDim.x);
+    const int sub = threadIdx.x / LN, lane = threadIdx.x % LN;
     double acc[2] = {0.0, 0.0};
     double gmax = 0.0;
-    for (int u = r0 + (int)threadIdx.x; u < r1; u += kBlock) {
-        const T* D = Dinv + (size_t)u * BS * BS;
-        double rs[BS];
-#pragma unroll
-        for (int i = 0; i < BS; ++i) rs[i] = 0.0;
-        for (int k = rowPtr[u]; k < rowPtr[u + 1]; ++k) {
-            const T* a = vals + (size_t)k * BS * BS;
+    for (int u = rc.r0 + sub; u < rc.r1; u += RPP) {
+        double D[BS * BS], rs[BS] = {};
+        ld_block<BS>(Dinv + (size_t)u * BS * BS, D);
+        for (int k = rowPtr[u] + lane; k < rowPtr[u + 1]; k += LN) {
+            double a[BS * BS];
+            ld_block<BS>(vals + (size_t)k * BS * BS, a);
 #pragma unroll
             for (int i = 0; i < BS; ++i)
 #pragma unroll
                 for (int j = 0; j < BS; ++j) {
                     double s = 0.0;
 #pragma unroll
-                    for (int c = 0; c < BS; ++c) s += (double)D[i * BS + c] * (double)a[c * BS + j];
+                    for (int c = 0; c < BS; ++c) s += D[i * BS + c] * a[c * BS + j];
                     rs[i] += fabs(s);
                 }
         }
+        group_sum<LN, BS>(rs);
         double gu = 0.0;
 #pragma unroll
         for (int i = 0; i < BS; ++i) gu = fmax(gu, rs[i]);
@@ -593,14 +605,15 @@ __global__ void __launch_bounds__(kBlock) k_lanczos_start(int n, const int* __re
         double h[BS];
 #pragma unroll
         for (int i = 0; i < BS; ++i) h[i] = hash_unit((unsigned)(u * BS + i)) * w4;
+        if (lane == 0)
 #pragma unroll
-        for (int i = 0; i < BS; ++i) {
-            double s = 0.0;
+            for (int i = 0; i < BS; ++i) {
+                double s = 0.0;
 #pragma unroll
-            for (int c = 0; c < BS; ++c) s += (double)D[i * BS + c] * h[c];
-            W[(size_t)u * BS + i] = s;
-            acc[1] += h[i] * s;
-        }
+                for (int c = 0; c < BS; ++c) s += D[i * BS + c] * h[c];
+                W[(size_t)u * BS + i] = s;
+                acc[1] += h[i] * s;
+            }
     }
     block_sum<2>(acc);
     // block maximum of g (values are >= 0)
@@ -618,76 +631,41 @@ __global__ void __launch_bounds__(kBlock) k_lanczos_start(int n, const int* __re
     if (blockIdx.x == 0 && threadIdx.x == 0) coef[2 * kLanczosSteps] = (double)nsteps;
 }
 
-// lam[1] = the Gershgorin bound; lam[0] = the largest eigenvalue of the
-// Lanczos tridiagonal (Sturm-count bisection), or, in the safe mode (no
-// Lanczos steps were run), the Gershgorin bound / 1.1 so that the smoother's
-// interval ends exactly at a guaranteed upper bound.
-__global__ void __launch_bounds__(kBlock) k_lanczos_finish(const double* __restrict__ partIn, int nPartIn,
-                                                           const double* __restrict__ gPart, int safe, int nsteps,
-                                                           double* coef, double* lam)
+// Largest eigenvalue of the m x m tridiagonal (al[0..m), be[i] couples rows i-1 and i), by one wave: multisection on
+// the Sturm count (number of eigenvalues below x), 64 points per round, one per lane, shrink [lo, hi] around it by
+// 65x; counts grow with x, so the first point below which all m eigenvalues lie brackets it. The count is the
+// number of sign changes of the leading minors of T - x I, whose recurrence needs no division (the divisions of
+// the ratio form are a serial chain of 90 of them). The coefficients stay in registers, row i's in lane i; a round
+// is one dependent FP64 chain, so the loop is unrolled enough to take the lane reads off it and no further (a kernel
+// that runs once also waits for its instruction fetch).
+__device__ __forceinline__ double tridiag_top(int m, const double* al, const double* be)
 {
-    __shared__ double red[kBlock];
-    {
-        double g = 0.0;
-        for (int b = threadIdx.x; b < nPartIn; b += blockDim.x) g = fmax(g, gPart[b]);
-        red[threadIdx.x] = g;
-        __syncthreads();
-        for (int w = kBlock / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) {
-            lam[1] = red[0];
-            if (safe) lam[0] = red[0] / 1.1;
-        }
-        if (safe) return;
-    }
-    const int m = (int)coef[2 * kLanczosSteps];
-    if (m == nsteps) {
-        double acc[2] = {0.0, 0.0};
-        for (int b = threadIdx.x; b < nPartIn; b += blockDim.x) {
-            acc[0] += partIn[2 * b];
-            acc[1] += partIn[2 * b + 1];
-        }
-        block_sum<2>(acc);
-        if (threadIdx.x == 0) coef[nsteps - 1] = acc[0];
-        __syncthreads();
-    }
-    if (m == 0) {  // start vector in the null space of A: no information
-        if (threadIdx.x == 0) lam[0] = 1.0;
-        return;
-    }
-    // T: al[0..m), be[i] couples rows i-1 and i (i >= 1)
-    __shared__ double al[kLanczosSteps], be[kLanczosSteps];
-    if ((int)threadIdx.x < m) {
-        al[threadIdx.x] = coef[threadIdx.x];
-        be[threadIdx.x] = coef[kLanczosSteps + threadIdx.x];
-    }
-    __syncthreads();
-    if (threadIdx.x >= kWave) return;  // the rest runs in wave 0
-    const int l = threadIdx.x;
-    // Gershgorin interval of T
-    double lo = 1e300, hi = -1e300;
+    const int l = threadIdx.x % kWave;
+    const double a = l < m ? al[l] : 0.0, b = l > 0 && l < m ? be[l] : 0.0, b2 = b * b;
+    double lo = 1e300, hi = -1e300;  // Gershgorin interval of T
     if (l < m) {
-        const double r = (l > 0 ? fabs(be[l]) : 0.0) + (l + 1 < m ? fabs(be[l + 1]) : 0.0);
-        lo = al[l] - r;
-        hi = al[l] + r;
+        const double r = fabs(b) + (l + 1 < m ? fabs(be[l + 1]) : 0.0);
+        lo = a - r;
+        hi = a + r;
     }
     lo = wave_min(lo);
     hi = wave_max(hi);
-    // Multisection on the Sturm count (number of eigenvalues of T below x):
-    // 64 points per round, one per lane, shrink [lo, hi] around lambda_max by
-    // 65x; counts grow with x, so the first point below which all m eigenvalues
-    // lie brackets lambda_max.
+#pragma unroll 1
     for (int round = 0; round < 6; ++round) {
         const double h = (hi - lo) / (kWave + 1);
         const double x = lo + (l + 1) * h;
         int cnt = 0;
-        double d = 1.0;
-        for (int i = 0; i < m; ++i) {
-            d = al[i] - x - (i > 0 ? be[i] * be[i] / d : 0.0);
-            if (d == 0.0) d = -1e-300;
-            if (d < 0.0) ++cnt;
+        double p0 = 0.0, p1 = 1.0;
+        bool neg = false;
+        static_assert(kLanczosSteps % 5 == 0, "unrolled by 5");
+#pragma unroll 5
+        for (int i = 0; i < kLanczosSteps; ++i) {
+            const double p = (read_lane(a, i) - x) * p1 - read_lane(b2, i) * p0;
+            const bool ng = p == 0.0 ? !neg : p < 0.0;  // a zero minor counts as a change
+            cnt += i < m && ng != neg;
+            neg = ng;
+            p0 = p1;
+            p1 = p;
         }
         const unsigned long long hits = __ballot(cnt == m);
         const int k = hits ? __ffsll((long long)hits) - 1 : kWave;
@@ -695,22 +673,211 @@ __global__ void __launch_bounds__(kBlock) k_lanczos_finish(const double* __restr
         lo = base + k * h;
         if (k < kWave) hi = base + (k + 1) * h;
     }
-    if (l == 0) lam[0] = hi;
+    return hi;
+}
+
+// lam[1] = the Gershgorin bound; lam[0] = the largest eigenvalue of the
+// Lanczos tridiagonal, or, in the safe mode (no Lanczos steps were run), the
+// Gershgorin bound / 1.1 so that the smoother's interval ends exactly at a
+// guaranteed upper bound.
+__global__ void __launch_bounds__(kBlock) k_lanczos_finish(const double* __restrict__ partIn, int nPartIn,
+                                                           const double* __restrict__ gPart, int safe, int nsteps,
+                                                           double* coef, double* lam)
+{
+    __shared__ double gsh[kBlock / kWave], al[kLanczosSteps], be[kLanczosSteps];
+    double g = 0.0;
+    double acc[1] = {0.0};
+    for (int b = threadIdx.x; b < nPartIn; b += blockDim.x) {
+        g = fmax(g, gPart[b]);
+        acc[0] += partIn[2 * b];
+    }
+    const int m = (int)coef[2 * kLanczosSteps];
+    if (threadIdx.x < kLanczosSteps) {
+        al[threadIdx.x] = coef[threadIdx.x];
+        be[threadIdx.x] = coef[kLanczosSteps + threadIdx.x];
+    }
+    g = wave_max(g);
+    if (threadIdx.x % kWave == 0) gsh[threadIdx.x / kWave] = g;
+    block_sum<1>(acc);  // ends in a barrier: gsh, al and be are complete
+    if (threadIdx.x >= kWave) return;
+    double gall = gsh[0];
+    for (int w = 1; w < kBlock / kWave; ++w) gall = fmax(gall, gsh[w]);
+    if (threadIdx.x == 0) {
+        lam[1] = gall;
+        if (safe) lam[0] = gall / 1.1;
+        else if (m == 0) lam[0] = 1.0;  // start vector in the null space of A: no information
+        if (!safe && m == nsteps) al[nsteps - 1] = acc[0];  // read by this wave only
+    }
+    if (safe || m == 0) return;
+    __builtin_amdgcn_wave_barrier();
+    const double top = tridiag_top(m, al, be);
+    if (threadIdx.x == 0) lam[0] = top;
+}
+
+// The whole estimate (start vector, Gershgorin bound, nsteps Lanczos steps and the tridiagonal's largest eigenvalue)
+// of a small level with 3x3 blocks in one workgroup: on a level of a few dozen nodes every launch of the general
+// path is one chain of dependent loads and a reduction (6 us a step), here the recurrence's vectors and the diagonal
+// blocks stay in LDS and a step is one pass over the row blocks between two barriers. 32 nodes: 77 -> 40 us; at
+// 250 nodes the single workgroup's four passes a step take as long as the launches (88 against 77 us).
+// Same formulas as k_lanczos_start, k_lanczos and k_lanczos_finish.
+constexpr int kLanczosSmallNodes = 128, kLanczosSmallThreads = 512;
+template <typename T>
+__global__ void __launch_bounds__(kLanczosSmallThreads) k_lanczos_small(int n, int safe, int nsteps, const int* __restrict__ rowPtr,
+                                                        const int* __restrict__ colIdx, const T* __restrict__ vals,
+                                                        const int* __restrict__ diagPos, double* lam)
+{
+    constexpr int BS = 3, LN = 16, GROUPS = kLanczosSmallThreads / LN, WAVES = kLanczosSmallThreads / kWave,
+                  ND = kLanczosSmallNodes * BS;
+    __shared__ double W[2][ND], v[2][ND], D[kLanczosSmallNodes * 9], Di[kLanczosSmallNodes * 9];
+    __shared__ double red[2][WAVES];
+    __shared__ double al[kLanczosSteps], be[kLanczosSteps];
+    const int sub = threadIdx.x / LN, lane = threadIdx.x % LN, wave = threadIdx.x / kWave;
+    // sums over the workgroup of two values that only lane 0 of each group holds, in every thread: per wave by
+    // shuffles, then every thread adds the waves' sums (broadcast reads) in the same order
+    const auto total = [&](double& x0, double& x1) {
+        __syncthreads();  // the readers of red are done, and the vectors written before this are complete
+        if (lane != 0) x0 = x1 = 0.0;
+        x0 += __shfl_xor(x0, 16);
+        x1 += __shfl_xor(x1, 16);
+        x0 += __shfl_xor(x0, 32);
+        x1 += __shfl_xor(x1, 32);
+        if (threadIdx.x % kWave == 0) {
+            red[0][wave] = x0;
+            red[1][wave] = x1;
+        }
+        __syncthreads();
+        x0 = x1 = 0.0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            x0 += red[0][w];
+            x1 += red[1][w];
+        }
+    };
+    for (int u = threadIdx.x; u < n; u += blockDim.x) {
+        double m[BS][BS], mi[BS][BS];
+        const T* a = vals + (size_t)diagPos[u] * 9;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) m[i / 3][i % 3] = (double)a[i];
+        block_inverse<BS>(m, mi);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            D[9 * u + i] = m[i / 3][i % 3];
+            Di[9 * u + i] = mi[i / 3][i % 3];
+        }
+    }
+    __syncthreads();
+    double gamma = 0.0, gmax = 0.0;
+    for (int u = sub; u < n; u += GROUPS) {
+        double rs[BS] = {};
+        for (int k = rowPtr[u] + lane; k < rowPtr[u + 1]; k += LN) {
+            double a[9];
+            ld_block<BS>(vals + (size_t)k * 9, a);
+#pragma unroll
+            for (int i = 0; i < BS; ++i)
+#pragma unroll
+                for (int j = 0; j < BS; ++j)
+                    rs[i] += fabs(Di[9 * u + 3 * i] * a[j] + Di[9 * u + 3 * i + 1] * a[3 + j] +
+                                  Di[9 * u + 3 * i + 2] * a[6 + j]);
+        }
+        group_sum<LN, BS>(rs);
+        const double gu = fmax(fmax(rs[0], rs[1]), rs[2]);
+        gmax = fmax(gmax, gu);
+        const double g2 = gu * gu, w4 = g2 * g2;
+        double h[BS];
+#pragma unroll
+        for (int i = 0; i < BS; ++i) h[i] = hash_unit((unsigned)(u * BS + i)) * w4;
+        if (lane == 0)
+#pragma unroll
+            for (int i = 0; i < BS; ++i) {
+                double s = 0.0;
+#pragma unroll
+                for (int c = 0; c < BS; ++c) s += Di[9 * u + 3 * i + c] * h[c];
+                W[0][3 * u + i] = s;
+                gamma += h[i] * s;
+            }
+    }
+    double unused = 0.0, aprev = 0.0, bprev = 0.0;
+    total(gamma, unused);
+    gmax = wave_max(gmax);
+    __syncthreads();
+    if (threadIdx.x % kWave == 0) red[0][wave] = gmax;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) gmax = fmax(gmax, red[0][w]);
+    if (threadIdx.x == 0) {
+        lam[1] = gmax;
+        if (safe) lam[0] = gmax / 1.1;
+    }
+    if (safe) return;
+    int m = nsteps;
+#pragma unroll 1
+    for (int j = 0; j < nsteps; ++j) {
+        const double b2 = gamma - aprev * aprev - bprev * bprev;
+        const double bj = (gamma > 0.0 && b2 > 1e-10 * gamma) ? sqrt(b2) : 0.0;
+        if (bj == 0.0) {  // the Krylov space is invariant: T so far is exact
+            m = j;
+            break;
+        }
+        if (threadIdx.x == 0) be[j] = bj;
+        const double inv = 1.0 / bj;
+        const double* Wp = W[j & 1];        // W_{j-1}, gathered
+        double* Wn = W[(j + 1) & 1];        // holds W_{j-2}; each row's own entry becomes W_j
+        const double* v1 = v[(j + 1) & 1];  // v_{j-1}
+        double* v2 = v[j & 1];              // v_{j-2}, becomes v_j
+        double s0 = 0.0, s1 = 0.0;
+#pragma unroll 1
+        for (int u = sub; u < n; u += GROUPS) {
+            double y[BS] = {};
+            for (int k = rowPtr[u] + lane; k < rowPtr[u + 1]; k += LN) {
+                double a[9];
+                ld_block<BS>(vals + (size_t)k * 9, a);
+                const double* g = Wp + 3 * colIdx[k];
+#pragma unroll
+                for (int i = 0; i < BS; ++i) y[i] += a[3 * i] * g[0] + a[3 * i + 1] * g[1] + a[3 * i + 2] * g[2];
+            }
+            group_sum<LN, BS>(y);
+            if (lane == 0) {
+                double w[BS], x[BS];
+#pragma unroll
+                for (int i = 0; i < BS; ++i) {
+                    const int q = 3 * u + i;
+                    double t = Di[9 * u + 3 * i] * y[0] + Di[9 * u + 3 * i + 1] * y[1] + Di[9 * u + 3 * i + 2] * y[2];
+                    t -= aprev * Wp[q];
+                    if (j >= 1) t -= bprev * Wn[q];
+                    w[i] = t * inv;
+                    double xv = Wp[q];
+                    if (j >= 1) xv -= aprev * v1[q];
+                    if (j >= 2) xv -= bprev * v2[q];
+                    x[i] = xv * inv;
+                }
+#pragma unroll
+                for (int i = 0; i < BS; ++i) {
+                    double z = 0.0;
+#pragma unroll
+                    for (int c = 0; c < BS; ++c) z += D[9 * u + 3 * i + c] * w[c];
+                    s0 += x[i] * z;
+                    s1 += w[i] * z;
+                    Wn[3 * u + i] = w[i];
+                    v2[3 * u + i] = x[i];
+                }
+            }
+        }
+        total(s0, s1);
+        bprev = j >= 1 ? bj : 0.0;  // beta_0 is the start's norm, not a coupling
+        aprev = s0;
+        gamma = s1;
+        if (threadIdx.x == 0) al[j] = aprev;
+    }
+    __syncthreads();
+    if (threadIdx.x >= kWave) return;
+    const double top = m == 0 ? 1.0 : tridiag_top(m, al, be);
+    if (threadIdx.x == 0) lam[0] = top;
 }
 
 // Lanes per output of the set-up kernels: the contribution lists of one
 // output are split over a lane group and reduced by shuffles, so their
 // scattered block loads are in flight together.
 constexpr int kSetupLanes = 8;
-
-template <int LANES, int NV>
-__device__ __forceinline__ void group_sum(double (&v)[NV])
-{
-#pragma unroll
-    for (int off = LANES / 2; off > 0; off >>= 1)
-#pragma unroll
-        for (int i = 0; i < NV; ++i) v[i] += __shfl_xor(v[i], off, LANES);
-}
 
 int setup_grid(long nOut, int lanes) { return (int)std::max<long>(1, (nOut * lanes + kBlock - 1) / kBlock); }
 
@@ -1477,7 +1644,8 @@ struct Amg<T>::Level : AmgHostLevel {
     // device
     int *dRowPtr = nullptr, *dColIdx = nullptr, *dDiagPos = nullptr;
     int *dAggPtr = nullptr, *dAggMem = nullptr, *dPPtr = nullptr, *dPCol = nullptr, *dPRow = nullptr,
-        *dPsPtr = nullptr, *dPsA = nullptr, *dRPtr = nullptr, *dRRow = nullptr, *dRPos = nullptr, *dTPtr = nullptr, *dTCol = nullptr, *dTcPtr = nullptr, *dTcA = nullptr,
+        *dPsPtr = nullptr, *dPsA = nullptr, *dRPtr = nullptr, *dRRow = nullptr, *dRPos = nullptr, *dTPtr = nullptr,
+        *dTCol = nullptr, *dTcPtr = nullptr, *dTcA = nullptr,
         *dTcP = nullptr, *dAcPtr = nullptr, *dAcP = nullptr, *dAcT = nullptr;
     unsigned char* dPIsTent = nullptr;
     T *vals = nullptr, *Dinv = nullptr, *Pt = nullptr, *P = nullptr, *R = nullptr, *Tv = nullptr;
@@ -1758,22 +1926,27 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
         double* gPart = dPartials + 2 * (size_t)nPartials;
         const int nsteps = lanczos_steps(l);
         const int lsafe = safe || nsteps == 0;
-        if (bs == 2)
-            hipLaunchKernelGGL((k_lanczos_start<T, 2>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.vals, A.Dinv,
-                               lb.W[0], part[1], gPart, coef, nsteps);
-        else
-            hipLaunchKernelGGL((k_lanczos_start<T, 3>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.vals, A.Dinv,
-                               lb.W[0], part[1], gPart, coef, nsteps);
-        for (int j = 0; j < (lsafe ? 0 : nsteps); ++j) {
+        if (bs == 3 && A.n <= kLanczosSmallNodes) {
+            hipLaunchKernelGGL(k_lanczos_small<T>, dim3(1), dim3(kLanczosSmallThreads), 0, s, A.n, lsafe, nsteps,
+                               A.dRowPtr, A.dColIdx, A.vals, A.dDiagPos, A.lam);
+        } else {
             if (bs == 2)
-                hipLaunchKernelGGL((k_lanczos<T, 2>), dim3(g), dim3(kBlock), 0, s, j, nsteps, A.n, A.dRowPtr,
-                                   A.dColIdx, A.vals, A.dDiagPos, lb, part[(j + 1) & 1], g, part[j & 1], coef);
+                hipLaunchKernelGGL((k_lanczos_start<T, 2>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.vals, A.Dinv,
+                                   lb.W[0], part[1], gPart, coef, nsteps);
             else
-                hipLaunchKernelGGL((k_lanczos<T, 3>), dim3(g), dim3(kBlock), 0, s, j, nsteps, A.n, A.dRowPtr,
-                                   A.dColIdx, A.vals, A.dDiagPos, lb, part[(j + 1) & 1], g, part[j & 1], coef);
+                hipLaunchKernelGGL((k_lanczos_start<T, 3>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.vals, A.Dinv,
+                                   lb.W[0], part[1], gPart, coef, nsteps);
+            for (int j = 0; j < (lsafe ? 0 : nsteps); ++j) {
+                if (bs == 2)
+                    hipLaunchKernelGGL((k_lanczos<T, 2>), dim3(g), dim3(kBlock), 0, s, j, nsteps, A.n, A.dRowPtr,
+                                       A.dColIdx, A.vals, A.dDiagPos, lb, part[(j + 1) & 1], g, part[j & 1], coef);
+                else
+                    hipLaunchKernelGGL((k_lanczos<T, 3>), dim3(g), dim3(kBlock), 0, s, j, nsteps, A.n, A.dRowPtr,
+                                       A.dColIdx, A.vals, A.dDiagPos, lb, part[(j + 1) & 1], g, part[j & 1], coef);
+            }
+            hipLaunchKernelGGL(k_lanczos_finish, dim3(1), dim3(kBlock), 0, s, part[(nsteps + 1) & 1], g, gPart, lsafe,
+                               nsteps, coef, A.lam);
         }
-        hipLaunchKernelGGL(k_lanczos_finish, dim3(1), dim3(kBlock), 0, s, part[(nsteps + 1) & 1], g, gPart, lsafe,
-                           nsteps, coef, A.lam);
         // tentative prolongator, smoothing, Galerkin product
         Level& N = *L[l + 1];
         const int nP = (int)A.pCol.size(), nT = (int)A.tCol.size(), nAc = (int)N.colIdx.size();

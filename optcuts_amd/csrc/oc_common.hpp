@@ -42,6 +42,14 @@ __device__ __forceinline__ CSum wave_csum(CSum v)
     return v;
 }
 
+// x of lane i (the same i in every lane)
+__device__ __forceinline__ double read_lane(double x, int i)
+{
+    const long long b = __double_as_longlong(x);
+    const unsigned int lo = __builtin_amdgcn_readlane((int)b, i), hi = __builtin_amdgcn_readlane((int)(b >> 32), i);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 __device__ __forceinline__ double wave_sum(double v)
 {
 #pragma unroll
