@@ -38,32 +38,6 @@ int rows_grid(int n, int rowsPerPass)
     return std::max(1, std::min((n + rowsPerPass - 1) / rowsPerPass, kAmgMaxGrid));
 }
 
-// y = sum over the row of A_uw x_w, LANES lanes per row (result in every lane of the group)
-template <typename T, int BS, int LANES, typename X>
-__device__ __forceinline__ void row_mv(const int* __restrict__ rowPtr, const int* __restrict__ colIdx,
-                                       const T* __restrict__ vals, const X* __restrict__ x, int u, int lane,
-                                       T (&y)[BS])
-{
-#pragma unroll
-    for (int i = 0; i < BS; ++i) y[i] = T(0);
-    const int k1 = rowPtr[u + 1];
-    for (int k = rowPtr[u] + lane; k < k1; k += LANES) {
-        const int w = colIdx[k];
-        const T* a = vals + (size_t)k * BS * BS;
-        T xw[BS];
-#pragma unroll
-        for (int j = 0; j < BS; ++j) xw[j] = (T)x[(size_t)w * BS + j];
-#pragma unroll
-        for (int i = 0; i < BS; ++i)
-#pragma unroll
-            for (int j = 0; j < BS; ++j) y[i] += a[i * BS + j] * xw[j];
-    }
-#pragma unroll
-    for (int off = LANES / 2; off > 0; off >>= 1)
-#pragma unroll
-        for (int i = 0; i < BS; ++i) y[i] += __shfl_xor(y[i], off, LANES);
-}
-
 // ---------------------------------------------------------------------------- numeric set-up kernels
 template <typename TI, typename T>
 __global__ void __launch_bounds__(kBlock) k_cvt(long n, const TI* __restrict__ in, T* out)
@@ -169,15 +143,6 @@ __device__ __forceinline__ double hash_unit(unsigned int i)
     i *= 0x846ca68bu;
     i ^= i >> 16;
     return (double)(i & 0xffffff) / (double)0x800000 - 1.0;
-}
-
-template <int LANES, int NV>
-__device__ __forceinline__ void group_sum(double (&v)[NV])
-{
-#pragma unroll
-    for (int off = LANES / 2; off > 0; off >>= 1)
-#pragma unroll
-        for (int i = 0; i < NV; ++i) v[i] += __shfl_xor(v[i], off, LANES);
 }
 
 // lambda_max(D^-1 A) by Lanczos in the D inner product (D^-1 A is self-adjoint
@@ -374,10 +339,7 @@ struct RowPass {
 #pragma unroll
                 for (int q = 0; q < BS; ++q) y[i] += (Y)ak[i * BS + q] * gk[q];
         }
-#pragma unroll
-        for (int off = LANES / 2; off > 0; off >>= 1)
-#pragma unroll
-            for (int i = 0; i < BS; ++i) y[i] += __shfl_xor(y[i], off, LANES);
+    group_sum<LANES, BS>(y);
     }
 };
 
@@ -403,11 +365,8 @@ __device__ __forceinline__ void lanczos_coeffs(int j, const double* __restrict__
                                                const double* __restrict__ coef, double& aprev, double& bprev,
                                                double& bj)
 {
-    double acc[2] = {0.0, 0.0};
-    for (int b = threadIdx.x; b < nPartIn; b += blockDim.x) {
-        acc[0] += partIn[2 * b];
-        acc[1] += partIn[2 * b + 1];
-    }
+    double acc[2];
+    sum_records<2>(partIn, nPartIn, 2, acc);
     block_sum<2>(acc);
     __shared__ double sh[2];
     if (threadIdx.x == 0) {
@@ -515,10 +474,7 @@ __global__ void __launch_bounds__(kBlock) k_lanczos(int j, int nsteps, int n, co
 #pragma unroll
                     for (int q = 0; q < BS; ++q) y[i] += ak[i * BS + q] * gk[q];
             }
-#pragma unroll
-            for (int off = LANES / 2; off > 0; off >>= 1)
-#pragma unroll
-                for (int i = 0; i < BS; ++i) y[i] += __shfl_xor(y[i], off, LANES);
+    group_sum<LANES, BS>(y);
             if (lane == 0 && u[r] < r1) {  // y = (A W_{j-1})_u
                 double m[BS][BS], mi[BS][BS];
 #pragma unroll
@@ -685,12 +641,16 @@ __global__ void __launch_bounds__(kBlock) k_lanczos_finish(const double* __restr
                                                            double* coef, double* lam)
 {
     __shared__ double gsh[kBlock / kWave], al[kLanczosSteps], be[kLanczosSteps];
-    double g = 0.0;
-    double acc[1] = {0.0};
-    for (int b = threadIdx.x; b < nPartIn; b += blockDim.x) {
-        g = fmax(g, gPart[b]);
-        acc[0] += partIn[2 * b];
+    double g = 0.0, gq[kAmgMaxGrid / kBlock];
+    double acc[1];
+#pragma unroll
+    for (int q = 0; q < kAmgMaxGrid / kBlock; ++q) {
+        const int b = threadIdx.x + q * kBlock;
+        gq[q] = b < nPartIn ? gPart[b] : 0.0;
     }
+    sum_records<1>(partIn, nPartIn, 2, acc);
+#pragma unroll
+    for (int q = 0; q < kAmgMaxGrid / kBlock; ++q) g = fmax(g, gq[q]);
     const int m = (int)coef[2 * kLanczosSteps];
     if (threadIdx.x < kLanczosSteps) {
         al[threadIdx.x] = coef[threadIdx.x];
@@ -1216,8 +1176,8 @@ __global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ st
 // residual's records hold; k_pcg_spmv keeps it from then on.
 __device__ __forceinline__ bool pcg_converged(const PcgStage& st)
 {
-    double acc[1] = {0.0};
-    for (int b = threadIdx.x; b < st.nRr; b += blockDim.x) acc[0] += st.partRr[(size_t)b * st.sRr];
+    double acc[1];
+    sum_records<1>(st.partRr, st.nRr, st.sRr, acc);
     const int it = st.ctrl->itNext;
     const double bbKept = st.ctrl->bb, tol2 = st.ctrl->tol2;
     block_sum<1>(acc);
@@ -1434,10 +1394,7 @@ __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int*
 #pragma unroll
                 for (int i = 0; i < NS; ++i) s[i] += (double)p[l * NS + i] * (double)ru[l];
         }
-#pragma unroll
-        for (int off = LN / 2; off > 0; off >>= 1)
-#pragma unroll
-            for (int i = 0; i < NS; ++i) s[i] += __shfl_xor(s[i], off, LN);
+    group_sum<LN, NS>(s);
         if (lane == 0) {
             T bt[NS];
 #pragma unroll
@@ -1495,10 +1452,7 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const int* __restrict__ stop
                 for (int c = 0; c < NS; ++c) s[i] += (double)p[i * NS + c] * (double)xcv[c];
         }
     }
-#pragma unroll
-    for (int off = LN / 2; off > 0; off >>= 1)
-#pragma unroll
-        for (int i = 0; i < BS; ++i) s[i] += __shfl_xor(s[i], off, LN);
+    group_sum<LN, BS>(s);
     if (u < n && lane == 0) {
 #pragma unroll
         for (int i = 0; i < BS; ++i) x[(size_t)u * BS + i] = (T)((double)x[(size_t)u * BS + i] + s[i]);

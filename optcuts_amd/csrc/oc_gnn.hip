@@ -152,11 +152,8 @@ __global__ void __launch_bounds__(kBlock) k_gnn_node_feat(int nV, const int* __r
 {
     __shared__ double mean;
     {
-        double acc[2] = {0.0, 0.0};
-        for (int b = threadIdx.x; b < nPart; b += blockDim.x) {
-            acc[0] += part[2 * b];
-            acc[1] += part[2 * b + 1];
-        }
+        double acc[2];
+        sum_records<2>(part, nPart, 2, acc);
         block_sum<2>(acc);
         if (threadIdx.x == 0) mean = acc[1] > 0.0 ? acc[0] / acc[1] : 0.0;
         __syncthreads();
@@ -894,8 +891,8 @@ __global__ void __launch_bounds__(32 * kReduceWays) k_gnn_reduce(int nRec, int s
 
 __global__ void __launch_bounds__(kBlock) k_gnn_sum_to(const double* __restrict__ part, int n, double* out)
 {
-    double acc[1] = {0.0};
-    for (int b = threadIdx.x; b < n; b += blockDim.x) acc[0] += part[b];
+    double acc[1];
+    sum_records<1>(part, n, 1, acc);
     block_sum<1>(acc);
     if (threadIdx.x == 0) *out += acc[0];
 }

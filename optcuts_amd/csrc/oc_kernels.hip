@@ -811,11 +811,7 @@ template <int NV>
 __device__ __forceinline__ void reduce_partials(const double* __restrict__ part, int nblk, double (&out)[NV])
 {
     double acc[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) acc[k] = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) acc[k] += part[(size_t)b * NV + k];
+    sum_records<NV>(part, nblk, NV, acc);
     block_sum<NV>(acc);
     __shared__ double sh[NV];
     if (threadIdx.x == 0)
@@ -829,8 +825,8 @@ __device__ __forceinline__ void reduce_partials(const double* __restrict__ part,
 // Sum of one value per record (record b at part[b*stride]), identical in every block.
 __device__ __forceinline__ double reduce_strided(const double* __restrict__ part, int nrec, int stride)
 {
-    double acc[1] = {0.0};
-    for (int b = threadIdx.x; b < nrec; b += blockDim.x) acc[0] += part[(size_t)b * stride];
+    double acc[1];
+    sum_records<1>(part, nrec, stride, acc);
     block_sum<1>(acc);
     __shared__ double sh;
     if (threadIdx.x == 0) sh = acc[0];
@@ -945,12 +941,9 @@ __device__ __forceinline__ double2 row_apply(const int* __restrict__ rowPtr, con
         yx += a.x * px + a.y * py;
         yy += a.z * px + a.w * py;
     }
-#pragma unroll
-    for (int off = kSpmvLanes / 2; off > 0; off >>= 1) {
-        yx += __shfl_xor(yx, off, kSpmvLanes);
-        yy += __shfl_xor(yy, off, kSpmvLanes);
-    }
-    return make_double2(yx, yy);
+    double y[2] = {yx, yy};
+    group_sum<kSpmvLanes, 2>(y);
+    return make_double2(y[0], y[1]);
 }
 
 __device__ __forceinline__ double4 to_double4(const double4& v) { return v; }
@@ -1053,11 +1046,10 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
                 yx += ak.x * px + ak.y * py;
                 yy += ak.z * px + ak.w * py;
             }
-#pragma unroll
-            for (int off = LANES / 2; off > 0; off >>= 1) {
-                yx += __shfl_xor(yx, off, LANES);
-                yy += __shfl_xor(yy, off, LANES);
-            }
+            double y[2] = {yx, yy};
+            group_sum<LANES, 2>(y);
+            yx = y[0];
+            yy = y[1];
             if (lane == 0 && u[r] < r1) {
                 const double2 pn = make_double2(oz[r].x + beta * op[r].x, oz[r].y + beta * op[r].y);
                 pNew[u[r]] = pn;
