@@ -283,21 +283,19 @@ __device__ __forceinline__ void st_vec(T* p, size_t u, const T (&x)[BS])
     }
 }
 
-// One pass of a row kernel: UNROLL block rows per LANES-lane group. load()
-// issues the row pointers, the first block of every lane (a row of at most
-// LANES blocks needs no other) and its gathered x entries, so the caller can
-// issue its own-row loads before any of them is consumed; mv() finishes
-// y = (A x)_u (remaining blocks, lane-group reduction; y in every lane).
+// One pass of a row kernel: UNROLL block rows per LANES-lane group. begin()
+// issues the row pointers, blocks() the first block of every lane (a row of
+// at most LANES blocks needs no other) and its column, gather() the gathered x
+// entries, so the caller can issue its own-row loads, look at the stop flag
+// or reduce records while they are in flight; mv() finishes y = (A x)_u
+// (remaining blocks, lane-group reduction; y in every lane).
 template <typename T, int BS, int UNROLL>
 struct RowPass {
     static constexpr int LANES = RowShape<BS>::lanes;
-    int u[UNROLL], kb[UNROLL], ke[UNROLL];
+    int u[UNROLL], kb[UNROLL], ke[UNROLL], w[UNROLL];
     T a[UNROLL][BS * BS], g[UNROLL][BS];
 
-    template <typename X>
-    __device__ __forceinline__ void load(int first, int stride, int r1, const int* __restrict__ rowPtr,
-                                         const int* __restrict__ colIdx, const T* __restrict__ vals,
-                                         const X* __restrict__ x, int lane)
+    __device__ __forceinline__ void begin(int first, int stride, int r1, const int* __restrict__ rowPtr)
     {
 #pragma unroll
         for (int r = 0; r < UNROLL; ++r) {
@@ -306,17 +304,28 @@ struct RowPass {
             kb[r] = valid ? rowPtr[u[r]] : 0;
             ke[r] = valid ? rowPtr[u[r] + 1] : 0;
         }
+    }
+
+    __device__ __forceinline__ void blocks(const int* __restrict__ colIdx, const T* __restrict__ vals, int lane)
+    {
 #pragma unroll
         for (int r = 0; r < UNROLL; ++r) {
             const int k = kb[r] + lane;
             const bool has = k < ke[r];
             const int kk = has ? k : 0;
+            w[r] = has ? colIdx[kk] : 0;
             ld_block<BS>(vals + (size_t)kk * BS * BS, a[r]);
-            ld_vec<BS>(x, has ? colIdx[kk] : 0, g[r]);
             if (!has)
 #pragma unroll
                 for (int i = 0; i < BS * BS; ++i) a[r][i] = T(0);
         }
+    }
+
+    template <typename X>
+    __device__ __forceinline__ void gather(const X* __restrict__ x)
+    {
+#pragma unroll
+        for (int r = 0; r < UNROLL; ++r) ld_vec<BS>(x, w[r], g[r]);
     }
 
     template <typename X, typename Y>
@@ -343,6 +352,12 @@ struct RowPass {
     }
 };
 
+// Whether a kernel is to return: `stop` (its flag's value) is set. first is the first value the kernel loads (a row
+// pointer, never negative), so that its load, and not only the flag's, comes before the branch: a kernel of a few
+// dependent round trips would otherwise spend one on the flag alone.
+__device__ __forceinline__ bool stopped(int stop, int first) { return (stop | (first & 0x80000000)) != 0; }
+__device__ __forceinline__ int stop_value(const int* __restrict__ stop) { return stop ? *stop : 0; }
+
 // Rows of this workgroup's chunk and the pass count (block-uniform).
 struct RowChunk {
     int r0, r1, passes;
@@ -361,12 +376,10 @@ __device__ __forceinline__ RowChunk row_chunk(int n, int b, int G)
     return rc;
 }
 
-__device__ __forceinline__ void lanczos_coeffs(int j, const double* __restrict__ partIn, int nPartIn,
-                                               const double* __restrict__ coef, double& aprev, double& bprev,
-                                               double& bj)
+// The coefficients of step j from the threads' shares of the previous step's records.
+__device__ __forceinline__ void lanczos_coeffs(int j, double (&acc)[2], const double* __restrict__ coef,
+                                               double& aprev, double& bprev, double& bj)
 {
-    double acc[2];
-    sum_records<2>(partIn, nPartIn, 2, acc);
     block_sum<2>(acc);
     __shared__ double sh[2];
     if (threadIdx.x == 0) {
@@ -405,8 +418,8 @@ __global__ void __launch_bounds__(kBlock) k_lanczos(int j, int nsteps, int n, co
     double aprev = 0.0, bprev = 0.0, inv = 1.0;
     double acc[2] = {0.0, 0.0};
     for (int p = 0; p < passes; ++p) {
-        int u[UNROLL], kb[UNROLL], ke[UNROLL];
-        double a[UNROLL][BS * BS], g[UNROLL][BS];
+        int u[UNROLL], kb[UNROLL], ke[UNROLL], dp[UNROLL], w[UNROLL];
+        double a[UNROLL][BS * BS], g[UNROLL][BS], rec[2];
         double oW[UNROLL][BS], oWp[UNROLL][BS], o1[UNROLL][BS], o2[UNROLL][BS], D[UNROLL][BS * BS];
 #pragma unroll
         for (int r = 0; r < UNROLL; ++r) {
@@ -414,35 +427,24 @@ __global__ void __launch_bounds__(kBlock) k_lanczos(int j, int nsteps, int n, co
             const bool valid = u[r] < r1;
             kb[r] = valid ? rowPtr[u[r]] : 0;
             ke[r] = valid ? rowPtr[u[r] + 1] : 0;
+            dp[r] = lane == 0 && valid ? diagPos[u[r]] : 0;
         }
+        if (p == 0) sum_records<2>(partIn, nPartIn, 2, rec);
         // first slice of every row (a row of at most LANES blocks needs no other)
 #pragma unroll
         for (int r = 0; r < UNROLL; ++r) {
             const int k = kb[r] + lane;
             const bool has = k < ke[r];
             const int kk = has ? k : 0;
+            w[r] = has ? colIdx[kk] : 0;
             ld_block<BS>(vals + (size_t)kk * BS * BS, a[r]);
-            ld_vec<BS>(Wp, has ? colIdx[kk] : 0, g[r]);
             if (!has)
 #pragma unroll
                 for (int i = 0; i < BS * BS; ++i) a[r][i] = 0.0;
-#pragma unroll
-            for (int i = 0; i < BS; ++i) oW[r][i] = oWp[r][i] = o1[r][i] = o2[r][i] = 0.0;
-#pragma unroll
-            for (int i = 0; i < BS * BS; ++i) D[r][i] = 0.0;
-            if (lane == 0 && u[r] < r1) {
-                ld_vec<BS>(Wp, u[r], oW[r]);
-                if (j >= 1) {
-                    ld_vec<BS>(Wpp, u[r], oWp[r]);
-                    ld_vec<BS>(v1, u[r], o1[r]);
-                }
-                if (j >= 2) ld_vec<BS>(v2, u[r], o2[r]);
-                ld_block<BS>(vals + (size_t)diagPos[u[r]] * BS * BS, D[r]);
-            }
         }
         if (p == 0) {
             double bj;
-            lanczos_coeffs(j, partIn, nPartIn, coef, aprev, bprev, bj);
+            lanczos_coeffs(j, rec, coef, aprev, bprev, bj);
             if (bj == 0.0) {  // the Krylov space is invariant: T so far is exact
                 if (blockIdx.x == 0 && threadIdx.x == 0) {
                     if (j > 0) coef[j - 1] = aprev;
@@ -455,6 +457,23 @@ __global__ void __launch_bounds__(kBlock) k_lanczos(int j, int nsteps, int n, co
                 coef[kLanczosSteps + j] = bj;
             }
             inv = 1.0 / bj;
+        }
+#pragma unroll
+        for (int r = 0; r < UNROLL; ++r) {
+            ld_vec<BS>(Wp, w[r], g[r]);
+#pragma unroll
+            for (int i = 0; i < BS; ++i) oW[r][i] = oWp[r][i] = o1[r][i] = o2[r][i] = 0.0;
+#pragma unroll
+            for (int i = 0; i < BS * BS; ++i) D[r][i] = 0.0;
+            if (lane == 0 && u[r] < r1) {
+                ld_vec<BS>(Wp, u[r], oW[r]);
+                if (j >= 1) {
+                    ld_vec<BS>(Wpp, u[r], oWp[r]);
+                    ld_vec<BS>(v1, u[r], o1[r]);
+                }
+                if (j >= 2) ld_vec<BS>(v2, u[r], o2[r]);
+                ld_block<BS>(vals + (size_t)dp[r] * BS * BS, D[r]);
+            }
         }
 #pragma unroll
         for (int r = 0; r < UNROLL; ++r) {
@@ -1171,13 +1190,11 @@ __global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ st
 // (post-smoothing): x += d + d'; 2 (the finest level's last step): z = x + d +
 // d' in FP64 and partial records of rFinal.z per workgroup. d is read for the
 // neighbours and not written. Launch with row_grid workgroups.
-// Whether the PCG's residual is within its tolerance (then its control record is set as k_pcg_spmv sets it): every
-// workgroup sums the r.r records itself, in the same order. bb, the right-hand side's norm, is what the first
+// Whether the PCG's residual is within its tolerance (then its control record is set as k_pcg_spmv sets it), from the
+// threads' shares of the r.r records: every workgroup sums them itself, in the same order. bb, the right-hand side's norm, is what the first
 // residual's records hold; k_pcg_spmv keeps it from then on.
-__device__ __forceinline__ bool pcg_converged(const PcgStage& st)
+__device__ __forceinline__ bool pcg_converged(const PcgStage& st, double (&acc)[1])
 {
-    double acc[1];
-    sum_records<1>(st.partRr, st.nRr, st.sRr, acc);
     const int it = st.ctrl->itNext;
     const double bbKept = st.ctrl->bb, tol2 = st.ctrl->tol2;
     block_sum<1>(acc);
@@ -1200,7 +1217,7 @@ __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int*
                                                const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                const T* __restrict__ Dinv, const double* __restrict__ lam,
                                                const T* __restrict__ d, T* x, const double* __restrict__ rFinal,
-                                               double* zFinal, double* rzPart, const PcgStage& st = {})
+                                               double* zFinal, double* rzPart, int stop = 0, const PcgStage& st = {})
 {
     constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
     const ChebP cp = cheb_params(*lam);
@@ -1212,7 +1229,13 @@ __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int*
     double acc[1] = {0.0};
     for (int p = 0; p < rc.passes; ++p) {
         RowPass<T, BS, UNROLL> rp;
-        rp.load(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr, colIdx, vals, d, lane);
+        rp.begin(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr);
+        double rr[1];
+        if (CHECK && p == 0) sum_records<1>(st.partRr, st.nRr, st.sRr, rr);
+        if (p == 0 && stopped(stop, rp.kb[0])) return;
+        rp.blocks(colIdx, vals, lane);
+        if (CHECK && p == 0 && pcg_converged(st, rr)) return;
+        rp.gather(d);
         double Dm[UNROLL][BS * BS], dd[UNROLL][BS], xo[UNROLL][BS], rf[UNROLL][BS];
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q)
@@ -1222,7 +1245,6 @@ __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int*
                 if (KIND >= 1) ld_vec<BS>(x, rp.u[q], xo[q]);
                 if (KIND == 2) ld_vec<BS>(rFinal, rp.u[q], rf[q]);
             }
-        if (CHECK && p == 0 && pcg_converged(st)) return;
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q) {
             double w[BS];
@@ -1264,8 +1286,8 @@ __global__ void __launch_bounds__(kBlock) k_cheb_step(const int* __restrict__ st
                                                       const T* __restrict__ d, T* x, const double* __restrict__ rFinal,
                                                       double* zFinal, double* rzPart)
 {
-    if (stop && *stop) return;
-    cheb_step_rows<T, BS, KIND>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, d, x, rFinal, zFinal, rzPart);
+    cheb_step_rows<T, BS, KIND>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, d, x, rFinal, zFinal, rzPart,
+                                stop_value(stop));
 }
 
 // The finest level's first kernel of a V-cycle inside a PCG: the pre-smoothing step behind the convergence test of the
@@ -1276,23 +1298,25 @@ __global__ void __launch_bounds__(kBlock) k_cheb_first(int n, const int* __restr
                                                        const T* __restrict__ Dinv, const double* __restrict__ lam,
                                                        const T* __restrict__ d, T* x, PcgStage st)
 {
-    if (st.ctrl->done) return;
     cheb_step_rows<T, 2, 0, true>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, Dinv, lam, d, x, nullptr, nullptr,
-                                  nullptr, st);
+                                  nullptr, st.ctrl->done, st);
 }
 
 // residual res = b - A x (row_grid workgroups); b is the FP64 right-hand side itself on the finest level
 template <typename T, int BS, typename B>
 __device__ __forceinline__ void residual_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
                                               const int* __restrict__ colIdx, const T* __restrict__ vals,
-                                              const B* __restrict__ b, const T* __restrict__ x, T* res)
+                                              const B* __restrict__ b, const T* __restrict__ x, T* res, int stop = 0)
 {
     constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
     const RowChunk rc = row_chunk<BS>(n, blk, G);
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
     for (int p = 0; p < rc.passes; ++p) {
         RowPass<T, BS, UNROLL> rp;
-        rp.load(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr, colIdx, vals, x, lane);
+        rp.begin(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr);
+        if (p == 0 && stopped(stop, rp.kb[0])) return;
+        rp.blocks(colIdx, vals, lane);
+        rp.gather(x);
         double bo[UNROLL][BS];
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q)
@@ -1316,8 +1340,7 @@ __global__ void __launch_bounds__(kBlock) k_residual(const int* __restrict__ sto
                                                      const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                      const B* __restrict__ b, const T* __restrict__ x, T* res)
 {
-    if (stop && *stop) return;
-    residual_rows<T, BS, B>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, b, x, res);
+    residual_rows<T, BS, B>(blockIdx.x, gridDim.x, n, rowPtr, colIdx, vals, b, x, res, stop_value(stop));
 }
 
 // post-smoothing, first step from the prolongated x: d = D^-1 (b - A x) / theta (row_grid workgroups)
@@ -1327,14 +1350,17 @@ __global__ void __launch_bounds__(kBlock) k_cheb_post1(const int* __restrict__ s
                                                        const T* __restrict__ Dinv, const double* __restrict__ lam,
                                                        const B* __restrict__ b, const T* __restrict__ x, T* d)
 {
-    if (stop && *stop) return;
     constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
+    const int st = stop_value(stop);
     const ChebP cp = cheb_params(*lam);
     const RowChunk rc = row_chunk<BS>(n, blockIdx.x, gridDim.x);
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
     for (int p = 0; p < rc.passes; ++p) {
         RowPass<T, BS, UNROLL> rp;
-        rp.load(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr, colIdx, vals, x, lane);
+        rp.begin(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr);
+        if (p == 0 && stopped(st, rp.kb[0])) return;
+        rp.blocks(colIdx, vals, lane);
+        rp.gather(x);
         double Dm[UNROLL][BS * BS], bo[UNROLL][BS];
 #pragma unroll
         for (int q = 0; q < UNROLL; ++q)
@@ -1377,15 +1403,18 @@ template <typename T, int BS, bool PRE1, int LN>
 __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int* __restrict__ rPtr,
                                               const int* __restrict__ rRow, const T* __restrict__ R,
                                               const T* __restrict__ res, T* bc,
-                                              const T* __restrict__ DinvN, const double* __restrict__ lamN, T* dN)
+                                              const T* __restrict__ DinvN, const double* __restrict__ lamN, T* dN,
+                                              int stop = 0)
 {
     const int cc = (nc + G - 1) / G;
     const int c0 = xcd_chunk(blk, G) * cc, c1 = min(nc, c0 + cc);
     constexpr int RPP = kBlock / LN;
     const int sub = threadIdx.x / LN, lane = threadIdx.x % LN;
     for (int c = c0 + sub; c < c1; c += RPP) {
+        const int q0 = rPtr[c], q1 = rPtr[c + 1];
+        if (stopped(stop, q0)) return;
         double s[NS] = {};
-        for (int q = rPtr[c] + lane; q < rPtr[c + 1]; q += LN) {
+        for (int q = q0 + lane; q < q1; q += LN) {
             T p[BS * NS], ru[BS];
             ld_blk<BS * NS>(R + (size_t)q * BS * NS, p);
             ld_vec<BS>(res, rRow[q], ru);
@@ -1425,8 +1454,8 @@ __global__ void __launch_bounds__(kBlock) k_restrict(const int* __restrict__ sto
                                                      const T* __restrict__ DinvN, const double* __restrict__ lamN,
                                                      T* dN)
 {
-    if (stop && *stop) return;
-    restrict_rows<T, BS, PRE1, LN>(blockIdx.x, gridDim.x, nc, rPtr, rRow, R, res, bc, DinvN, lamN, dN);
+    restrict_rows<T, BS, PRE1, LN>(blockIdx.x, gridDim.x, nc, rPtr, rRow, R, res, bc, DinvN, lamN, dN,
+                                   stop_value(stop));
 }
 
 // x_u += sum over P blocks (u,c) of P xc_c, kProlongLanes lanes per fine row (one P block each per pass, the
@@ -1437,13 +1466,14 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const int* __restrict__ stop
                                                     const int* __restrict__ pCol, const T* __restrict__ P,
                                                     const T* __restrict__ xc, T* x)
 {
-    if (stop && *stop) return;
     constexpr int LN = kProlongLanes;
     const int t = blockIdx.x * kBlock + threadIdx.x;
     const int u = t / LN, lane = t % LN;
+    const int st = stop_value(stop), j0 = u < n ? pPtr[u] : 0, j1 = u < n ? pPtr[u + 1] : 0;
+    if (stopped(st, j0)) return;
     double s[BS] = {};
     if (u < n) {
-        for (int j = pPtr[u] + lane; j < pPtr[u + 1]; j += LN) {
+        for (int j = j0 + lane; j < j1; j += LN) {
             const T* p = P + (size_t)j * BS * NS;
             const T* xcv = xc + (size_t)pCol[j] * NS;
 #pragma unroll
@@ -1476,7 +1506,7 @@ __device__ __forceinline__ void correct_rows(int blk, int G, int n, const int* _
                                              const int* __restrict__ tPtr, const int* __restrict__ tCol,
                                              const T* __restrict__ Tv, const T* __restrict__ Dinv,
                                              const double* __restrict__ lam, const T* __restrict__ xc,
-                                             const T* __restrict__ res, T* x, T* d)
+                                             const T* __restrict__ res, T* x, T* d, int stop = 0)
 {
     constexpr int LN = kCorrectLanes, RPP = kBlock / LN;
     const double theta = cheb_params(*lam).theta;
@@ -1485,6 +1515,7 @@ __device__ __forceinline__ void correct_rows(int blk, int G, int n, const int* _
     const int sub = threadIdx.x / LN, lane = threadIdx.x % LN;
     for (int u = r0 + sub; u < r1; u += RPP) {
         const int j0 = pPtr[u], j1 = pPtr[u + 1], t0 = tPtr[u], t1 = tPtr[u + 1];
+        if (stopped(stop, j0)) return;
         double Dm[BS * BS], ro[BS], xo[BS], s[2 * BS] = {};  // (A P) xc, then P xc
         if (lane == 0) {
             ld_block<BS>(Dinv + (size_t)u * BS * BS, Dm);
@@ -1534,8 +1565,8 @@ __global__ void __launch_bounds__(kBlock) k_correct(const int* __restrict__ stop
                                                     const double* __restrict__ lam, const T* __restrict__ xc,
                                                     const T* __restrict__ res, T* x, T* d)
 {
-    if (stop && *stop) return;
-    correct_rows<T, BS>(blockIdx.x, gridDim.x, n, pPtr, pCol, P, tPtr, tCol, Tv, Dinv, lam, xc, res, x, d);
+    correct_rows<T, BS>(blockIdx.x, gridDim.x, n, pPtr, pCol, P, tPtr, tCol, Tv, Dinv, lam, xc, res, x, d,
+                        stop_value(stop));
 }
 
 template <typename T>

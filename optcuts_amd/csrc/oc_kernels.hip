@@ -799,39 +799,29 @@ void launch_ls_decide_commit(hipStream_t s, const double* cand, const unsigned l
 // device-scope fences: kernel boundaries order everything.
 // Rows are split into one contiguous chunk per workgroup, so the neighbour
 // gathers of a chunk stay in the L2 of the XCD that runs it.
-__device__ __forceinline__ double2 apply_M(const double* Minv, int v, double2 r)
+__device__ __forceinline__ double4 to_double4(const double4& v) { return v; }
+__device__ __forceinline__ double4 to_double4(const float4& v)
 {
-    const double4 m = reinterpret_cast<const double4*>(Minv)[v];
-    return make_double2(m.x * r.x + m.y * r.y, m.z * r.x + m.w * r.y);
+    return make_double4((double)v.x, (double)v.y, (double)v.z, (double)v.w);
 }
 
-// Sum of NV-value partial records (record b at part[b*NV + k]) over nblk
-// records, identical in every block.
+// Workgroup sums of every thread's values, identical in every thread of every workgroup that sums the same values.
 template <int NV>
-__device__ __forceinline__ void reduce_partials(const double* __restrict__ part, int nblk, double (&out)[NV])
+__device__ __forceinline__ void all_sum(double (&acc)[NV])
 {
-    double acc[NV];
-    sum_records<NV>(part, nblk, NV, acc);
-    block_sum<NV>(acc);
-    __shared__ double sh[NV];
-    if (threadIdx.x == 0)
+    __shared__ double sh[kBlock / kWave][NV];
 #pragma unroll
-        for (int k = 0; k < NV; ++k) sh[k] = acc[k];
+    for (int k = 0; k < NV; ++k) acc[k] = wave_sum(acc[k]);
+    if (threadIdx.x % kWave == 0)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) sh[threadIdx.x / kWave][k] = acc[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < NV; ++k) out[k] = sh[k];
-}
-
-// Sum of one value per record (record b at part[b*stride]), identical in every block.
-__device__ __forceinline__ double reduce_strided(const double* __restrict__ part, int nrec, int stride)
-{
-    double acc[1];
-    sum_records<1>(part, nrec, stride, acc);
-    block_sum<1>(acc);
-    __shared__ double sh;
-    if (threadIdx.x == 0) sh = acc[0];
-    __syncthreads();
-    return sh;
+    for (int k = 0; k < NV; ++k) {
+        acc[k] = sh[0][k];
+#pragma unroll
+        for (int w = 1; w < kBlock / kWave; ++w) acc[k] += sh[w][k];
+    }
 }
 
 __device__ __forceinline__ void row_chunk(int nV, int& r0, int& r1)
@@ -846,18 +836,23 @@ __device__ __forceinline__ void row_chunk(int nV, int& r0, int& r1)
 enum { kPcgExternal = 0, kPcgApplyM = 1, kPcgFirst64 = 2, kPcgFirst32 = 3 };
 
 template <int MODE>
-__device__ __forceinline__ void pcg_first(const FirstStep& f, double theta, int v, double2 r)
+__device__ __forceinline__ double4 pcg_row_matrix(const double* __restrict__ Minv, const FirstStep& f, int v)
 {
-    if constexpr (MODE == kPcgFirst64) {
-        const double4 m = reinterpret_cast<const double4*>(f.Dinv)[v];
-        reinterpret_cast<double2*>(f.d)[v] =
-            make_double2((m.x * r.x + m.y * r.y) / theta, (m.z * r.x + m.w * r.y) / theta);
-    } else if constexpr (MODE == kPcgFirst32) {
-        const float4 m = reinterpret_cast<const float4*>(f.Dinv)[v];
-        reinterpret_cast<float2*>(f.d)[v] =
-            make_float2((float)(((double)m.x * r.x + (double)m.y * r.y) / theta),
-                        (float)(((double)m.z * r.x + (double)m.w * r.y) / theta));
-    }
+    if constexpr (MODE == kPcgApplyM) return reinterpret_cast<const double4*>(Minv)[v];
+    if constexpr (MODE == kPcgFirst64) return reinterpret_cast<const double4*>(f.Dinv)[v];
+    if constexpr (MODE == kPcgFirst32) return to_double4(reinterpret_cast<const float4*>(f.Dinv)[v]);
+    return make_double4(0.0, 0.0, 0.0, 0.0);
+}
+
+// z = m r (returned; kPcgApplyM) or d = m r / theta (written)
+template <int MODE>
+__device__ __forceinline__ double2 pcg_first(const FirstStep& f, double theta, int v, const double4& m, double2 r)
+{
+    const double2 t = make_double2(m.x * r.x + m.y * r.y, m.z * r.x + m.w * r.y);
+    if constexpr (MODE == kPcgFirst64) reinterpret_cast<double2*>(f.d)[v] = make_double2(t.x / theta, t.y / theta);
+    if constexpr (MODE == kPcgFirst32)
+        reinterpret_cast<float2*>(f.d)[v] = make_float2((float)(t.x / theta), (float)(t.y / theta));
+    return t;
 }
 
 template <int MODE>
@@ -874,12 +869,11 @@ __global__ void __launch_bounds__(kBlock) k_pcg_init(int nV, const double2* __re
         const double2 bv = b[v];
         x[v] = make_double2(0.0, 0.0);
         r[v] = bv;
+        const double2 zv = pcg_first<MODE>(first, theta, v, pcg_row_matrix<MODE>(Minv, first, v), bv);
         if (APPLY_M) {
-            const double2 zv = apply_M(Minv, v, bv);
             z[v] = zv;
             acc[0] += bv.x * zv.x + bv.y * zv.y;
         }
-        pcg_first<MODE>(first, theta, v, bv);
         acc[1] += bv.x * bv.x + bv.y * bv.y;
     }
     block_sum<2>(acc);
@@ -946,12 +940,6 @@ __device__ __forceinline__ double2 row_apply(const int* __restrict__ rowPtr, con
     return make_double2(y[0], y[1]);
 }
 
-__device__ __forceinline__ double4 to_double4(const double4& v) { return v; }
-__device__ __forceinline__ double4 to_double4(const float4& v)
-{
-    return make_double4((double)v.x, (double)v.y, (double)v.z, (double)v.w);
-}
-
 // PCG direction and product: p_new = z + beta p_old, q = A p_new, partial
 // records of p_new.q. beta needs the previous update's reductions, so the
 // row loads (blocks, gathered z and p_old) are issued first and the records
@@ -969,8 +957,11 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
                                                      const double* __restrict__ partRr, int nRr, int sRr,
                                                      double* partS, PcgCtrl* ctrl)
 {
-    if (ctrl->done) return;
-    const int it = ctrl->itNext;
+    // The control record, the row pointers and the previous kernel's records are loaded together; the blocks follow
+    // and are in flight while the records are reduced, the gathers come last: three dependent round trips in all. A
+    // finished PCG is seen with the records (the loads before it are harmless, nothing is written).
+    const int done = ctrl->done, it = ctrl->itNext, maxit = ctrl->maxit;
+    const double bbKept = ctrl->bb, tol2 = ctrl->tol2, rzOld = ctrl->rzSlot[(it + 1) & 1];
     constexpr int LANES = kPcgLanes, UNROLL = kPcgRows, RPP = kBlock / LANES;
     const int G = gridDim.x;
     const int c = (nV + G - 1) / G;
@@ -981,15 +972,23 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
     double beta = 0.0;
     double acc[1] = {0.0};
     for (int pass = 0; pass < passes; ++pass) {
-        int u[UNROLL], kb[UNROLL], ke[UNROLL];
+        int u[UNROLL], kb[UNROLL], ke[UNROLL], w[UNROLL];
         double4 a[UNROLL];
         double2 gz[UNROLL], gp[UNROLL], oz[UNROLL], op[UNROLL];
+        double rec[2];
 #pragma unroll
         for (int r = 0; r < UNROLL; ++r) {
             u[r] = r0 + sub + (pass * UNROLL + r) * RPP;
             const bool valid = u[r] < r1;
             kb[r] = valid ? rowPtr[u[r]] : 0;
             ke[r] = valid ? rowPtr[u[r] + 1] : 0;
+        }
+        if (pass == 0) {
+            double one[1];
+            sum_records<1>(partRz, nRz, sRz, one);
+            rec[0] = one[0];
+            sum_records<1>(partRr, nRr, sRr, one);
+            rec[1] = one[0];
         }
 #pragma unroll
         for (int r = 0; r < UNROLL; ++r) {
@@ -998,22 +997,16 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
             const int kk = has ? k : 0;
             const double4 av = to_double4(vals[kk]);
             a[r] = has ? av : make_double4(0.0, 0.0, 0.0, 0.0);
-            const int w = has ? colIdx[kk] : 0;
-            gz[r] = z[w];
-            gp[r] = first ? make_double2(0.0, 0.0) : pOld[w];
-            oz[r] = op[r] = make_double2(0.0, 0.0);
-            if (lane == 0 && u[r] < r1) {
-                oz[r] = z[u[r]];
-                if (!first) op[r] = pOld[u[r]];
-            }
+            w[r] = has ? colIdx[kk] : 0;
         }
         if (pass == 0) {
-            const double rz = reduce_strided(partRz, nRz, sRz);
-            const double rr = reduce_strided(partRr, nRr, sRr);
-            const double bb = first ? rr : ctrl->bb;
-            const bool conv = (bb == 0.0) || (rr <= ctrl->tol2 * bb);
-            const bool capped = it >= ctrl->maxit;
+            all_sum<2>(rec);
+            const double rz = rec[0], rr = rec[1];
+            const double bb = first ? rr : bbKept;
+            const bool conv = (bb == 0.0) || (rr <= tol2 * bb);
+            const bool capped = it >= maxit;
             const bool indef = !conv && !(rz > 0.0);  // preconditioner not positive definite on r
+            if (done) return;
             if (blockIdx.x == 0 && threadIdx.x == 0) {
                 if (first) ctrl->bb = bb;
                 ctrl->rzSlot[it & 1] = rz;
@@ -1025,7 +1018,17 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
                 else if (capped) ctrl->done = 2;
             }
             if (conv || capped || indef) return;
-            beta = first ? 0.0 : rz / ctrl->rzSlot[(it + 1) & 1];
+            beta = first ? 0.0 : rz / rzOld;
+        }
+#pragma unroll
+        for (int r = 0; r < UNROLL; ++r) {
+            gz[r] = z[w[r]];
+            gp[r] = first ? make_double2(0.0, 0.0) : pOld[w[r]];
+            oz[r] = op[r] = make_double2(0.0, 0.0);
+            if (lane == 0 && u[r] < r1) {
+                oz[r] = z[u[r]];
+                if (!first) op[r] = pOld[u[r]];
+            }
         }
 #pragma unroll
         for (int r = 0; r < UNROLL; ++r) {
@@ -1033,13 +1036,13 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
             double yx = a[r].x * px + a[r].y * py;
             double yy = a[r].z * px + a[r].w * py;
             for (int k = kb[r] + lane + LANES; k < ke[r]; k += LANES) {
-                const int w = colIdx[k];
+                const int wk = colIdx[k];
                 const double4 ak = to_double4(vals[k]);
-                const double2 zw = z[w];
+                const double2 zw = z[wk];
                 px = zw.x;
                 py = zw.y;
                 if (!first) {
-                    const double2 pw = pOld[w];
+                    const double2 pw = pOld[wk];
                     px += beta * pw.x;
                     py += beta * pw.y;
                 }
@@ -1087,36 +1090,54 @@ __global__ void __launch_bounds__(kBlock) k_pcg_update(int nV, const double2* __
                                                        double* partUout, PcgCtrl* ctrl)
 {
     constexpr bool APPLY_M = MODE == kPcgApplyM;
-    if (ctrl->done) return;
+    // the thread's first row is loaded together with the records, before either is used
+    const int done = ctrl->done, it = ctrl->itCur;
+    const double rzCur = ctrl->rzSlot[it & 1];
     const double theta = MODE >= kPcgFirst64 ? cheb_params(*first.lam).theta : 0.0;
+    int r0, r1;
+    row_chunk(nV, r0, r1);
+    int v = r0 + threadIdx.x;
+    double2 pv, qv, xv, rv;
+    double4 m;
+    if (v < r1) {
+        pv = p[v];
+        qv = q[v];
+        xv = x[v];
+        rv = r[v];
+        m = pcg_row_matrix<MODE>(Minv, first, v);
+    }
     double pq[1];
-    reduce_partials<1>(partS, nPartS, pq);
+    sum_records<1>(partS, nPartS, 1, pq);
+    all_sum<1>(pq);
+    if (done) return;
     if (!(pq[0] > 0.0)) {  // breakdown: A not positive definite along p
         if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->done = 3;
         return;
     }
-    const int it = ctrl->itCur;
-    const double alpha = ctrl->rzSlot[it & 1] / pq[0];
+    const double alpha = rzCur / pq[0];
     if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->itNext = it + 1;
-    int r0, r1;
-    row_chunk(nV, r0, r1);
     double acc[2] = {0.0, 0.0};
-    for (int v = r0 + threadIdx.x; v < r1; v += blockDim.x) {
-        const double2 pv = p[v], qv = q[v];
-        double2 xv = x[v], rv = r[v];
+    while (v < r1) {
         xv.x += alpha * pv.x;
         xv.y += alpha * pv.y;
         rv.x -= alpha * qv.x;
         rv.y -= alpha * qv.y;
         x[v] = xv;
         r[v] = rv;
+        const double2 zv = pcg_first<MODE>(first, theta, v, m, rv);
         if (APPLY_M) {
-            const double2 zv = apply_M(Minv, v, rv);
             z[v] = zv;
             acc[0] += rv.x * zv.x + rv.y * zv.y;
         }
-        pcg_first<MODE>(first, theta, v, rv);
         acc[1] += rv.x * rv.x + rv.y * rv.y;
+        v += blockDim.x;
+        if (v < r1) {
+            pv = p[v];
+            qv = q[v];
+            xv = x[v];
+            rv = r[v];
+            m = pcg_row_matrix<MODE>(Minv, first, v);
+        }
     }
     block_sum<2>(acc);
     if (threadIdx.x == 0) {
