@@ -364,10 +364,10 @@ struct RowChunk {
 };
 // Row chunk of workgroup b of G (the V-cycle kernels' bodies also run as one
 // workgroup covering every row: b = 0, G = 1).
-template <int BS>
+template <int BS, int NT = kBlock>
 __device__ __forceinline__ RowChunk row_chunk(int n, int b, int G)
 {
-    constexpr int RPP = kBlock / RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll;
+    constexpr int RPP = NT / RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll;
     const int c = (n + G - 1) / G;
     RowChunk rc;
     rc.r0 = xcd_chunk(b, G) * c;
@@ -1212,19 +1212,19 @@ __device__ __forceinline__ bool pcg_converged(const PcgStage& st, double (&acc)[
     return true;
 }
 
-template <typename T, int BS, int KIND, bool CHECK = false>
+template <typename T, int BS, int KIND, bool CHECK = false, int NT = kBlock>
 __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
                                                const int* __restrict__ colIdx, const T* __restrict__ vals,
                                                const T* __restrict__ Dinv, const double* __restrict__ lam,
                                                const T* __restrict__ d, T* x, const double* __restrict__ rFinal,
                                                double* zFinal, double* rzPart, int stop = 0, const PcgStage& st = {})
 {
-    constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
+    constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = NT / LANES;
     const ChebP cp = cheb_params(*lam);
     const double rho0 = 1.0 / cp.sigma;
     const double rho1 = 1.0 / (2.0 * cp.sigma - rho0);
     const double c1 = rho1 * rho0, c2 = 2.0 * rho1 / cp.delta;
-    const RowChunk rc = row_chunk<BS>(n, blk, G);
+    const RowChunk rc = row_chunk<BS, NT>(n, blk, G);
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
     double acc[1] = {0.0};
     for (int p = 0; p < rc.passes; ++p) {
@@ -1303,13 +1303,13 @@ __global__ void __launch_bounds__(kBlock) k_cheb_first(int n, const int* __restr
 }
 
 // residual res = b - A x (row_grid workgroups); b is the FP64 right-hand side itself on the finest level
-template <typename T, int BS, typename B>
+template <typename T, int BS, typename B, int NT = kBlock>
 __device__ __forceinline__ void residual_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
                                               const int* __restrict__ colIdx, const T* __restrict__ vals,
                                               const B* __restrict__ b, const T* __restrict__ x, T* res, int stop = 0)
 {
-    constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = kBlock / LANES;
-    const RowChunk rc = row_chunk<BS>(n, blk, G);
+    constexpr int LANES = RowShape<BS>::lanes, UNROLL = RowShape<BS>::unroll, RPP = NT / LANES;
+    const RowChunk rc = row_chunk<BS, NT>(n, blk, G);
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
     for (int p = 0; p < rc.passes; ++p) {
         RowPass<T, BS, UNROLL> rp;
@@ -1399,7 +1399,7 @@ __global__ void __launch_bounds__(kBlock) k_cheb_post1(const int* __restrict__ s
 // 38 us, now 24; 200k faces 9.9, now 6.0).
 // PRE1: the next level's first pre-smoothing step (k_cheb_pre1) is row-local,
 // so it runs here on each restricted row instead of in a launch of its own.
-template <typename T, int BS, bool PRE1, int LN>
+template <typename T, int BS, bool PRE1, int LN, int NT = kBlock>
 __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int* __restrict__ rPtr,
                                               const int* __restrict__ rRow, const T* __restrict__ R,
                                               const T* __restrict__ res, T* bc,
@@ -1408,7 +1408,7 @@ __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int*
 {
     const int cc = (nc + G - 1) / G;
     const int c0 = xcd_chunk(blk, G) * cc, c1 = min(nc, c0 + cc);
-    constexpr int RPP = kBlock / LN;
+    constexpr int RPP = NT / LN;
     const int sub = threadIdx.x / LN, lane = threadIdx.x % LN;
     for (int c = c0 + sub; c < c1; c += RPP) {
         const int q0 = rPtr[c], q1 = rPtr[c + 1];
@@ -1500,7 +1500,7 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const int* __restrict__ stop
 // 3016, 203k 4953 / 4809, 501k 9084 / 8977. kCorrectLanes lanes per fine row.
 constexpr int kCorrectLanes = 8;
 constexpr int kCorrectMaxFine = 131072;
-template <typename T, int BS>
+template <typename T, int BS, int NT = kBlock>
 __device__ __forceinline__ void correct_rows(int blk, int G, int n, const int* __restrict__ pPtr,
                                              const int* __restrict__ pCol, const T* __restrict__ P,
                                              const int* __restrict__ tPtr, const int* __restrict__ tCol,
@@ -1508,7 +1508,7 @@ __device__ __forceinline__ void correct_rows(int blk, int G, int n, const int* _
                                              const double* __restrict__ lam, const T* __restrict__ xc,
                                              const T* __restrict__ res, T* x, T* d, int stop = 0)
 {
-    constexpr int LN = kCorrectLanes, RPP = kBlock / LN;
+    constexpr int LN = kCorrectLanes, RPP = NT / LN;
     const double theta = cheb_params(*lam).theta;
     const int c = (n + G - 1) / G;
     const int r0 = xcd_chunk(blk, G) * c, r1 = min(n, r0 + c);
@@ -1964,11 +1964,8 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
 
 // x = D^-1 b on a block-diagonal coarsest level (exact)
 template <typename T, int BS>
-__device__ __forceinline__ void coarse_diag_rows(int blk, int n, const T* __restrict__ Dinv, const T* __restrict__ b,
-                                                 T* x)
+__device__ __forceinline__ void coarse_diag_row(int u, const T* __restrict__ Dinv, const T* __restrict__ b, T* x)
 {
-    const int u = blk * kBlock + threadIdx.x;
-    if (u >= n) return;
     const T* D = Dinv + (size_t)u * BS * BS;
 #pragma unroll
     for (int i = 0; i < BS; ++i) {
@@ -1984,7 +1981,8 @@ __global__ void __launch_bounds__(kBlock) k_coarse_diag(const int* __restrict__ 
                                                         const T* __restrict__ b, T* x)
 {
     if (stop && *stop) return;
-    coarse_diag_rows<T, BS>(blockIdx.x, n, Dinv, b, x);
+    const int u = blockIdx.x * kBlock + threadIdx.x;
+    if (u < n) coarse_diag_row<T, BS>(u, Dinv, b, x);
 }
 
 // The last smoothed level's part of the V-cycle, with 3x3 blocks, in one
@@ -2003,7 +2001,7 @@ __global__ void __launch_bounds__(kBlock) k_coarse_diag(const int* __restrict__ 
 constexpr int kTailMaxNodes = OC_TAIL_MAX_NODES;  // largest last smoothed level run as one workgroup (0: never)
 struct TailArgs {
     // smoothed level (3x3 blocks)
-    int n;
+    int n, nnz, nP, nT;
     const int *rowPtr, *colIdx, *rPtr, *rRow, *pPtr, *pCol, *tPtr, *tCol;
     const void *vals, *Dinv, *P, *R, *Tv;
     const double* lam;
@@ -2015,35 +2013,61 @@ struct TailArgs {
     void *bC, *xC;
 };
 
-template <typename T, int LN>
-__global__ void __launch_bounds__(kBlock) k_vcycle_tail(const int* __restrict__ stop, TailArgs a)
+// 1,024 threads are a 16-lane group for each of 64 rows, so most tails are one pass per phase; with 256 threads and the
+// matrices fetched phase by phase the 32-node tail of the 200k disc took 17 us, with both 13.
+constexpr int kTailThreads = 1024;
+
+// Touches every line of n bytes: the tail's matrices come into its XCD's L2 in one round trip instead of phase by
+// phase (nothing of them is in that L2 when the kernel starts).
+__device__ __forceinline__ int touch(const void* p, size_t n)
 {
+    int x = 0;
+    const char* c = static_cast<const char*>(p);
+    for (size_t i = (size_t)threadIdx.x * 128; i < n; i += (size_t)kTailThreads * 128)
+        x |= *reinterpret_cast<const int*>(c + i);
+    return x;
+}
+
+template <typename T, int LN>
+__global__ void __launch_bounds__(kTailThreads) k_vcycle_tail(const int* __restrict__ stop, TailArgs a)
+{
+    constexpr int NT = kTailThreads;
     if (stop && *stop) return;
     const T* vals = static_cast<const T*>(a.vals);
     const T* Dinv = static_cast<const T*>(a.Dinv);
     const T* P = static_cast<const T*>(a.P);
+    const T* R = static_cast<const T*>(a.R);
+    const T* Tv = static_cast<const T*>(a.Tv);
     T *b = static_cast<T*>(a.b), *x = static_cast<T*>(a.x), *r = static_cast<T*>(a.r), *d = static_cast<T*>(a.d);
     T *bC = static_cast<T*>(a.bC), *xC = static_cast<T*>(a.xC);
-    cheb_step_rows<T, 3, 0>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, x, nullptr, nullptr, nullptr);
+    int seen = touch(vals, sizeof(T) * 9 * (size_t)a.nnz) | touch(a.colIdx, sizeof(int) * (size_t)a.nnz) |
+               touch(R, sizeof(T) * 9 * (size_t)a.nP) | touch(P, sizeof(T) * 9 * (size_t)a.nP) |
+               touch(Tv, sizeof(T) * 9 * (size_t)a.nT) | touch(a.rRow, sizeof(int) * (size_t)a.nP) |
+               touch(a.pCol, sizeof(int) * (size_t)a.nP) | touch(a.tCol, sizeof(int) * (size_t)a.nT) |
+               touch(Dinv, sizeof(T) * 9 * (size_t)a.n) | touch(b, sizeof(T) * 3 * (size_t)a.n);
+    if (a.dense) seen |= touch(a.Inv, sizeof(double) * (size_t)(a.nc * a.cbs) * (a.nc * a.cbs));
+    asm volatile("" ::"v"(seen));  // the loads are not to be dropped
+    cheb_step_rows<T, 3, 0, false, NT>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, x, nullptr, nullptr,
+                                       nullptr);
     __syncthreads();
-    residual_rows<T, 3, T>(0, 1, a.n, a.rowPtr, a.colIdx, vals, b, x, r);
+    residual_rows<T, 3, T, NT>(0, 1, a.n, a.rowPtr, a.colIdx, vals, b, x, r);
     __syncthreads();
-    restrict_rows<T, 3, false, LN>(0, 1, a.nc, a.rPtr, a.rRow, static_cast<const T*>(a.R), r, bC, nullptr, nullptr,
-                                   nullptr);
+    restrict_rows<T, 3, false, LN, NT>(0, 1, a.nc, a.rPtr, a.rRow, R, r, bC, nullptr, nullptr, nullptr);
     __syncthreads();
     if (a.dense) {
         dense_apply_rows<T>(a.nc * a.cbs, a.Inv, bC, xC);
     } else {
         const T* DinvC = static_cast<const T*>(a.DinvC);
-        for (int blk = 0; blk * kBlock < a.nc; ++blk) {
-            if (a.cbs == 2) coarse_diag_rows<T, 2>(blk, a.nc, DinvC, bC, xC);
-            else coarse_diag_rows<T, 3>(blk, a.nc, DinvC, bC, xC);
+        for (int u = threadIdx.x; u < a.nc; u += NT) {
+            if (a.cbs == 2) coarse_diag_row<T, 2>(u, DinvC, bC, xC);
+            else coarse_diag_row<T, 3>(u, DinvC, bC, xC);
         }
     }
     __syncthreads();
-    correct_rows<T, 3>(0, 1, a.n, a.pPtr, a.pCol, P, a.tPtr, a.tCol, static_cast<const T*>(a.Tv), Dinv, a.lam, xC, r, x, d);
+    correct_rows<T, 3, NT>(0, 1, a.n, a.pPtr, a.pCol, P, a.tPtr, a.tCol, Tv, Dinv, a.lam, xC, r, x, d);
     __syncthreads();
-    cheb_step_rows<T, 3, 1>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, x, nullptr, nullptr, nullptr);
+    cheb_step_rows<T, 3, 1, false, NT>(0, 1, a.n, a.rowPtr, a.colIdx, vals, Dinv, a.lam, d, x, nullptr, nullptr,
+                                       nullptr);
 }
 
 int correct_grid(int n) { return (rows_grid(n, kBlock / kCorrectLanes) + 7) & ~7; }
@@ -2101,6 +2125,9 @@ void Amg<T>::vcycle_tail(hipStream_t s, int l, const int* stop)
     Level& C = *L[l + 1];
     TailArgs a;
     a.n = A.n;
+    a.nnz = (int)A.colIdx.size();
+    a.nP = (int)A.pCol.size();
+    a.nT = (int)A.tCol.size();
     a.rowPtr = A.dRowPtr;
     a.colIdx = A.dColIdx;
     a.rPtr = A.dRPtr;
@@ -2129,9 +2156,9 @@ void Amg<T>::vcycle_tail(hipStream_t s, int l, const int* stop)
     // lanes per coarse node as restrict_to picks them
     const long meanLen = A.nc > 0 ? (long)A.rP.size() / A.nc : 0;
     const int ln = meanLen >= 48 ? 64 : (meanLen >= 24 ? 32 : 16);
-    if (ln == 64) hipLaunchKernelGGL((k_vcycle_tail<T, 64>), dim3(1), dim3(kBlock), 0, s, stop, a);
-    else if (ln == 32) hipLaunchKernelGGL((k_vcycle_tail<T, 32>), dim3(1), dim3(kBlock), 0, s, stop, a);
-    else hipLaunchKernelGGL((k_vcycle_tail<T, 16>), dim3(1), dim3(kBlock), 0, s, stop, a);
+    if (ln == 64) hipLaunchKernelGGL((k_vcycle_tail<T, 64>), dim3(1), dim3(kTailThreads), 0, s, stop, a);
+    else if (ln == 32) hipLaunchKernelGGL((k_vcycle_tail<T, 32>), dim3(1), dim3(kTailThreads), 0, s, stop, a);
+    else hipLaunchKernelGGL((k_vcycle_tail<T, 16>), dim3(1), dim3(kTailThreads), 0, s, stop, a);
 }
 
 // One smoothed level of the V-cycle below the finest (or the coarsest solve): from N.b and the direction that the
