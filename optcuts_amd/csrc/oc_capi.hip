@@ -3228,14 +3228,14 @@ int oc_newton_step(oc_ctx* c, oc_iter_stats* S, int* done)
     // gradient (and element Hessians in the same pass)
     system_element_pass(c, T);
     oc::launch_gather_grad(s, nVt, c->dVcPtr.as<int>(), c->dVcSrc.as<int>(), c->dFixedMaskSys.as<unsigned char>(),
-                           c->dElemG.as<double>(), c->dG.as<double>(), c->dPartials.as<double>(), scalar(c, 6));
+                           c->dElemG.as<double>(), c->dG.as<double>(), c->dPartials.as<double>(), scalar(c, 6),
+                           c->dB.as<double>());
     OC_HIP(c, hipGetLastError());
     // ||g||^2 travels to the host while the Newton system is assembled and the preconditioner set up (work
     // that is simply dropped on the one step whose gradient test succeeds)
     OC_HIP(c, hipMemcpyAsync(c->mail, scalar(c, 6), sizeof(double), hipMemcpyDeviceToHost, s));
     OC_HIP(c, hipEventRecord(c->evGsq, s));
     system_assemble(c);
-    oc::launch_scale_copy(s, 2L * nVt, -1.0, c->dG.as<double>(), c->dB.as<double>());
     if (int st = launch_precond_setup(c, S)) return st;
     OC_HIP(c, hipGetLastError());
     OC_HIP(c, hipEventSynchronize(c->evGsq));
@@ -3273,11 +3273,7 @@ int oc_newton_step(oc_ctx* c, oc_iter_stats* S, int* done)
     constexpr int K = oc::kLSCand;
     unsigned long long* om = c->dOrdMin.as<unsigned long long>();
     unsigned long long* omAir = c->nFair ? om + 1 : nullptr;  // the air and the mesh triangles' own bounds
-    oc::launch_set_u64(s, om, oc::dbl_to_ordered_host(1.0));
-    if (omAir) {
-        oc::launch_set_u64(s, omAir, oc::dbl_to_ordered_host(1.0));
-        oc::launch_set_u64(s, omAir + 1, oc::dbl_to_ordered_host(1.0));
-    }
+    oc::launch_set_u64(s, om, oc::dbl_to_ordered_host(1.0), omAir ? 3 : 1);
     oc::launch_step_bound(s, T, c->dUV.as<double>(), dir, om, 1.0, omAir);
     const double* esum = nullptr;
     if (c->nFair) {  // the scaffold changed: the energy is recomputed (Optimizer.cpp:588-592)
@@ -3285,11 +3281,10 @@ int oc_newton_step(oc_ctx* c, oc_iter_stats* S, int* done)
                            scalar(c, 4), f32);
         esum = scalar(c, 4);
     }
-    oc::launch_linesearch(s, T, c->dUV.as<double>(), dir, 0.0, 0, c->dPartials.as<double>(), c->dLsOut.as<double>(),
-                          f32, om);
     oc::LsDecision* dDec = c->dLsDec.as<oc::LsDecision>();
-    oc::launch_ls_decide_commit(s, c->dLsOut.as<double>(), om, omAir, esum, c->lastE, c->a0, T.sAir, dDec, 2L * nVt,
-                                dir, c->dUV.as<double>());
+    oc::launch_linesearch(s, T, c->dUV.as<double>(), dir, 0.0, 0, c->dPartials.as<double>(), c->dLsOut.as<double>(),
+                          f32, om, oc::LsDecide{dDec, om, omAir, esum, c->lastE});
+    oc::launch_ls_commit(s, dDec, 2L * nVt, dir, c->dUV.as<double>());
     OC_HIP(c, hipGetLastError());
     double* cand = c->mail;
     oc::LsDecision* D = reinterpret_cast<oc::LsDecision*>(c->mail + 4 * K);

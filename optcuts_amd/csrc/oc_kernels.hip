@@ -281,24 +281,34 @@ void launch_triplets(hipStream_t s, const TriSet& T, const double* UV, const lon
 }
 
 // ----------------------------------------------------------------------------
+constexpr int kGatherBatch = 4;
 __global__ void __launch_bounds__(kBlock) k_gather_grad(int nV, const int* __restrict__ vcPtr,
                                                         const int* __restrict__ vcSrc,
                                                         const unsigned char* __restrict__ fixedMask,
                                                         const double2* __restrict__ elemG, double2* g,
-                                                        double* partials)
+                                                        double2* negG, double* partials)
 {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     double sq[1] = {0.0};
     if (v < nV) {
         double2 s = make_double2(0.0, 0.0);
-        if (!fixedMask[v]) {
-            for (int k = vcPtr[v]; k < vcPtr[v + 1]; ++k) {
-                const double2 e = elemG[vcSrc[k]];
-                s.x += e.x;
-                s.y += e.y;
+        const int k0 = vcPtr[v], k1 = vcPtr[v + 1];
+        // a vertex has about six triangles: their contributions are loaded together and added in triangle order (one
+        // at a time, each is two dependent round trips: 54 us at 1M faces)
+        if (!fixedMask[v])
+            for (int k = k0; k < k1; k += kGatherBatch) {
+                double2 e[kGatherBatch];
+#pragma unroll
+                for (int q = 0; q < kGatherBatch; ++q)
+                    e[q] = k + q < k1 ? elemG[vcSrc[k + q]] : make_double2(0.0, 0.0);
+#pragma unroll
+                for (int q = 0; q < kGatherBatch; ++q) {
+                    s.x += e[q].x;
+                    s.y += e[q].y;
+                }
             }
-        }
         g[v] = s;
+        if (negG) negG[v] = make_double2(-s.x, -s.y);
         sq[0] = s.x * s.x + s.y * s.y;
     }
     if (partials) {
@@ -308,12 +318,12 @@ __global__ void __launch_bounds__(kBlock) k_gather_grad(int nV, const int* __res
 }
 
 void launch_gather_grad(hipStream_t s, int nV, const int* vcPtr, const int* vcSrc, const unsigned char* fixedMask,
-                        const double* elemG, double* g, double* partials, double* gsq)
+                        const double* elemG, double* g, double* partials, double* gsq, double* negG)
 {
     const int grid = grid_for(nV);
     hipLaunchKernelGGL(k_gather_grad, dim3(grid), dim3(kBlock), 0, s, nV, vcPtr, vcSrc, fixedMask,
                        reinterpret_cast<const double2*>(elemG), reinterpret_cast<double2*>(g),
-                       gsq ? partials : nullptr);
+                       reinterpret_cast<double2*>(negG), gsq ? partials : nullptr);
     if (gsq) hipLaunchKernelGGL(k_finish_csum<1>, dim3(1), dim3(kBlock), 0, s, partials, grid, gsq);
 }
 
@@ -517,18 +527,24 @@ __global__ void __launch_bounds__(kBlock) k_assemble(int nUB, const int* __restr
     if (b >= nUB) return;
     const int u = ubRow[b], w = ubCol[b];
     double4 s = make_double4(0.0, 0.0, 0.0, 0.0);
-    for (int k = ubCPtr[b]; k < ubCPtr[b + 1]; ++k) {
-        const unsigned int code = (unsigned int)ubCSrc[k];
-        double4 e = load_block(elemH, (int)(code & 0x7fffffffu));
-        if (code >> 31) {
-            const double tmp = e.y;
-            e.y = e.z;
-            e.z = tmp;
+    const int k0 = ubCPtr[b], k1 = ubCPtr[b + 1];
+    // two contributions in flight (an edge inside the mesh has exactly two triangles), added in triangle order
+    for (int k = k0; k < k1; k += 2) {
+        unsigned int code[2];
+        double4 e[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) code[q] = k + q < k1 ? (unsigned int)ubCSrc[k + q] : 0u;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            e[q] = k + q < k1 ? load_block(elemH, (int)(code[q] & 0x7fffffffu)) : make_double4(0.0, 0.0, 0.0, 0.0);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const bool tr = (code[q] >> 31) != 0;
+            s.x += e[q].x;
+            s.y += tr ? e[q].z : e[q].y;
+            s.z += tr ? e[q].y : e[q].z;
+            s.w += e[q].w;
         }
-        s.x += e.x;
-        s.y += e.y;
-        s.z += e.z;
-        s.w += e.w;
     }
     if (u == w) {
         if (fixedMask[u]) {
@@ -610,38 +626,36 @@ void launch_step_bound(hipStream_t s, const TriSet& T, const double* UV, const d
 }
 
 // ----------------------------------------------------------------------------
+// The candidates' energies of one 256-triangle tile into Es[k][thread] and the inversion counts added to
+// cnt[k][wave]. A kernel with all candidates' code and reductions unrolled is 27-38 KB of straight-line code, and
+// fetching it took most of its time (k_linesearch 37 us, its finisher 28 us at 200k faces); the candidates are a
+// loop, and their sums go through LDS so that each wave reduces whole candidates (lsWaveSums).
 template <typename EP>
-__global__ void __launch_bounds__(kBlock) k_linesearch(TriSet T, const double2* __restrict__ UV,
-                                                       const double2* __restrict__ dir, double alphaK0,
-                                                       const unsigned long long* __restrict__ boundOrd,
-                                                       double* partials)
+__device__ __forceinline__ void ls_tile(const TriSet& T, const double2* __restrict__ UV,
+                                        const double2* __restrict__ dir, int t, bool on, bool isMesh, double alpha,
+                                        double (&Es)[kLSCand][kBlock], int (&cnt)[kLSCand][kBlock / kWave])
 {
-    constexpr int K = kLSCand;
-    if (boundOrd) alphaK0 = ordered_to_dbl(*boundOrd) * 0.99;  // Optimizer.cpp:578: 0.99 x injectivity bound
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    CSum acc[3 * K];
-#pragma unroll
-    for (int k = 0; k < 3 * K; ++k) acc[k] = CSum{0.0, 0.0};
-    if (t < T.nF) {
-        const bool isMesh = t < T.nFmesh;
+    double2 u0[3], d[3];
+    RestT<EP> r;
+    if (on) {
         const int vi[3] = {T.f0[t], T.f1[t], T.f2[t]};
-        double2 u0[3], d[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             u0[k] = UV[vi[k]];
             d[k] = dir[vi[k]];
         }
-        const RestT<EP> r = rest_as<EP>(load_rest(T, t, isMesh));
-        double alpha = alphaK0;
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
+        r = rest_as<EP>(load_rest(T, t, isMesh));
+    }
+#pragma unroll 1
+    for (int k = 0; k < kLSCand; ++k) {
+        double E = 0.0, dbA = 0.0;
+        if (on) {
             double p[3][2];
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 p[q][0] = add_rn(u0[q].x, mul_rn(alpha, d[q].x));
                 p[q][1] = add_rn(u0[q].y, mul_rn(alpha, d[q].y));
             }
-            double E, dbA;
             if constexpr (std::is_same<EP, double>::value) {
                 E = sd_energy<double>(p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], r, dbA);
             } else {
@@ -652,83 +666,114 @@ __global__ void __launch_bounds__(kBlock) k_linesearch(TriSet T, const double2* 
                 E = (double)sd_energy<EP>(EP(0), EP(0), EP(ax), EP(ay), EP(bx), EP(by), r, dbAf);
                 dbA = ax * by - ay * bx;
             }
-            acc[k].s = isMesh ? E : 0.0;
-            acc[K + k].s = isMesh ? 0.0 : E;
-            acc[2 * K + k].s = (dbA < 0.0) ? 1.0 : 0.0;  // inversion count (exact small integers)
-            alpha = alpha / 2.0;
         }
+        Es[k][threadIdx.x] = E;
+        const unsigned long long inv = __ballot(dbA < 0.0);
+        if (threadIdx.x % kWave == 0) cnt[k][threadIdx.x / kWave] += (int)__popcll(inv);
+        alpha = alpha / 2.0;
     }
-    publish_csum<3 * K>(acc, partials);
 }
+// Candidates per wave in the reduction of a tile's energies.
+constexpr int kLsPerWave = kLSCand / (kBlock / kWave);
 
-__global__ void __launch_bounds__(kBlock) k_finish_linesearch(const double* __restrict__ partials, int nblk,
-                                                              double sM, double sA, double* out)
+// Energies at K = kLSCand halvings of the step, per-workgroup compensated records [mesh K, air K, inverted K]; at most
+// kLsMaxGrid workgroups walk the tiles.
+constexpr int kLsMaxGrid = 1024;
+template <typename EP>
+__global__ void __launch_bounds__(kBlock) k_linesearch(TriSet T, const double2* __restrict__ UV,
+                                                       const double2* __restrict__ dir, double alphaK0,
+                                                       const unsigned long long* __restrict__ boundOrd,
+                                                       double* partials)
 {
     constexpr int K = kLSCand;
-    __shared__ double res[3 * K];
-    finish_csum<3 * K>(partials, nblk, res);
-    __syncthreads();
-    if (threadIdx.x == 0) {
+    __shared__ double Es[K][kBlock];
+    __shared__ int cnt[K][kBlock / kWave];
+    if (boundOrd) alphaK0 = ordered_to_dbl(*boundOrd) * 0.99;  // Optimizer.cpp:578: 0.99 x injectivity bound
+    if (threadIdx.x < K * (kBlock / kWave)) cnt[threadIdx.x / (kBlock / kWave)][threadIdx.x % (kBlock / kWave)] = 0;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    CSum mesh[kLsPerWave], air[kLsPerWave];
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            out[k] = sM * res[k] + sA * res[K + k];
-            out[K + k] = res[k];
-            out[2 * K + k] = res[K + k];
-            out[3 * K + k] = res[2 * K + k];
+    for (int c = 0; c < kLsPerWave; ++c) mesh[c] = air[c] = CSum{0.0, 0.0};
+    const int tiles = (T.nF + kBlock - 1) / kBlock;
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int t = tile * kBlock + threadIdx.x;
+        __syncthreads();
+        ls_tile<EP>(T, UV, dir, t, t < T.nF, t < T.nFmesh, alphaK0, Es, cnt);
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < kLsPerWave; ++c)
+#pragma unroll
+            for (int q = 0; q < kBlock / kWave; ++q) {
+                const int i = q * kWave + lane;
+                const CSum e{Es[wave * kLsPerWave + c][i], 0.0};
+                if (tile * kBlock + i < T.nFmesh) mesh[c] = csum_add(mesh[c], e);
+                else air[c] = csum_add(air[c], e);
+            }
+    }
+    double2* rec = reinterpret_cast<double2*>(partials) + (size_t)blockIdx.x * 3 * K;
+    const bool hasAir = T.nF > T.nFmesh;
+#pragma unroll 1
+    for (int c = 0; c < kLsPerWave; ++c) {
+        const int k = wave * kLsPerWave + c;
+        const CSum m = wave_csum(c == 0 ? mesh[0] : mesh[1]);
+        CSum a{0.0, 0.0};
+        if (hasAir) a = wave_csum(c == 0 ? air[0] : air[1]);
+        if (lane == 0) {
+            rec[k] = make_double2(m.s, m.c);
+            rec[K + k] = make_double2(a.s, a.c);
         }
+    }
+    static_assert(kLsPerWave == 2, "two candidates per wave");
+    if (threadIdx.x < K) {
+        int n = 0;
+        for (int w = 0; w < kBlock / kWave; ++w) n += cnt[threadIdx.x][w];
+        rec[2 * K + threadIdx.x] = make_double2((double)n, 0.0);  // exact small integers
     }
 }
 
-void launch_linesearch(hipStream_t s, const TriSet& T, const double* UV, const double* dir, double alpha0, int k0,
-                       double* partials, double* out, int f32, const unsigned long long* boundOrd)
+// res[v] = compensated sum over the records b of value v of NV, one value per wave at a time, four records of a
+// lane in flight.
+template <int NV, int THREADS>
+__device__ __forceinline__ void sum_csum_records(const double* __restrict__ partials, int nblk, double* res)
 {
-    double a = alpha0;
-    for (int k = 0; k < k0; ++k) a = a / 2.0;
-    const int grid = grid_for(T.nF);
-    if (f32)
-        hipLaunchKernelGGL(k_linesearch<float>, dim3(grid), dim3(kBlock), 0, s, T,
-                           reinterpret_cast<const double2*>(UV), reinterpret_cast<const double2*>(dir), a, boundOrd,
-                           partials);
-    else
-        hipLaunchKernelGGL(k_linesearch<double>, dim3(grid), dim3(kBlock), 0, s, T,
-                           reinterpret_cast<const double2*>(UV), reinterpret_cast<const double2*>(dir), a, boundOrd,
-                           partials);
-    hipLaunchKernelGGL(k_finish_linesearch, dim3(1), dim3(kBlock), 0, s, partials, grid, T.sMesh, T.sAir, out);
-}
-
-// ----------------------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock) k_axpy_commit(long n, double alpha, const double* __restrict__ d,
-                                                        double* UV)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) UV[i] = add_rn(UV[i], mul_rn(alpha, d[i]));
-}
-
-void launch_axpy_commit(hipStream_t s, long n, double alpha, const double* d, double* UV)
-{
-    hipLaunchKernelGGL(k_axpy_commit, dim3(grid_for(n)), dim3(kBlock), 0, s, n, alpha, d, UV);
+    const double2* rec = reinterpret_cast<const double2*>(partials);
+    const int lane = threadIdx.x % kWave;
+#pragma unroll 1
+    for (int v = threadIdx.x / kWave; v < NV; v += THREADS / kWave) {
+        CSum acc{0.0, 0.0};
+        for (int b = lane; b < nblk; b += 4 * kWave) {
+            double2 x[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int bb = b + q * kWave;
+                x[q] = bb < nblk ? rec[(size_t)bb * NV + v] : make_double2(0.0, 0.0);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc = csum_add(acc, CSum{x[q].x, x[q].y});
+        }
+        acc = wave_csum(acc);
+        if (lane == 0) res[v] = acc.s + acc.c;
+    }
 }
 
 // The reference's line-search rule (Optimizer.cpp:575-629) applied to the K candidates of one k_linesearch
 // launch from the bound: halve while E(alpha) > lastE, then while a triangle is inverted; alpha reaching 0 stops.
 // lastE is the host's value, or (esum non-null: the scaffold changed since it was computed, :588-592)
-// sMesh esum[0] + sAir esum[1] of the energy pass at the current UV. One thread.
-__global__ void k_ls_decide(const double* __restrict__ cand, const unsigned long long* __restrict__ boundOrd,
-                            const unsigned long long* __restrict__ airOrd, const double* __restrict__ esum,
-                            double lastEHost, double sMesh, double sAir, LsDecision* out)
+// sMesh esum[0] + sAir esum[1] of the energy pass at the current UV.
+__device__ __forceinline__ void ls_decide(const double* cand, const LsDecide& a, double sMesh, double sAir)
 {
     constexpr int K = kLSCand;
     LsDecision r{};
-    if (esum) {
-        r.lastESD = esum[0];
-        r.lastEScaf = esum[1] * sAir;
-        r.lastE = sMesh * esum[0] + r.lastEScaf;
+    if (a.esum) {
+        r.lastESD = a.esum[0];
+        r.lastEScaf = a.esum[1] * sAir;
+        r.lastE = sMesh * a.esum[0] + r.lastEScaf;
     } else {
-        r.lastE = lastEHost;
+        r.lastE = a.lastE;
     }
-    r.bound = ordered_to_dbl(*boundOrd);
-    r.airBound = airOrd ? ordered_to_dbl(airOrd[0]) : r.bound;
-    r.meshBound = airOrd ? ordered_to_dbl(airOrd[1]) : r.bound;
+    r.bound = ordered_to_dbl(*a.bound);
+    r.airBound = a.airBound ? ordered_to_dbl(a.airBound[0]) : r.bound;
+    r.meshBound = a.airBound ? ordered_to_dbl(a.airBound[1]) : r.bound;
     double alpha = r.bound * 0.99, alphaCommit = alpha;
     int k = 0, halv = 0, status = 0;
     double testE = cand[0];
@@ -760,7 +805,59 @@ __global__ void k_ls_decide(const double* __restrict__ cand, const unsigned long
     r.testES = cand[2 * K + kk] * sAir;
     r.halvings = halv;
     r.status = status;
-    *out = r;
+    *a.out = r;
+}
+
+constexpr int kLsFinishThreads = 1024;
+__global__ void __launch_bounds__(kLsFinishThreads) k_finish_linesearch(const double* __restrict__ partials, int nblk,
+                                                                        double sM, double sA, double* out,
+                                                                        LsDecide decide)
+{
+    constexpr int K = kLSCand;
+    __shared__ double res[3 * K], cand[4 * K];
+    sum_csum_records<3 * K, kLsFinishThreads>(partials, nblk, res);
+    __syncthreads();
+    const int k = threadIdx.x;
+    if (k < K) {
+        out[k] = cand[k] = sM * res[k] + sA * res[K + k];
+        out[K + k] = cand[K + k] = res[k];
+        out[2 * K + k] = cand[2 * K + k] = res[K + k];
+        out[3 * K + k] = cand[3 * K + k] = res[2 * K + k];
+    }
+    __syncthreads();
+    if (k == 0 && decide.out) ls_decide(cand, decide, sM, sA);
+}
+
+void launch_linesearch(hipStream_t s, const TriSet& T, const double* UV, const double* dir, double alpha0, int k0,
+                       double* partials, double* out, int f32, const unsigned long long* boundOrd,
+                       const LsDecide& decide)
+{
+    double a = alpha0;
+    for (int k = 0; k < k0; ++k) a = a / 2.0;
+    const int grid = std::min(grid_for(T.nF), kLsMaxGrid);
+    if (f32)
+        hipLaunchKernelGGL(k_linesearch<float>, dim3(grid), dim3(kBlock), 0, s, T,
+                           reinterpret_cast<const double2*>(UV), reinterpret_cast<const double2*>(dir), a, boundOrd,
+                           partials);
+    else
+        hipLaunchKernelGGL(k_linesearch<double>, dim3(grid), dim3(kBlock), 0, s, T,
+                           reinterpret_cast<const double2*>(UV), reinterpret_cast<const double2*>(dir), a, boundOrd,
+                           partials);
+    hipLaunchKernelGGL(k_finish_linesearch, dim3(1), dim3(kLsFinishThreads), 0, s, partials, grid, T.sMesh, T.sAir, out,
+                       decide);
+}
+
+// ----------------------------------------------------------------------------
+__global__ void __launch_bounds__(kBlock) k_axpy_commit(long n, double alpha, const double* __restrict__ d,
+                                                        double* UV)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) UV[i] = add_rn(UV[i], mul_rn(alpha, d[i]));
+}
+
+void launch_axpy_commit(hipStream_t s, long n, double alpha, const double* d, double* UV)
+{
+    hipLaunchKernelGGL(k_axpy_commit, dim3(grid_for(n)), dim3(kBlock), 0, s, n, alpha, d, UV);
 }
 
 __global__ void __launch_bounds__(kBlock) k_axpy_commit_dev(long n, const LsDecision* __restrict__ dec,
@@ -770,12 +867,8 @@ __global__ void __launch_bounds__(kBlock) k_axpy_commit_dev(long n, const LsDeci
     if (i < n && dec->status != 1) UV[i] = add_rn(UV[i], mul_rn(dec->alphaCommit, d[i]));
 }
 
-void launch_ls_decide_commit(hipStream_t s, const double* cand, const unsigned long long* boundOrd,
-                             const unsigned long long* airOrd, const double* esum, double lastEHost, double sMesh,
-                             double sAir, LsDecision* dec, long n, const double* d, double* UV)
+void launch_ls_commit(hipStream_t s, const LsDecision* dec, long n, const double* d, double* UV)
 {
-    hipLaunchKernelGGL(k_ls_decide, dim3(1), dim3(1), 0, s, cand, boundOrd, airOrd, esum, lastEHost, sMesh, sAir,
-                       dec);
     hipLaunchKernelGGL(k_axpy_commit_dev, dim3(grid_for(n)), dim3(kBlock), 0, s, n, dec, d, UV);
 }
 
@@ -1247,11 +1340,11 @@ void launch_count_inverted(hipStream_t s, const TriSet& T, const double* UV, uns
                        reinterpret_cast<const double2*>(UV), count);
 }
 
-__global__ void k_set_u64(unsigned long long* p, unsigned long long v) { *p = v; }
+__global__ void k_set_u64(unsigned long long* p, unsigned long long v) { p[threadIdx.x] = v; }
 
-void launch_set_u64(hipStream_t s, unsigned long long* p, unsigned long long v)
+void launch_set_u64(hipStream_t s, unsigned long long* p, unsigned long long v, int n)
 {
-    hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, s, p, v);
+    hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(n), 0, s, p, v);
 }
 
 __global__ void __launch_bounds__(kBlock) k_scale_copy(long n, double sign, const double* __restrict__ g,
@@ -1432,36 +1525,29 @@ __global__ void __launch_bounds__(kBlock) k_chart_linesearch(TriSet T, const dou
                                                              const double* __restrict__ alphaChart, double* partials)
 {
     constexpr int K = kLSCand;
+    __shared__ double Es[K][kBlock];
+    __shared__ int cnt[K][kBlock / kWave];
     const int2 rg = blkRange[blockIdx.x];
-    const int t = rg.x + threadIdx.x;
-    CSum acc[2 * K];
+    const int t = rg.x + threadIdx.x, wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    if (threadIdx.x < K * (kBlock / kWave)) cnt[threadIdx.x / (kBlock / kWave)][threadIdx.x % (kBlock / kWave)] = 0;
+    __syncthreads();
+    ls_tile<double>(T, UV, dir, t, t < rg.y, true, alphaChart[blkChart[blockIdx.x]], Es, cnt);
+    __syncthreads();
+    double2* rec = reinterpret_cast<double2*>(partials) + (size_t)blockIdx.x * 2 * K;
+#pragma unroll 1
+    for (int c = 0; c < kLsPerWave; ++c) {
+        const int k = wave * kLsPerWave + c;
+        CSum m{0.0, 0.0};
 #pragma unroll
-    for (int k = 0; k < 2 * K; ++k) acc[k] = CSum{0.0, 0.0};
-    if (t < rg.y) {
-        const int vi[3] = {T.f0[t], T.f1[t], T.f2[t]};
-        double2 u0[3], d[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            u0[k] = UV[vi[k]];
-            d[k] = dir[vi[k]];
-        }
-        const RestT<double> r = load_rest(T, t, true);
-        double alpha = alphaChart[blkChart[blockIdx.x]];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            double p[3][2];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                p[q][0] = add_rn(u0[q].x, mul_rn(alpha, d[q].x));
-                p[q][1] = add_rn(u0[q].y, mul_rn(alpha, d[q].y));
-            }
-            double dbA;
-            acc[k].s = sd_energy<double>(p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], r, dbA);
-            acc[K + k].s = dbA < 0.0 ? 1.0 : 0.0;
-            alpha = alpha / 2.0;
-        }
+        for (int q = 0; q < kBlock / kWave; ++q) m = csum_add(m, CSum{Es[k][q * kWave + lane], 0.0});
+        m = wave_csum(m);
+        if (lane == 0) rec[k] = make_double2(m.s, m.c);
     }
-    publish_csum<2 * K>(acc, partials);
+    if (threadIdx.x < K) {
+        int n = 0;
+        for (int w = 0; w < kBlock / kWave; ++w) n += cnt[threadIdx.x][w];
+        rec[K + threadIdx.x] = make_double2((double)n, 0.0);
+    }
 }
 
 __global__ void __launch_bounds__(kBlock) k_chart_linesearch_finish(const double* __restrict__ partials,
@@ -1470,10 +1556,7 @@ __global__ void __launch_bounds__(kBlock) k_chart_linesearch_finish(const double
     constexpr int K = kLSCand;
     const int c = blockIdx.x;
     const int b0 = chartBlk[c], nb = chartBlk[c + 1] - chartBlk[c];
-    __shared__ double res[2 * K];
-    finish_csum<2 * K>(partials + (size_t)b0 * 4 * K, nb, res);
-    __syncthreads();
-    if (threadIdx.x < 2 * K) out[(size_t)c * 2 * K + threadIdx.x] = res[threadIdx.x];
+    sum_csum_records<2 * K, kBlock>(partials + (size_t)b0 * 4 * K, nb, out + (size_t)c * 2 * K);
 }
 
 void launch_chart_linesearch(hipStream_t s, const TriSet& T, const double* UV, const double* dir, int nBlk,

@@ -51,9 +51,10 @@ void launch_triplets(hipStream_t s, const TriSet& T, const double* UV, const lon
                      const unsigned char* vFree, int* I, int* J, double* V);
 
 // g[v] = sum of contributions (in triangle order) unless vertex v is fixed;
-// gsq = ||g||^2 (last block).
+// gsq = ||g||^2 (last block); negG (may be null) = -g.
 void launch_gather_grad(hipStream_t s, int nV, const int* vcPtr, const int* vcSrc, const unsigned char* fixedMask,
-                        const double* elemG, double* g, double* partials, double* gsq);
+                        const double* elemG, double* g, double* partials, double* gsq,
+                        double* negG = nullptr);
 
 // out = total rest length of the cohesive edges that count as seam (cohE:
 // nC x 4 ids, rows with a negative id skipped; tri-soup mode: only edges
@@ -87,16 +88,7 @@ void launch_assemble(hipStream_t s, int nUB, const int* ubRow, const int* ubCol,
 void launch_step_bound(hipStream_t s, const TriSet& T, const double* UV, const double* dir,
                        unsigned long long* ordMin, double cap, unsigned long long* ordMinAir = nullptr);
 
-// Line-search energies at K candidate steps alpha_k = alpha0 / 2^(k0+k),
-// k = 0..K-1: out[k] = sMesh*E_mesh + sAir*E_air, out[K+k] = E_mesh,
-// out[2K+k] = E_air, out[3K+k] = number of triangles with negative
-// doubled area (always FP64). f32: FP32 element energies, FP64 sums.
-// boundOrd non-null: alpha0 = 0.99 x the step bound it holds (order-preserving uint64, as launch_step_bound
-// leaves it), read on the device; k0 must then be 0.
 constexpr int kLSCand = 8;
-void launch_linesearch(hipStream_t s, const TriSet& T, const double* UV, const double* dir, double alpha0, int k0,
-                       double* partials, double* out, int f32 = 0, const unsigned long long* boundOrd = nullptr);
-
 // Outcome of the line-search rule applied on the device to one batch of candidates (k_ls_decide).
 struct LsDecision {
     double alphaCommit;  // step the UV moved by (status 0 and 2)
@@ -110,13 +102,29 @@ struct LsDecision {
     int status;  // 0 accepted, 1 more than kLSCand halvings needed (nothing committed), 2 alpha underflowed to 0
     int pad[2];
 };
-// Applies Optimizer::lineSearch's rule (:597-629) to the candidates `cand` of a launch_linesearch from boundOrd
-// and, unless more candidates are needed, commits UV += alphaCommit d (n doubles). lastE: lastEHost, or with
-// esum non-null sMesh esum[0] + sAir esum[1]. airOrd (may be null): the air triangles' and the mesh triangles'
-// bounds (two words), reported.
-void launch_ls_decide_commit(hipStream_t s, const double* cand, const unsigned long long* boundOrd,
-                             const unsigned long long* airOrd, const double* esum, double lastEHost, double sMesh,
-                             double sAir, LsDecision* dec, long n, const double* d, double* UV);
+// Optimizer::lineSearch's rule (:597-629) applied to a batch of candidates that starts at 0.99 x *bound. lastE: the
+// energy they are compared with, or with esum non-null sMesh esum[0] + sAir esum[1]. airBound (may be null): the air
+// triangles' and the mesh triangles' bounds (two words), reported.
+struct LsDecide {
+    LsDecision* out = nullptr;  // null: not applied
+    const unsigned long long* bound = nullptr;
+    const unsigned long long* airBound = nullptr;
+    const double* esum = nullptr;
+    double lastE = 0.0;
+};
+
+// Line-search energies at K candidate steps alpha_k = alpha0 / 2^(k0+k),
+// k = 0..K-1: out[k] = sMesh*E_mesh + sAir*E_air, out[K+k] = E_mesh,
+// out[2K+k] = E_air, out[3K+k] = number of triangles with negative
+// doubled area (always FP64). f32: FP32 element energies, FP64 sums.
+// boundOrd non-null: alpha0 = 0.99 x the step bound it holds (order-preserving uint64, as launch_step_bound
+// leaves it), read on the device; k0 must then be 0. decide.out non-null: the rule is applied to the candidates.
+void launch_linesearch(hipStream_t s, const TriSet& T, const double* UV, const double* dir, double alpha0, int k0,
+                       double* partials, double* out, int f32 = 0, const unsigned long long* boundOrd = nullptr,
+                       const LsDecide& decide = {});
+
+// Unless the decision asks for more candidates, commits UV += alphaCommit d (n doubles).
+void launch_ls_commit(hipStream_t s, const LsDecision* dec, long n, const double* d, double* UV);
 
 // UV[i] = UV[i] + alpha * d[i] for i < n (two roundings, as the reference's
 // stepForward, Optimizer.cpp:666-669).
@@ -185,7 +193,7 @@ namespace oc {
 // *count += number of triangles with negative doubled signed UV area.
 void launch_count_inverted(hipStream_t s, const TriSet& T, const double* UV, unsigned int* count);
 // *p = v (one thread; keeps device scalars out of hipMemset so streams stay capturable).
-void launch_set_u64(hipStream_t s, unsigned long long* p, unsigned long long v);
+void launch_set_u64(hipStream_t s, unsigned long long* p, unsigned long long v, int n = 1);
 // The 2x2-block matrix newVals (current pattern) mapped onto an earlier pattern of the same n rows (oldRowPtr;
 // map: per earlier block the current block of the same (u, w) or -1; dropPtr/drop: per row the current blocks the
 // earlier pattern lacks, whose Frobenius norms go onto both diagonal entries of the row's diagonal block, oldDiag).
