@@ -500,6 +500,9 @@ __global__ void __launch_bounds__(kBlock) k_lanczos(int j, int nsteps, int n, co
                 for (int i = 0; i < BS; ++i)
 #pragma unroll
                     for (int q = 0; q < BS; ++q) m[i][q] = D[r][i * BS + q];
+#pragma unroll
+                for (int i = 0; i < BS; ++i)
+                    if (m[i][i] == 0.0) m[i][i] = 1.0;
                 block_inverse<BS>(m, mi);
                 double w[BS], x[BS];
 #pragma unroll
@@ -543,12 +546,13 @@ __global__ void __launch_bounds__(kBlock) k_lanczos(int j, int nsteps, int n, co
 // where those vectors live. h = hash * g^4, W_{-1} = D^-1 h, partial records
 // of h^T D^-1 h = |W_{-1}|_D^2 and of max g (gPart).
 // One lane group per row as in the row kernels (a thread per row walked a coarse row's 10-30 blocks one after
-// another: 13-15 us on every coarse level, now 4-5).
+// another: 13-15 us on every coarse level, now 4-6), which also forms the row's inverse diagonal block: every lane
+// inverts it, lane 0 writes it (as k_blockinv, a launch less per level; a zero diagonal entry is set to 1 in the
+// matrix itself on the coarse levels only, the finest one may be the caller's).
 template <typename T, int BS>
 __global__ void __launch_bounds__(kBlock) k_lanczos_start(int n, const int* __restrict__ rowPtr,
-                                                          const T* __restrict__ vals, const T* __restrict__ Dinv,
-                                                          double* W, double* partOut, double* gPart, double* coef,
-                                                          int nsteps)
+                                                          const int* __restrict__ diagPos, T* vals, T* Dinv, double* W,
+                                                          double* partOut, double* gPart, double* coef, int nsteps)
 {
     constexpr int LN = RowShape<BS>::lanes, RPP = kBlock / LN;
     const RowChunk rc = row_chunk<BS>(n, blockIdx.x, gridDim.x);
@@ -556,11 +560,38 @@ __global__ void __launch_bounds__(kBlock) k_lanczos_start(int n, const int* __re
     double acc[2] = {0.0, 0.0};
     double gmax = 0.0;
     for (int u = rc.r0 + sub; u < rc.r1; u += RPP) {
-        double D[BS * BS], rs[BS] = {};
-        ld_block<BS>(Dinv + (size_t)u * BS * BS, D);
-        for (int k = rowPtr[u] + lane; k < rowPtr[u + 1]; k += LN) {
+        const int k0 = rowPtr[u], k1 = rowPtr[u + 1], kd = diagPos[u];
+        double D[BS * BS], dv[BS * BS], rs[BS] = {};
+        ld_block<BS>(vals + (size_t)kd * BS * BS, dv);
+        {
+            double m[BS][BS], inv[BS][BS];
+#pragma unroll
+            for (int i = 0; i < BS; ++i)
+#pragma unroll
+                for (int j = 0; j < BS; ++j) m[i][j] = dv[i * BS + j];
+#pragma unroll
+            for (int i = 0; i < BS; ++i)
+                if (m[i][i] == 0.0) {
+                    m[i][i] = dv[i * BS + i] = 1.0;
+                    if (BS == 3 && lane == 0) vals[(size_t)kd * BS * BS + i * BS + i] = T(1);
+                }
+            block_inverse<BS>(m, inv);
+            T dt[BS * BS];
+#pragma unroll
+            for (int i = 0; i < BS * BS; ++i) {
+                dt[i] = (T)inv[i / BS][i % BS];
+                D[i] = (double)dt[i];
+            }
+            if (lane == 0)
+#pragma unroll
+                for (int i = 0; i < BS * BS; ++i) Dinv[(size_t)u * BS * BS + i] = dt[i];
+        }
+        for (int k = k0 + lane; k < k1; k += LN) {
             double a[BS * BS];
             ld_block<BS>(vals + (size_t)k * BS * BS, a);
+            if (k == kd)
+#pragma unroll
+                for (int i = 0; i < BS * BS; ++i) a[i] = dv[i];
 #pragma unroll
             for (int i = 0; i < BS; ++i)
 #pragma unroll
@@ -655,9 +686,9 @@ __device__ __forceinline__ double tridiag_top(int m, const double* al, const dou
 // Lanczos tridiagonal, or, in the safe mode (no Lanczos steps were run), the
 // Gershgorin bound / 1.1 so that the smoother's interval ends exactly at a
 // guaranteed upper bound.
-__global__ void __launch_bounds__(kBlock) k_lanczos_finish(const double* __restrict__ partIn, int nPartIn,
-                                                           const double* __restrict__ gPart, int safe, int nsteps,
-                                                           double* coef, double* lam)
+__device__ __forceinline__ void lanczos_finish(const double* __restrict__ partIn, int nPartIn,
+                                               const double* __restrict__ gPart, int safe, int nsteps,
+                                               const double* __restrict__ coef, double* lam)
 {
     __shared__ double gsh[kBlock / kWave], al[kLanczosSteps], be[kLanczosSteps];
     double g = 0.0, gq[kAmgMaxGrid / kBlock];
@@ -702,8 +733,8 @@ __global__ void __launch_bounds__(kBlock) k_lanczos_finish(const double* __restr
 constexpr int kLanczosSmallNodes = 128, kLanczosSmallThreads = 512;
 template <typename T>
 __global__ void __launch_bounds__(kLanczosSmallThreads) k_lanczos_small(int n, int safe, int nsteps, const int* __restrict__ rowPtr,
-                                                        const int* __restrict__ colIdx, const T* __restrict__ vals,
-                                                        const int* __restrict__ diagPos, double* lam)
+                                                        const int* __restrict__ colIdx, T* vals,
+                                                        const int* __restrict__ diagPos, T* Dinv, double* lam)
 {
     constexpr int BS = 3, LN = 16, GROUPS = kLanczosSmallThreads / LN, WAVES = kLanczosSmallThreads / kWave,
                   ND = kLanczosSmallNodes * BS;
@@ -734,14 +765,21 @@ __global__ void __launch_bounds__(kLanczosSmallThreads) k_lanczos_small(int n, i
     };
     for (int u = threadIdx.x; u < n; u += blockDim.x) {
         double m[BS][BS], mi[BS][BS];
-        const T* a = vals + (size_t)diagPos[u] * 9;
+        T* a = vals + (size_t)diagPos[u] * 9;
 #pragma unroll
         for (int i = 0; i < 9; ++i) m[i / 3][i % 3] = (double)a[i];
+#pragma unroll
+        for (int i = 0; i < BS; ++i)
+            if (m[i][i] == 0.0) {
+                m[i][i] = 1.0;
+                a[4 * i] = T(1);
+            }
         block_inverse<BS>(m, mi);
 #pragma unroll
         for (int i = 0; i < 9; ++i) {
             D[9 * u + i] = m[i / 3][i % 3];
             Di[9 * u + i] = mi[i / 3][i % 3];
+            Dinv[(size_t)u * 9 + i] = (T)mi[i / 3][i % 3];
         }
     }
     __syncthreads();
@@ -865,14 +903,26 @@ int setup_grid(long nOut, int lanes) { return (int)std::max<long>(1, (nOut * lan
 // dropped: zero Q column, zero R row). Q rows go to Pt (per member node),
 // R to Bout (the coarse node's near-null-space rows). kSetupLanes lanes per
 // aggregate share its members.
+// The estimate's last step (lanczos_finish, 9 us of one workgroup) has no part in this and runs as the launch's first
+// workgroup (200k faces: 9.5 + 8 us in two launches, 10 in one).
+struct LanczosEnd {
+    const double *part, *gPart, *coef;
+    double* lam;  // null: no estimate to finish
+    int nPart, safe, nsteps;
+};
 template <typename T, int BS>
 __global__ void __launch_bounds__(kBlock) k_tentative(int nc, const int* __restrict__ aggPtr,
                                                       const int* __restrict__ aggMem,
                                                       const double2* __restrict__ UV,
-                                                      const double* __restrict__ Bin, T* Pt, double* Bout)
+                                                      const double* __restrict__ Bin, T* Pt, double* Bout,
+                                                      LanczosEnd end)
 {
+    if (blockIdx.x == 0) {
+        if (end.lam) lanczos_finish(end.part, end.nPart, end.gPart, end.safe, end.nsteps, end.coef, end.lam);
+        return;
+    }
     constexpr int LANES = kSetupLanes;
-    const int c = (blockIdx.x * blockDim.x + threadIdx.x) / LANES, lane = threadIdx.x % LANES;
+    const int c = ((blockIdx.x - 1) * blockDim.x + threadIdx.x) / LANES, lane = threadIdx.x % LANES;
     const bool active = c < nc;  // whole lane groups are active or not
     if (!active) return;
     const int m0 = aggPtr[c], m1 = aggPtr[c + 1];
@@ -1633,7 +1683,9 @@ struct Amg<T>::Level : AmgHostLevel {
         *dTCol = nullptr, *dTcPtr = nullptr, *dTcA = nullptr,
         *dTcP = nullptr, *dAcPtr = nullptr, *dAcP = nullptr, *dAcT = nullptr;
     unsigned char* dPIsTent = nullptr;
-    T *vals = nullptr, *Dinv = nullptr, *Pt = nullptr, *P = nullptr, *R = nullptr, *Tv = nullptr;
+    T* vals = nullptr;      // the level's blocks; finest level in double: the caller's (numeric()), not owned
+    T* ownVals = nullptr;   // the buffer behind vals where the level has its own
+    T *Dinv = nullptr, *Pt = nullptr, *P = nullptr, *R = nullptr, *Tv = nullptr;
     T *b = nullptr, *x = nullptr, *r = nullptr, *d = nullptr;  // right-hand side, iterate, residual, direction
     double *Bnext = nullptr, *lz = nullptr, *lam = nullptr;  // lz: 6 Lanczos vectors, then alpha/beta/count
     // hand every buffer back to the owner's pool
@@ -1642,7 +1694,7 @@ struct Amg<T>::Level : AmgHostLevel {
         for (void* p : {(void*)dRowPtr, (void*)dColIdx, (void*)dDiagPos, (void*)dAggPtr, (void*)dAggMem, (void*)dPPtr,
                         (void*)dPCol, (void*)dPRow, (void*)dPsPtr, (void*)dPsA, (void*)dRPtr, (void*)dRRow, (void*)dRPos, (void*)dTPtr, (void*)dTCol,
                         (void*)dTcPtr, (void*)dTcA, (void*)dTcP, (void*)dAcPtr, (void*)dAcP, (void*)dAcT,
-                        (void*)dPIsTent, (void*)vals, (void*)Dinv, (void*)Pt, (void*)P, (void*)R, (void*)Tv, (void*)b,
+                        (void*)dPIsTent, (void*)ownVals, (void*)Dinv, (void*)Pt, (void*)P, (void*)R, (void*)Tv, (void*)b,
                         (void*)x, (void*)r, (void*)d, (void*)Bnext, (void*)lz, (void*)lam})
             if (p) pool.put(p);
     }
@@ -1731,8 +1783,8 @@ void Amg<T>::lanczos0_prepare(hipStream_t s)
     const size_t nv = (size_t)A.n * 2;
     double* coef = A.lz + 6 * nv;
     LanczosBufs lb{{A.lz, A.lz + nv, A.lz + 2 * nv}, {A.lz + 3 * nv, A.lz + 4 * nv, A.lz + 5 * nv}};
-    hipLaunchKernelGGL((k_lanczos_start<T, 2>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.vals, A.Dinv, lb.W[0],
-                       part[1], dPartials + 2 * (size_t)nPartials, coef, kLanczosSteps);
+    hipLaunchKernelGGL((k_lanczos_start<T, 2>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.dDiagPos, A.vals, A.Dinv,
+                       lb.W[0], part[1], dPartials + 2 * (size_t)nPartials, coef, kLanczosSteps);
     for (int j = 0; j < 2; ++j)
         hipLaunchKernelGGL((k_lanczos<T, 2>), dim3(g), dim3(kBlock), 0, s, j, kLanczosSteps, A.n, A.dRowPtr,
                            A.dColIdx, A.vals, A.dDiagPos, lb, part[(j + 1) & 1], g, part[j & 1], coef);
@@ -1805,7 +1857,9 @@ int Amg<T>::setup(hipStream_t s, int nV, const std::vector<int>& rowPtr, const s
         up(pool_, s, A.dRowPtr, A.rowPtr);
         up(pool_, s, A.dColIdx, A.colIdx);
         up(pool_, s, A.dDiagPos, A.diagPos);
-        dalloc(pool_, A.vals, A.colIdx.size() * bs * bs);
+        // the double hierarchy reads the caller's matrix in place (numeric())
+        if (l > 0 || !std::is_same<T, double>::value) dalloc(pool_, A.ownVals, A.colIdx.size() * bs * bs);
+        A.vals = A.ownVals;
         dalloc(pool_, A.Dinv, (size_t)A.n * bs * bs);
         dalloc(pool_, A.b, (size_t)A.n * bs);
         dalloc(pool_, A.x, (size_t)A.n * bs);
@@ -1879,12 +1933,24 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
         const int bs = A.bs;
         const long nvals = (long)A.colIdx.size() * bs * bs;
         if (l == 0) {
-            if (vals32)
-                hipLaunchKernelGGL((k_cvt<float, T>), dim3(grid_for(nvals)), dim3(kBlock), 0, s, nvals,
-                                   static_cast<const float*>(A0vals), A.vals);
-            else
-                hipLaunchKernelGGL((k_cvt<double, T>), dim3(grid_for(nvals)), dim3(kBlock), 0, s, nvals,
-                                   static_cast<const double*>(A0vals), A.vals);
+            if (std::is_same<T, double>::value && !vals32) {
+                // the matrix itself: a copy would be one more pass (14 us at 200k faces), and the PCG's product and
+                // the V-cycle would each bring their own 25 MB into the same 32 MB of L2 (with one matrix the
+                // product falls from 12.2 to 9.7 us, k_cheb_first from 10.3 to 8.8, k_correct from 13.5 to 12.4)
+                T* const a0 = static_cast<T*>(const_cast<void*>(A0vals));
+                if (A.vals != a0) ++generation_;  // captured launches name the old one
+                A.vals = a0;
+            } else {
+                if (!A.ownVals) dalloc(pool_, A.ownVals, A.colIdx.size() * bs * bs);
+                if (A.vals != A.ownVals) ++generation_;
+                A.vals = A.ownVals;
+                if (vals32)
+                    hipLaunchKernelGGL((k_cvt<float, T>), dim3(grid_for(nvals)), dim3(kBlock), 0, s, nvals,
+                                       static_cast<const float*>(A0vals), A.vals);
+                else
+                    hipLaunchKernelGGL((k_cvt<double, T>), dim3(grid_for(nvals)), dim3(kBlock), 0, s, nvals,
+                                       static_cast<const double*>(A0vals), A.vals);
+            }
         }
         if (std::is_same<T, float>::value) {  // keep the FP32-stored level positive definite
             constexpr double kShift = 4.0 / 16777216.0;
@@ -1895,14 +1961,16 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
                 hipLaunchKernelGGL((k_shift_diag<T, 3>), dim3(grid_for(A.n)), dim3(kBlock), 0, s, A.n, A.dRowPtr,
                                    A.dDiagPos, A.vals, kShift);
         }
-        if (bs == 2)
-            hipLaunchKernelGGL((k_blockinv<T, 2>), dim3(grid_for(A.n)), dim3(kBlock), 0, s, A.n, A.dDiagPos, A.vals,
-                               A.Dinv);
-        else
-            hipLaunchKernelGGL((k_blockinv<T, 3>), dim3(grid_for(A.n)), dim3(kBlock), 0, s, A.n, A.dDiagPos, A.vals,
-                               A.Dinv);
-        if (l + 1 == L.size()) break;
-        // lambda_max(D^-1 A) by Lanczos
+        if (l + 1 == L.size()) {
+            if (bs == 2)
+                hipLaunchKernelGGL((k_blockinv<T, 2>), dim3(grid_for(A.n)), dim3(kBlock), 0, s, A.n, A.dDiagPos,
+                                   A.vals, A.Dinv);
+            else
+                hipLaunchKernelGGL((k_blockinv<T, 3>), dim3(grid_for(A.n)), dim3(kBlock), 0, s, A.n, A.dDiagPos,
+                                   A.vals, A.Dinv);
+            break;
+        }
+        // lambda_max(D^-1 A) by Lanczos, and the inverse diagonal blocks on the way
         const int g = row_grid(A.n, bs);
         double* part[2] = {dPartials, dPartials + nPartials};
         const size_t nv = (size_t)A.n * bs;
@@ -1911,16 +1979,17 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
         double* gPart = dPartials + 2 * (size_t)nPartials;
         const int nsteps = lanczos_steps(l);
         const int lsafe = safe || nsteps == 0;
+        LanczosEnd end{};
         if (bs == 3 && A.n <= kLanczosSmallNodes) {
             hipLaunchKernelGGL(k_lanczos_small<T>, dim3(1), dim3(kLanczosSmallThreads), 0, s, A.n, lsafe, nsteps,
-                               A.dRowPtr, A.dColIdx, A.vals, A.dDiagPos, A.lam);
+                               A.dRowPtr, A.dColIdx, A.vals, A.dDiagPos, A.Dinv, A.lam);
         } else {
             if (bs == 2)
-                hipLaunchKernelGGL((k_lanczos_start<T, 2>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.vals, A.Dinv,
-                                   lb.W[0], part[1], gPart, coef, nsteps);
+                hipLaunchKernelGGL((k_lanczos_start<T, 2>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.dDiagPos,
+                                   A.vals, A.Dinv, lb.W[0], part[1], gPart, coef, nsteps);
             else
-                hipLaunchKernelGGL((k_lanczos_start<T, 3>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.vals, A.Dinv,
-                                   lb.W[0], part[1], gPart, coef, nsteps);
+                hipLaunchKernelGGL((k_lanczos_start<T, 3>), dim3(g), dim3(kBlock), 0, s, A.n, A.dRowPtr, A.dDiagPos,
+                                   A.vals, A.Dinv, lb.W[0], part[1], gPart, coef, nsteps);
             for (int j = 0; j < (lsafe ? 0 : nsteps); ++j) {
                 if (bs == 2)
                     hipLaunchKernelGGL((k_lanczos<T, 2>), dim3(g), dim3(kBlock), 0, s, j, nsteps, A.n, A.dRowPtr,
@@ -1929,16 +1998,15 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
                     hipLaunchKernelGGL((k_lanczos<T, 3>), dim3(g), dim3(kBlock), 0, s, j, nsteps, A.n, A.dRowPtr,
                                        A.dColIdx, A.vals, A.dDiagPos, lb, part[(j + 1) & 1], g, part[j & 1], coef);
             }
-            hipLaunchKernelGGL(k_lanczos_finish, dim3(1), dim3(kBlock), 0, s, part[(nsteps + 1) & 1], g, gPart, lsafe,
-                               nsteps, coef, A.lam);
+            end = LanczosEnd{part[(nsteps + 1) & 1], gPart, coef, A.lam, g, lsafe, nsteps};
         }
         // tentative prolongator, smoothing, Galerkin product
         Level& N = *L[l + 1];
         const int nP = (int)A.pCol.size(), nT = (int)A.tCol.size(), nAc = (int)N.colIdx.size();
         const double* Bin = l == 0 ? nullptr : L[l - 1]->Bnext;
         if (bs == 2) {
-            hipLaunchKernelGGL((k_tentative<T, 2>), dim3(setup_grid(A.nc, kSetupLanes)), dim3(kBlock), 0, s, A.nc, A.dAggPtr,
-                               A.dAggMem, reinterpret_cast<const double2*>(UV), Bin, A.Pt, A.Bnext);
+            hipLaunchKernelGGL((k_tentative<T, 2>), dim3(1 + setup_grid(A.nc, kSetupLanes)), dim3(kBlock), 0, s, A.nc,
+                               A.dAggPtr, A.dAggMem, reinterpret_cast<const double2*>(UV), Bin, A.Pt, A.Bnext, end);
             hipLaunchKernelGGL((k_smooth_p<T, 2>), dim3(setup_grid(nP, kSetupLanes)), dim3(kBlock), 0, s, nP, A.dPRow, A.dPIsTent,
                                A.dPsPtr, A.dPsA, A.dColIdx, A.vals, A.Dinv, A.Pt, A.lam, A.dRPos, A.P, A.R);
             hipLaunchKernelGGL((k_ap<T, 2>), dim3(setup_grid(nT, kSetupLanes)), dim3(kBlock), 0, s, nT, A.dTcPtr, A.dTcA, A.dTcP,
@@ -1946,8 +2014,8 @@ void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double
             hipLaunchKernelGGL((k_ptap<T, 2>), dim3(setup_grid(nAc, kSetupLanes)), dim3(kBlock), 0, s, nAc, A.dAcPtr, A.dAcP,
                                A.dAcT, A.P, A.Tv, N.vals);
         } else {
-            hipLaunchKernelGGL((k_tentative<T, 3>), dim3(setup_grid(A.nc, kSetupLanes)), dim3(kBlock), 0, s, A.nc, A.dAggPtr,
-                               A.dAggMem, reinterpret_cast<const double2*>(UV), Bin, A.Pt, A.Bnext);
+            hipLaunchKernelGGL((k_tentative<T, 3>), dim3(1 + setup_grid(A.nc, kSetupLanes)), dim3(kBlock), 0, s, A.nc,
+                               A.dAggPtr, A.dAggMem, reinterpret_cast<const double2*>(UV), Bin, A.Pt, A.Bnext, end);
             hipLaunchKernelGGL((k_smooth_p<T, 3>), dim3(setup_grid(nP, kSetupLanes)), dim3(kBlock), 0, s, nP, A.dPRow, A.dPIsTent,
                                A.dPsPtr, A.dPsA, A.dColIdx, A.vals, A.Dinv, A.Pt, A.lam, A.dRPos, A.P, A.R);
             hipLaunchKernelGGL((k_ap<T, 3>), dim3(setup_grid(nT, kSetupLanes)), dim3(kBlock), 0, s, nT, A.dTcPtr, A.dTcA, A.dTcP,
@@ -2227,6 +2295,18 @@ void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, co
     }
     hipLaunchKernelGGL((k_cheb_step<T, 2, 2>), dim3(g), dim3(kBlock), 0, s, stop, A.n, A.dRowPtr, A.dColIdx, A.vals,
                        A.Dinv, A.lam, A.d, A.x, r, z, rzPart);
+}
+
+template <typename T>
+bool Amg<T>::has_values() const
+{
+    return !L.empty() && L[0]->vals != nullptr;
+}
+
+template <typename T>
+void Amg<T>::drop_values()
+{
+    if (!L.empty() && L[0]->vals != L[0]->ownVals) L[0]->vals = nullptr;
 }
 
 template <typename T>

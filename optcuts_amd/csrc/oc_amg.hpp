@@ -60,6 +60,11 @@ public:
     virtual void cheb_step_level(hipStream_t s, int l) = 0;
     virtual int level_block_size(int l) const = 0;
     virtual bool ready() const = 0;
+    // The double hierarchy reads the finest matrix where numeric() was handed it: that buffer has to live and keep
+    // its values until the next numeric(). drop_values() forgets it (its owner is about to free or replace it);
+    // apply() and the timing launches need has_values().
+    virtual bool has_values() const = 0;
+    virtual void drop_values() = 0;
     // Largest last smoothed level (nodes) whose part of the V-cycle runs as one workgroup launch (0: never);
     // takes effect at the next setup().
     virtual void set_tail_max(int nodes) = 0;
@@ -82,8 +87,9 @@ public:
               const std::vector<unsigned char>* late = nullptr) override;
 
     // Numeric hierarchy from the fine-level block values (same layout as the
-    // pattern; double, or float when vals32) and the current UV (for the
-    // rigid near-null space).
+    // pattern; double, or float when vals32; the double hierarchy keeps
+    // reading them in place) and the current UV (for the rigid near-null
+    // space).
     void numeric(hipStream_t s, const void* A0vals, int vals32, const double* UV, int safe = 0) override;
 
     // z = M r (one V-cycle) for FP64 vectors of 2*nV; writes per-workgroup
@@ -102,6 +108,8 @@ public:
     void cheb_step_level(hipStream_t s, int l) override;
     int level_block_size(int l) const override;
     bool ready() const override { return ready_; }
+    bool has_values() const override;
+    void drop_values() override;
     void set_tail_max(int nodes) override { tailPending_ = nodes; }
 
 private:

@@ -761,6 +761,7 @@ int build_system(oc_ctx* c, bool airOnly = false)
     c->tSetup[2] = ms_since(tp);
     tp = std::chrono::steady_clock::now();
     c->amgValid = false;
+    c->amg64.drop_values();  // upload_pattern (or amg_remap below) may have replaced the buffer it reads
     c->amg = nullptr;
     c->ext = nullptr;
     c->tSetup[3] = c->tSetup[4] = 0.0;
@@ -3412,6 +3413,7 @@ int oc_time_kernel(oc_ctx* c, int which, int reps, double* ms)
     }
     (void)hipSetDevice(c->device);
     hipStream_t s = c->stream;
+    if (c->amgValid && !c->amg->has_values()) amg_numeric(c, 0);  // no step since oc_newton_init
     const TriSet T = system_set(c);
     PcgCtrl* ctrl = c->dCtrl.as<PcgCtrl>();
     // Timing copies of the partial records: the update reads a live p.q record
