@@ -196,6 +196,7 @@ struct oc_ctx {
     // matrix dVals32, each on the FP64 residual of the accumulated solution dXir
     int irMax = 0;
     DevBuf dVals32, dXir, dRir, dIrPart;
+    DevBuf dPcgSmall;                         // slot-major blocks of the one-workgroup PCG
     // block IC(0) of the Newton matrix: the preconditioner of OC_PRECOND_IC0, and the learned form's fallback
     // (its structure then built when first needed for the current pattern)
     oc::Ic0 ic0;
@@ -421,6 +422,7 @@ int ensure_pcg(oc_ctx* c, int nV)
     }
     OC_HIP(c, c->dPcgPart.ensure(sizeof(double) * (4 * (size_t)oc::pcg_grid_update(nV) +
                                                    (size_t)oc::pcg_grid_spmv(nV) + kRzRecords)));
+    OC_HIP(c, c->dPcgSmall.ensure(oc::pcg_small_bytes(nV)));
     return ensure_scratch(c, 2L * nV);
 }
 
@@ -439,6 +441,31 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
     h.maxit = maxIter;
     OC_HIP(c, hipMemcpyAsync(&ctrl->tol2, &h.tol2, sizeof(double), hipMemcpyHostToDevice, c->stream));
     OC_HIP(c, hipMemcpyAsync(&ctrl->maxit, &h.maxit, sizeof(int), hipMemcpyHostToDevice, c->stream));
+    const auto result = [&] {
+        iters = h.iter;
+        relRes = h.bb > 0.0 ? std::sqrt(h.rr / h.bb) : 0.0;
+        if (h.done == 3) {
+            c->err = "PCG breakdown (p^T A p <= 0)";
+            return OC_ERR_BREAKDOWN;
+        }
+        if (h.done == 2) {
+            c->err = "PCG reached maxIter before the tolerance";
+            return OC_ERR_NOT_CONVERGED;
+        }
+        return OC_OK;
+    };
+    if (!amg && nV <= oc::kPcgSmallRows) {
+        constexpr int kSpan = 1024;  // iterations per launch, which bounds its length (2.5-6 ms)
+        for (int it = 0; !h.done; it += kSpan) {
+            oc::launch_pcg_small(c->stream, nV, P.dRowPtr.as<int>(), P.dColIdx.as<int>(), V, V32, b,
+                                 P.dMinv.as<double>(), c->dX.as<double>(), c->dR.as<double>(), c->dP0.as<double>(),
+                                 c->dPcgSmall.p, it, it + kSpan, ctrl);
+            OC_HIP(c, hipGetLastError());
+            OC_HIP(c, hipMemcpyAsync(&h, ctrl, sizeof(PcgCtrl), hipMemcpyDeviceToHost, c->stream));
+            OC_HIP(c, hipStreamSynchronize(c->stream));
+        }
+        return result();
+    }
     const int GU = oc::pcg_grid_update(nV), GS = oc::pcg_grid_spmv(nV);
     double* partU[2] = {c->dPcgPart.as<double>(), c->dPcgPart.as<double>() + 2 * (size_t)GU};
     double* partS = c->dPcgPart.as<double>() + 4 * (size_t)GU;
@@ -548,17 +575,7 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
         batch = next;
         if (next < maxBatch) next *= 2;
     }
-    iters = h.iter;
-    relRes = h.bb > 0.0 ? std::sqrt(h.rr / h.bb) : 0.0;
-    if (h.done == 3) {
-        c->err = "PCG breakdown (p^T A p <= 0)";
-        return OC_ERR_BREAKDOWN;
-    }
-    if (h.done == 2) {
-        c->err = "PCG reached maxIter before the tolerance";
-        return OC_ERR_NOT_CONVERGED;
-    }
-    return OC_OK;
+    return result();
 }
 
 int ensure_tri_storage(oc_ctx* c, int nFtot)

@@ -1255,6 +1255,241 @@ void launch_pcg_update(hipStream_t s, int nV, const double* pNew, const double* 
     else launch(k_pcg_update<kPcgFirst64>);
 }
 
+// The whole Jacobi-PCG of a small system in one workgroup: as launches its two kernels an iteration cost their
+// latencies (9.2 us at 1,024 rows), here an iteration is three barriers and, bound by the LDS gathers of p, 2.4 us
+// (4.2 at 1,089 rows, 5.6 at 2,025, by the second row's blocks). x and the own p in registers too measured slower
+// (2.5 us: 128 registers are the limit of 16 waves, and it spills). A thread owns rows t, t + 1024, ...: its
+// first row's blocks stay in registers for the whole solve (kPcgSmallSlots of them; 64 registers in double), the second
+// row's come from the slot-major copy of k_pcg_small_pack (coalesced, from the L2 that one CU reads at 64 B a clock)
+// and p and x are in LDS. Blocks past kPcgSmallSlots of a row (a vertex of more than 7 neighbours) are read in place.
+// Iterations [it0, itEnd) of the same rule as k_pcg_spmv + k_pcg_update, state in x, r, p and ctrl between launches.
+constexpr int kPcgSmallThreads = 1024, kPcgSmallSlots = 8;
+
+template <typename V4>
+__global__ void __launch_bounds__(kBlock) k_pcg_small_pack(int nV, const int* __restrict__ rowPtr,
+                                                           const int* __restrict__ colIdx,
+                                                           const V4* __restrict__ vals, V4* ell, unsigned short* ellCol)
+{
+    const int n = nV - kPcgSmallThreads;  // rows past each thread's first
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n * kPcgSmallSlots) return;
+    const int s = q / n, v = kPcgSmallThreads + q % n;
+    const int k = rowPtr[v] + s;
+    const bool has = k < rowPtr[v + 1];
+    ell[q] = has ? vals[k] : V4{};
+    ellCol[q] = (unsigned short)(has ? colIdx[k] : v);
+}
+
+template <typename V4, int R>
+__global__ void __launch_bounds__(kPcgSmallThreads) k_pcg_small(int nV, const int* __restrict__ rowPtr,
+                                                                const int* __restrict__ colIdx,
+                                                                const V4* __restrict__ vals,
+                                                                const V4* __restrict__ ell,
+                                                                const unsigned short* __restrict__ ellCol,
+                                                                const double2* __restrict__ b,
+                                                                const double4* __restrict__ Minv, double2* x,
+                                                                double2* r, double2* p, int it0, int itEnd,
+                                                                PcgCtrl* ctrl)
+{
+    constexpr int T = kPcgSmallThreads, S = kPcgSmallSlots, WAVES = T / kWave;
+    static_assert(WAVES == 16, "the waves' sums are one row of lanes");
+    __shared__ double2 sp[R * T], sx[R * T];
+    __shared__ double4 sm[R > 1 ? (R - 1) * T : 1];  // Minv past the first row
+    __shared__ double red[2][2][WAVES];
+    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+    const int n = nV - T;
+    // Sums over the workgroup, the same in every thread; `slot` alternates so that one barrier is enough.
+    const auto sum2 = [&](int slot, double& a, double& c) {
+        a = wave_sum(a);
+        c = wave_sum(c);
+        if (lane == 0) {
+            red[slot][0][wave] = a;
+            red[slot][1][wave] = c;
+        }
+        __syncthreads();
+        double s[2] = {red[slot][0][lane % WAVES], red[slot][1][lane % WAVES]};
+        group_sum<WAVES, 2>(s);
+        a = read_lane(s[0], 0);
+        c = read_lane(s[1], 0);
+    };
+    const auto precond = [&](const double4& m, double2 v) {
+        return make_double2(m.x * v.x + m.y * v.y, m.z * v.x + m.w * v.y);
+    };
+    // the first row's blocks
+    V4 a[S];
+    int w[S / 2];  // two columns each
+    int over[R], end[R];  // [over, end): the row's blocks past the kept ones
+    double4 m0 = make_double4(0.0, 0.0, 0.0, 0.0);
+    {
+        const bool own = t < nV;
+        const int k0 = own ? rowPtr[t] : 0, k1 = own ? rowPtr[t + 1] : 0;
+        over[0] = k0 + S;
+        end[0] = k1;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const bool has = k0 + s < k1;
+            a[s] = has ? vals[k0 + s] : V4{};
+            const int c = has ? colIdx[k0 + s] : t;
+            w[s / 2] = s % 2 ? w[s / 2] | (c << 16) : c;
+        }
+        if (own) m0 = Minv[t];
+    }
+    const double tol2 = ctrl->tol2;
+    const int maxit = ctrl->maxit;
+    double2 rv[R], z[R];
+    double rz = 0.0, rr = 0.0, rzOld = ctrl->rzSlot[(it0 + 1) & 1], bb = ctrl->bb;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int v = t + i * T;
+        rv[i] = z[i] = make_double2(0.0, 0.0);
+        if (v < nV) {
+            rv[i] = it0 == 0 ? b[v] : r[v];
+            sx[v] = it0 == 0 ? make_double2(0.0, 0.0) : x[v];
+            sp[v] = it0 == 0 ? make_double2(0.0, 0.0) : p[v];
+            if (i > 0) {
+                sm[v - T] = Minv[v];
+                over[i] = rowPtr[v] + S;
+                end[i] = rowPtr[v + 1];
+            }
+            z[i] = precond(i == 0 ? m0 : sm[v - T], rv[i]);
+            rz += rv[i].x * z[i].x + rv[i].y * z[i].y;
+            rr += rv[i].x * rv[i].x + rv[i].y * rv[i].y;
+        }
+    }
+    sum2(0, rz, rr);
+    if (it0 == 0) bb = rr;
+    int it = it0, done = 0;
+    for (;; ++it) {
+        const bool conv = (bb == 0.0) || (rr <= tol2 * bb);
+        if (conv) done = 1;
+        else if (!(rz > 0.0)) done = 3;  // preconditioner not positive definite on r
+        else if (it >= maxit) done = 2;
+        if (done || it == itEnd) break;
+        const double beta = it == 0 ? 0.0 : rz / rzOld;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int v = t + i * T;
+            if (v < nV) {
+                const double2 o = sp[v];
+                sp[v] = make_double2(z[i].x + beta * o.x, z[i].y + beta * o.y);
+            }
+        }
+        __syncthreads();
+        double pq = 0.0, none = 0.0;
+        double2 q[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            q[i] = make_double2(0.0, 0.0);
+            const int v = t + i * T;
+            if (v >= nV) continue;
+            if (i == 0) {
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    const double4 as = to_double4(a[s]);
+                    const double2 ps = sp[s % 2 ? (unsigned)w[s / 2] >> 16 : w[s / 2] & 0xffff];
+                    q[0].x += as.x * ps.x + as.y * ps.y;
+                    q[0].y += as.z * ps.x + as.w * ps.y;
+                }
+            } else {
+#pragma unroll 4
+                for (int s = 0; s < S; ++s) {
+                    const int e = s * n + v - T;
+                    const double4 as = to_double4(ell[e]);
+                    const double2 ps = sp[ellCol[e]];
+                    q[i].x += as.x * ps.x + as.y * ps.y;
+                    q[i].y += as.z * ps.x + as.w * ps.y;
+                }
+            }
+            for (int k = over[i]; k < end[i]; ++k) {
+                const double4 as = to_double4(vals[k]);
+                const double2 ps = sp[colIdx[k]];
+                q[i].x += as.x * ps.x + as.y * ps.y;
+                q[i].y += as.z * ps.x + as.w * ps.y;
+            }
+            const double2 pv = sp[v];
+            pq += pv.x * q[i].x + pv.y * q[i].y;
+        }
+        sum2(1, pq, none);
+        if (!(pq > 0.0)) {  // breakdown: A not positive definite along p
+            done = 3;
+            break;
+        }
+        const double alpha = rz / pq;
+        rzOld = rz;
+        rz = rr = 0.0;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int v = t + i * T;
+            if (v < nV) {
+                const double2 pv = sp[v];
+                double2 xv = sx[v];
+                xv.x += alpha * pv.x;
+                xv.y += alpha * pv.y;
+                sx[v] = xv;
+                rv[i].x -= alpha * q[i].x;
+                rv[i].y -= alpha * q[i].y;
+                z[i] = precond(i == 0 ? m0 : sm[v - T], rv[i]);
+                rz += rv[i].x * z[i].x + rv[i].y * z[i].y;
+                rr += rv[i].x * rv[i].x + rv[i].y * rv[i].y;
+            }
+        }
+        sum2(0, rz, rr);
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int v = t + i * T;
+        if (v < nV) {
+            x[v] = sx[v];
+            r[v] = rv[i];
+            p[v] = sp[v];
+        }
+    }
+    if (t == 0) {
+        ctrl->bb = bb;
+        ctrl->rr = rr;
+        ctrl->rzSlot[it & 1] = rz;
+        ctrl->rzSlot[(it + 1) & 1] = rzOld;
+        ctrl->iter = it;
+        ctrl->done = done;
+    }
+}
+
+size_t pcg_small_bytes(int nV)
+{
+    return nV > kPcgSmallThreads && nV <= kPcgSmallRows ? (size_t)(nV - kPcgSmallThreads) * kPcgSmallSlots * (sizeof(double4) + 2) : 0;
+}
+
+template <typename V4>
+static void pcg_small(hipStream_t s, int nV, const int* rowPtr, const int* colIdx, const V4* vals, const double* b,
+                      const double* Minv, double* x, double* r, double* p, void* work, int it0, int itEnd,
+                      PcgCtrl* ctrl)
+{
+    const int n = (nV - kPcgSmallThreads) * kPcgSmallSlots;
+    V4* ell = static_cast<V4*>(work);
+    unsigned short* ellCol = reinterpret_cast<unsigned short*>(ell + std::max(0, n));
+    if (n > 0 && it0 == 0)
+        hipLaunchKernelGGL(k_pcg_small_pack<V4>, dim3(grid_for(n)), dim3(kBlock), 0, s, nV, rowPtr, colIdx, vals, ell,
+                           ellCol);
+    const auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(1), dim3(kPcgSmallThreads), 0, s, nV, rowPtr, colIdx, vals, ell, ellCol,
+                           reinterpret_cast<const double2*>(b), reinterpret_cast<const double4*>(Minv),
+                           reinterpret_cast<double2*>(x), reinterpret_cast<double2*>(r),
+                           reinterpret_cast<double2*>(p), it0, itEnd, ctrl);
+    };
+    if (nV <= kPcgSmallThreads) launch(k_pcg_small<V4, 1>);
+    else launch(k_pcg_small<V4, 2>);
+}
+
+void launch_pcg_small(hipStream_t s, int nV, const int* rowPtr, const int* colIdx, const void* vals, int vals32,
+                      const double* b, const double* Minv, double* x, double* r, double* p, void* work, int it0,
+                      int itEnd, PcgCtrl* ctrl)
+{
+    if (vals32)
+        pcg_small(s, nV, rowPtr, colIdx, static_cast<const float4*>(vals), b, Minv, x, r, p, work, it0, itEnd, ctrl);
+    else
+        pcg_small(s, nV, rowPtr, colIdx, static_cast<const double4*>(vals), b, Minv, x, r, p, work, it0, itEnd, ctrl);
+}
+
 // ----------------------------------------------------------------------------
 template <typename V4>
 __global__ void __launch_bounds__(kBlock) k_spmv(int nV, const int* __restrict__ rowPtr,

@@ -155,6 +155,15 @@ void launch_pcg_spmv(hipStream_t s, int nV, const int* rowPtr, const int* colIdx
 void launch_pcg_update(hipStream_t s, int nV, const double* pNew, const double* q, const double* Minv,
                        double* x, double* r, double* z, const double* partS, double* partUout, PcgCtrl* ctrl,
                        const FirstStep& first = {});
+// Jacobi-PCG in one workgroup for systems of at most kPcgSmallRows rows: iterations [it0, itEnd) in one launch (it0 = 0
+// starts), with pcg_small_bytes of workspace. A Newton step at 1e-10 by it, and by two launches an iteration: 0.37 and
+// 1.19 ms at 100 rows, 1.40 and 4.8 at 1,024, 4.7 and 7.4 at 2,025; with four rows a thread 15.6 and 10.6 at 3,844,
+// hence the limit of two.
+constexpr int kPcgSmallRows = 2048;
+size_t pcg_small_bytes(int nV);
+void launch_pcg_small(hipStream_t s, int nV, const int* rowPtr, const int* colIdx, const void* vals, int vals32,
+                      const double* b, const double* Minv, double* x, double* r, double* p, void* work, int it0,
+                      int itEnd, PcgCtrl* ctrl);
 
 // y = A x (2x2-block CSR; float blocks when vals32).
 void launch_spmv(hipStream_t s, int nV, const int* rowPtr, const int* colIdx, const void* vals, int vals32,
