@@ -983,11 +983,12 @@ __global__ void __launch_bounds__(kBlock) k_pcg_init(int nV, const double2* __re
 }
 
 int pcg_grid_update(int nV) { return std::max(1, std::min((nV + kBlock - 1) / kBlock, kPcgMaxGrid)); }
-// Workgroups of the PCG product: one pass of kPcgRows rows per kPcgLanes-lane
-// group, at most kPcgMaxGrid, a multiple of 8 (XCD-contiguous chunk order).
+// Workgroups of the PCG product: one row per kPcgLanes-lane group, at most kPcgMaxGrid, a multiple of 8 (XCD-contiguous
+// chunk order). Past the limit a workgroup makes several passes: up to 2,048 workgroups (one pass at 200k faces) cost
+// 6-9% there by their records, fewer with equal passes up to 2% more (405k faces).
 int pcg_grid_spmv(int nV)
 {
-    constexpr int rows = (kBlock / kPcgLanes) * kPcgRows;
+    constexpr int rows = kBlock / kPcgLanes;
     const int g = std::max(1, std::min((nV + rows - 1) / rows, kPcgMaxGrid));
     return (g + 7) & ~7;
 }
@@ -1037,8 +1038,11 @@ __device__ __forceinline__ double2 row_apply(const int* __restrict__ rowPtr, con
 // records of p_new.q. beta needs the previous update's reductions, so the
 // row loads (blocks, gathered z and p_old) are issued first and the records
 // reduced while they are in flight; p_w = z_w + beta p_old_w is formed per
-// gathered entry. kPcgRows rows per kPcgLanes-lane group; workgroup b takes
-// row chunk (b % 8) * (G / 8) + b / 8 so each XCD owns a contiguous eighth of
+// gathered entry. One row per kPcgLanes-lane group and pass, kPcgSlots blocks
+// per lane in flight (two rows a group with one block each, the second blocks
+// in a loop behind: 9.2 us an iteration at 2,116 rows and 10.1 at 100k faces
+// with the update, now 7.9 and 9.3; 8 lanes a row 7.8 and 10.0, 2 lanes of 4
+// blocks 8.2 and 9.6); workgroup b takes row chunk (b % 8) * (G / 8) + b / 8 so each XCD owns a contiguous eighth of
 // the rows (G = pcg_grid_spmv, a multiple of 8).
 template <typename V4>
 __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restrict__ rowPtr,
@@ -1055,27 +1059,23 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
     // finished PCG is seen with the records (the loads before it are harmless, nothing is written).
     const int done = ctrl->done, it = ctrl->itNext, maxit = ctrl->maxit;
     const double bbKept = ctrl->bb, tol2 = ctrl->tol2, rzOld = ctrl->rzSlot[(it + 1) & 1];
-    constexpr int LANES = kPcgLanes, UNROLL = kPcgRows, RPP = kBlock / LANES;
+    constexpr int LANES = kPcgLanes, SLOTS = kPcgSlots, RPP = kBlock / LANES;
     const int G = gridDim.x;
     const int c = (nV + G - 1) / G;
     const int r0 = ((int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3)) * c, r1 = min(nV, r0 + c);
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
-    const int passes = max(1, (c + RPP * UNROLL - 1) / (RPP * UNROLL));
+    const int passes = max(1, (c + RPP - 1) / RPP);
     const bool first = it == 0;
     double beta = 0.0;
     double acc[1] = {0.0};
     for (int pass = 0; pass < passes; ++pass) {
-        int u[UNROLL], kb[UNROLL], ke[UNROLL], w[UNROLL];
-        double4 a[UNROLL];
-        double2 gz[UNROLL], gp[UNROLL], oz[UNROLL], op[UNROLL];
+        int w[SLOTS];
+        double4 a[SLOTS];
+        double2 gz[SLOTS], gp[SLOTS], oz, op;
         double rec[2];
-#pragma unroll
-        for (int r = 0; r < UNROLL; ++r) {
-            u[r] = r0 + sub + (pass * UNROLL + r) * RPP;
-            const bool valid = u[r] < r1;
-            kb[r] = valid ? rowPtr[u[r]] : 0;
-            ke[r] = valid ? rowPtr[u[r] + 1] : 0;
-        }
+        const int u = r0 + sub + pass * RPP;
+        const bool valid = u < r1;
+        const int kb = valid ? rowPtr[u] : 0, ke = valid ? rowPtr[u + 1] : 0;
         if (pass == 0) {
             double one[1];
             sum_records<1>(partRz, nRz, sRz, one);
@@ -1084,9 +1084,9 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
             rec[1] = one[0];
         }
 #pragma unroll
-        for (int r = 0; r < UNROLL; ++r) {
-            const int k = kb[r] + lane;
-            const bool has = k < ke[r];
+        for (int r = 0; r < SLOTS; ++r) {
+            const int k = kb + lane + r * LANES;
+            const bool has = k < ke;
             const int kk = has ? k : 0;
             const double4 av = to_double4(vals[kk]);
             a[r] = has ? av : make_double4(0.0, 0.0, 0.0, 0.0);
@@ -1113,45 +1113,42 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
             if (conv || capped || indef) return;
             beta = first ? 0.0 : rz / rzOld;
         }
+        oz = op = make_double2(0.0, 0.0);
 #pragma unroll
-        for (int r = 0; r < UNROLL; ++r) {
+        for (int r = 0; r < SLOTS; ++r) {
             gz[r] = z[w[r]];
             gp[r] = first ? make_double2(0.0, 0.0) : pOld[w[r]];
-            oz[r] = op[r] = make_double2(0.0, 0.0);
-            if (lane == 0 && u[r] < r1) {
-                oz[r] = z[u[r]];
-                if (!first) op[r] = pOld[u[r]];
-            }
         }
+        if (lane == 0 && valid) {
+            oz = z[u];
+            if (!first) op = pOld[u];
+        }
+        double y[2] = {0.0, 0.0};
 #pragma unroll
-        for (int r = 0; r < UNROLL; ++r) {
-            double px = gz[r].x + beta * gp[r].x, py = gz[r].y + beta * gp[r].y;
-            double yx = a[r].x * px + a[r].y * py;
-            double yy = a[r].z * px + a[r].w * py;
-            for (int k = kb[r] + lane + LANES; k < ke[r]; k += LANES) {
-                const int wk = colIdx[k];
-                const double4 ak = to_double4(vals[k]);
-                const double2 zw = z[wk];
-                px = zw.x;
-                py = zw.y;
-                if (!first) {
-                    const double2 pw = pOld[wk];
-                    px += beta * pw.x;
-                    py += beta * pw.y;
-                }
-                yx += ak.x * px + ak.y * py;
-                yy += ak.z * px + ak.w * py;
+        for (int r = 0; r < SLOTS; ++r) {
+            const double px = gz[r].x + beta * gp[r].x, py = gz[r].y + beta * gp[r].y;
+            y[0] += a[r].x * px + a[r].y * py;
+            y[1] += a[r].z * px + a[r].w * py;
+        }
+        for (int k = kb + lane + SLOTS * LANES; k < ke; k += LANES) {
+            const int wk = colIdx[k];
+            const double4 ak = to_double4(vals[k]);
+            const double2 zw = z[wk];
+            double px = zw.x, py = zw.y;
+            if (!first) {
+                const double2 pw = pOld[wk];
+                px += beta * pw.x;
+                py += beta * pw.y;
             }
-            double y[2] = {yx, yy};
-            group_sum<LANES, 2>(y);
-            yx = y[0];
-            yy = y[1];
-            if (lane == 0 && u[r] < r1) {
-                const double2 pn = make_double2(oz[r].x + beta * op[r].x, oz[r].y + beta * op[r].y);
-                pNew[u[r]] = pn;
-                q[u[r]] = make_double2(yx, yy);
-                acc[0] += pn.x * yx + pn.y * yy;
-            }
+            y[0] += ak.x * px + ak.y * py;
+            y[1] += ak.z * px + ak.w * py;
+        }
+        group_sum<LANES, 2>(y);
+        if (lane == 0 && valid) {
+            const double2 pn = make_double2(oz.x + beta * op.x, oz.y + beta * op.y);
+            pNew[u] = pn;
+            q[u] = make_double2(y[0], y[1]);
+            acc[0] += pn.x * y[0] + pn.y * y[1];
         }
     }
     block_sum<1>(acc);
