@@ -204,7 +204,7 @@ struct oc_ctx {
     oc::Preconditioner* ext = nullptr;     // the external preconditioner of the Newton PCG, if any
 
     // ---- PCG workspace ---------------------------------------------------------
-    DevBuf dX, dR, dZ, dP0, dP1, dQ, dB, dCtrl, dPcgPart;
+    DevBuf dX, dR, dR1, dZ, dP0, dP1, dQ, dB, dCtrl, dPcgPart;
     // PCG iterations replayed from captured HIP graphs (an even iteration,
     // an odd one, an even+odd pair, a run of pairs), valid for the buffers
     // and sizes recorded in pcgSig
@@ -411,6 +411,7 @@ int ensure_pcg(oc_ctx* c, int nV)
     const size_t b = sizeof(double) * 2 * (size_t)std::max(1, nV);
     OC_HIP(c, c->dX.ensure(b));
     OC_HIP(c, c->dR.ensure(b));
+    OC_HIP(c, c->dR1.ensure(b));
     OC_HIP(c, c->dZ.ensure(b));
     OC_HIP(c, c->dP0.ensure(b));
     OC_HIP(c, c->dP1.ensure(b));
@@ -420,7 +421,7 @@ int ensure_pcg(oc_ctx* c, int nV)
         OC_HIP(c, c->dCtrl.ensure(sizeof(PcgCtrl)));
         OC_HIP(c, hipMemsetAsync(c->dCtrl.p, 0, sizeof(PcgCtrl), c->stream));
     }
-    OC_HIP(c, c->dPcgPart.ensure(sizeof(double) * (4 * (size_t)oc::pcg_grid_update(nV) +
+    OC_HIP(c, c->dPcgPart.ensure(sizeof(double) * (4 * (size_t)std::max(oc::pcg_grid_update(nV), oc::pcg_grid_spmv(nV)) +
                                                    (size_t)oc::pcg_grid_spmv(nV) + kRzRecords)));
     OC_HIP(c, c->dPcgSmall.ensure(oc::pcg_small_bytes(nV)));
     return ensure_scratch(c, 2L * nV);
@@ -466,7 +467,8 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
         }
         return result();
     }
-    const int GU = oc::pcg_grid_update(nV), GS = oc::pcg_grid_spmv(nV);
+    const bool fused = amg && amg->update_records() > 0;
+    const int GU = fused ? amg->update_records() : oc::pcg_grid_update(nV), GS = oc::pcg_grid_spmv(nV);
     double* partU[2] = {c->dPcgPart.as<double>(), c->dPcgPart.as<double>() + 2 * (size_t)GU};
     double* partS = c->dPcgPart.as<double>() + 4 * (size_t)GU;
     double* partRZ = partS + GS;
@@ -479,9 +481,10 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
         amg->apply(c->stream, c->dR.as<double>(), c->dZ.as<double>(), partRZ, &ctrl->done, first.d ? &stage : nullptr);
     };
     oc::launch_pcg_init(c->stream, nV, b, Minv, c->dX.as<double>(), c->dR.as<double>(), c->dZ.as<double>(), partU[0],
-                        ctrl, first);
+                        GU, ctrl, first);
     if (amg) precondition(partU[0]);
     double* pbuf[2] = {c->dP0.as<double>(), c->dP1.as<double>()};
+    double* rbuf[2] = {c->dR.as<double>(), c->dR1.as<double>()};  // a fused update alternates
     // One iteration's launches. The kernels take the iteration number from
     // the control record, so the launches depend only on its parity (which
     // buffers alternate) and every iteration of one parity is the same graph.
@@ -497,6 +500,13 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
             oc::launch_pcg_spmv(c->stream, nV, P.dRowPtr.as<int>(), P.dColIdx.as<int>(), V, V32,
                                 c->dZ.as<double>(), pOld, pNew, c->dQ.as<double>(), pu, GU, 2, pu + 1, GU, 2, partS,
                                 ctrl);
+        if (fused) {
+            amg->update_apply(c->stream,
+                              oc::PcgUpdate{pNew, c->dQ.as<double>(), rbuf[par], c->dX.as<double>(), rbuf[par ^ 1],
+                                            partS, GS, partU[par ^ 1], ctrl},
+                              c->dZ.as<double>(), partRZ);
+            return;
+        }
         oc::launch_pcg_update(c->stream, nV, pNew, c->dQ.as<double>(), Minv, c->dX.as<double>(), c->dR.as<double>(),
                               c->dZ.as<double>(), partS, partU[par ^ 1], ctrl, first);
         if (amg) precondition(partU[par ^ 1]);
@@ -509,6 +519,7 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
         const uintptr_t sig[] = {(uintptr_t)nV,           (uintptr_t)P.dRowPtr.p, (uintptr_t)P.dColIdx.p,
                                  (uintptr_t)V,            (uintptr_t)V32,         (uintptr_t)Minv,
                                  (uintptr_t)c->dX.p,      (uintptr_t)c->dR.p,     (uintptr_t)c->dZ.p,
+                                 (uintptr_t)c->dR1.p,
                                  (uintptr_t)c->dP0.p,     (uintptr_t)c->dP1.p,    (uintptr_t)c->dQ.p,
                                  (uintptr_t)c->dPcgPart.p, (uintptr_t)ctrl,       (uintptr_t)amg,
                                  amg ? (uintptr_t)amg->generation() : 0, amg ? (uintptr_t)amg->rz_records() : 0};

@@ -189,6 +189,25 @@ __device__ __forceinline__ void block_sum(double (&v)[NV])
     __syncthreads();
 }
 
+// Workgroup sums of every thread's values, identical in every thread of every workgroup that sums the same values.
+template <int NV>
+__device__ __forceinline__ void all_sum(double (&acc)[NV])
+{
+    __shared__ double sh[kBlock / kWave][NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) acc[k] = wave_sum(acc[k]);
+    if (threadIdx.x % kWave == 0)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) sh[threadIdx.x / kWave][k] = acc[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        acc[k] = sh[0][k];
+#pragma unroll
+        for (int w = 1; w < kBlock / kWave; ++w) acc[k] += sh[w][k];
+    }
+}
+
 // Order-preserving map of a double to uint64 (for atomicMin over doubles of
 // either sign); NaN inputs are filtered by the caller.
 __device__ __forceinline__ unsigned long long dbl_to_ordered(double x)

@@ -381,6 +381,46 @@ __device__ __forceinline__ double2 probe(int u, unsigned int seed, unsigned int 
                         (probe_hash(2u * u + 1u, seed, j) & 1u) ? 1.0 : -1.0);
 }
 
+// The factor products: kRowLanes lanes per row with kRowEdges edges each in flight, the rest in a loop (a thread per
+// row walked its 6 edges one after another with a wave per SIMD of 99 CUs at 50k faces: G 4.7 us, G^T 6.2 us). With
+// k_gnn_update_G (5.6 us, G^T 4.6) a learned Newton step took 8.3 -> 7.1 ms at 50k faces and 21.4 -> 17.5 at 79k; four lanes of two
+// edges 6.9 and 19.7, eight of one 8.0 and 21.7 (more passes of the at most kGnnMaxGrid workgroups, each on a
+// contiguous chunk of rows).
+constexpr int kRowLanes = 2, kRowEdges = 4;
+int row_blocks(int nV) { return blocks_for((long)nV * kRowLanes, kBlock); }
+
+// Sum over row u's edges into lower (LOWER: w < u) or upper neighbours, in every lane of the row: body(e, w) gives the
+// edge's term.
+template <bool LOWER, typename Body>
+__device__ __forceinline__ double2 edge_sum(const int* __restrict__ ew, int u, int e0, int e1, int lane,
+                                            const Body& body)
+{
+    double y[2] = {0.0, 0.0};
+    int w[kRowEdges];
+#pragma unroll
+    for (int k = 0; k < kRowEdges; ++k) {
+        const int e = e0 + lane + k * kRowLanes;
+        w[k] = e < e1 ? ew[e] : u;
+    }
+#pragma unroll
+    for (int k = 0; k < kRowEdges; ++k)
+        if (LOWER ? w[k] < u : w[k] > u) {
+            const double2 t = body(e0 + lane + k * kRowLanes, w[k]);
+            y[0] += t.x;
+            y[1] += t.y;
+        }
+    for (int e = e0 + lane + kRowEdges * kRowLanes; e < e1; e += kRowLanes) {
+        const int v = ew[e];
+        if (LOWER ? v < u : v > u) {
+            const double2 t = body(e, v);
+            y[0] += t.x;
+            y[1] += t.y;
+        }
+    }
+    group_sum<kRowLanes, 2>(y);
+    return make_double2(y[0], y[1]);
+}
+
 enum { kApplyPrecond = 0, kApplyLoss = 1 };
 
 // out = G^ s, s_x = C^-1 in_x (precond) or in_x (loss: then out = 2 norm (G^ t - w), loss records)
@@ -395,33 +435,88 @@ __global__ void __launch_bounds__(kBlock) k_gnn_apply_G(int nV, const int* __res
     if (stop && *stop) return;
     long r0, r1;
     chunk(nV, r0, r1);
+    const int sub = threadIdx.x / kRowLanes, lane = threadIdx.x % kRowLanes;
     double acc[1] = {0.0};
-    for (long u = r0 + threadIdx.x; u < r1; u += blockDim.x) {
+    for (int u = (int)r0 + sub; u < r1; u += kBlock / kRowLanes) {
         double2 su = in[u];
         if (MODE == kApplyPrecond) su = bmv(Cinv[u], su);
         double2 o = bmv(Gd[u], su);
-        for (int e = rowE[u]; e < rowE[u + 1]; ++e) {
-            const int w = ew[e];
-            if (w >= u) continue;
+        const double2 t = edge_sum<true>(ew, u, rowE[u], rowE[u + 1], lane, [&](int e, int w) {
             double2 sw = in[w];
             if (MODE == kApplyPrecond) sw = bmv(Cinv[w], sw);
-            const double2 g = bmv(Go[e], sw);
-            o.x += g.x;
-            o.y += g.y;
-        }
+            return bmv(Go[e], sw);
+        });
+        o.x += t.x;
+        o.y += t.y;
         if (MODE == kApplyLoss) {
-            const double2 wv = probe((int)u, seed, pj);
+            const double2 wv = probe(u, seed, pj);
             o.x -= wv.x;
             o.y -= wv.y;
-            acc[0] += o.x * o.x + o.y * o.y;
+            if (lane == 0) acc[0] += o.x * o.x + o.y * o.y;
             o.x *= 2.0 * norm;
             o.y *= 2.0 * norm;
         }
-        out[u] = o;
+        if (lane == 0) out[u] = o;
     }
     if (MODE == kApplyLoss) {
         block_sum<1>(acc);
         if (threadIdx.x == 0) part[blockIdx.x] = acc[0] * norm;
+    }
+}
+
+// A PCG update with the product by G^ on the new residual in the same launch (a launch less of four an iteration): a
+// gathered residual is formed as r_w - alpha q_w again, so the new one goes to another buffer.
+__global__ void __launch_bounds__(kBlock) k_gnn_update_G(int nV, const int* __restrict__ rowE,
+                                                         const int* __restrict__ ew, const float4* __restrict__ Cinv,
+                                                         const float4* __restrict__ Go, const float4* __restrict__ Gd,
+                                                         const double2* __restrict__ p, const double2* __restrict__ q,
+                                                         const double2* __restrict__ rOld, double2* x, double2* rNew,
+                                                         double2* out, const double* __restrict__ partS, int nPartS,
+                                                         double* partU, PcgCtrl* ctrl)
+{
+    const int done = ctrl->done, it = ctrl->itCur;
+    const double rzCur = ctrl->rzSlot[it & 1];
+    long r0, r1;
+    chunk(nV, r0, r1);
+    const int sub = threadIdx.x / kRowLanes, lane = threadIdx.x % kRowLanes;
+    double pq[1];
+    sum_records<1>(partS, nPartS, 1, pq);
+    all_sum<1>(pq);
+    if (done) return;
+    if (!(pq[0] > 0.0)) {  // breakdown: A not positive definite along p
+        if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->done = 3;
+        return;
+    }
+    const double alpha = rzCur / pq[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->itNext = it + 1;
+    double acc[2] = {0.0, 0.0};
+    const auto residual = [&](int w) {
+        double2 r = rOld[w];
+        const double2 qw = q[w];
+        r.x -= alpha * qw.x;
+        r.y -= alpha * qw.y;
+        return r;
+    };
+    for (int u = (int)r0 + sub; u < r1; u += kBlock / kRowLanes) {
+        const double2 ru = residual(u);
+        double2 o = bmv(Gd[u], bmv(Cinv[u], ru));
+        const double2 t = edge_sum<true>(ew, u, rowE[u], rowE[u + 1], lane,
+                                         [&](int e, int w) { return bmv(Go[e], bmv(Cinv[w], residual(w))); });
+        if (lane == 0) {
+            const double2 pu = p[u];
+            double2 xu = x[u];
+            xu.x += alpha * pu.x;
+            xu.y += alpha * pu.y;
+            x[u] = xu;
+            rNew[u] = ru;
+            out[u] = make_double2(o.x + t.x, o.y + t.y);
+            acc[1] += ru.x * ru.x + ru.y * ru.y;
+        }
+    }
+    block_sum<2>(acc);
+    if (threadIdx.x == 0) {
+        partU[2 * blockIdx.x] = acc[0];
+        partU[2 * blockIdx.x + 1] = acc[1];
     }
 }
 
@@ -440,24 +535,23 @@ __global__ void __launch_bounds__(kBlock) k_gnn_apply_GT(int nV, const int* __re
     if (stop && *stop) return;
     long r0, r1;
     chunk(nV, r0, r1);
+    const int sub = threadIdx.x / kRowLanes, lane = threadIdx.x % kRowLanes;
     double acc[1] = {0.0};
-    for (long u = r0 + threadIdx.x; u < r1; u += blockDim.x) {
-        const double2 iu = MODE == kGTProbe ? probe((int)u, seed, pj) : in[u];
+    for (int u = (int)r0 + sub; u < r1; u += kBlock / kRowLanes) {
+        const double2 iu = MODE == kGTProbe ? probe(u, seed, pj) : in[u];
         double2 y = bmtv(Gd[u], iu);
-        for (int e = rowE[u]; e < rowE[u + 1]; ++e) {
-            const int w = ew[e];
-            if (w <= u) continue;
+        const double2 t = edge_sum<false>(ew, u, rowE[u], rowE[u + 1], lane, [&](int e, int w) {
             const double2 iw = MODE == kGTProbe ? probe(w, seed, pj) : in[w];
-            const double2 g = bmtv(Go[rev[e]], iw);
-            y.x += g.x;
-            y.y += g.y;
-        }
+            return bmtv(Go[rev[e]], iw);
+        });
+        y.x += t.x;
+        y.y += t.y;
         if (MODE == kGTPrecond) {
             y = bmtv(Cinv[u], y);
             const double2 rv = r[u];
-            acc[0] += rv.x * y.x + rv.y * y.y;
+            if (lane == 0) acc[0] += rv.x * y.x + rv.y * y.y;
         }
-        out[u] = y;
+        if (lane == 0) out[u] = y;
     }
     if (MODE == kGTPrecond) {
         block_sum<1>(acc);
@@ -1085,20 +1179,35 @@ void Gnn::forward(hipStream_t s, const void* vals, int vals32)
                        dTheta, dFixed, reinterpret_cast<float4*>(dGd));
 }
 
-int Gnn::rz_records() const { return blocks_for(nV, kBlock); }
+int Gnn::rz_records() const { return row_blocks(nV); }
+int Gnn::update_records() const { return row_blocks(nV); }
 
 void Gnn::apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop, const PcgStage*)
 {
-    const int g = blocks_for(nV, kBlock);
-    const float4* Ci = reinterpret_cast<const float4*>(dCinv);
-    const float4* Go = reinterpret_cast<const float4*>(dGo);
-    const float4* Gd = reinterpret_cast<const float4*>(dGd);
-    hipLaunchKernelGGL(k_gnn_apply_G<kApplyPrecond>, dim3(g), dim3(kBlock), 0, s, nV, dRowE, dEw, Ci, Go, Gd,
-                       reinterpret_cast<const double2*>(r), reinterpret_cast<double2*>(dTmp), 0.0, 0u, 0u, nullptr,
-                       stop);
-    hipLaunchKernelGGL(k_gnn_apply_GT<kGTPrecond>, dim3(g), dim3(kBlock), 0, s, nV, dRowE, dEw, dRev, Ci, Go, Gd,
-                       reinterpret_cast<const double2*>(dTmp), reinterpret_cast<double2*>(z),
-                       reinterpret_cast<const double2*>(r), rzPart, 0u, 0u, stop);
+    hipLaunchKernelGGL(k_gnn_apply_G<kApplyPrecond>, dim3(row_blocks(nV)), dim3(kBlock), 0, s, nV, dRowE, dEw,
+                       reinterpret_cast<const float4*>(dCinv), reinterpret_cast<const float4*>(dGo),
+                       reinterpret_cast<const float4*>(dGd), reinterpret_cast<const double2*>(r),
+                       reinterpret_cast<double2*>(dTmp), 0.0, 0u, 0u, nullptr, stop);
+    apply_GT(s, r, z, rzPart, stop);
+}
+
+void Gnn::apply_GT(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop)
+{
+    hipLaunchKernelGGL(k_gnn_apply_GT<kGTPrecond>, dim3(row_blocks(nV)), dim3(kBlock), 0, s, nV, dRowE, dEw, dRev,
+                       reinterpret_cast<const float4*>(dCinv), reinterpret_cast<const float4*>(dGo),
+                       reinterpret_cast<const float4*>(dGd), reinterpret_cast<const double2*>(dTmp),
+                       reinterpret_cast<double2*>(z), reinterpret_cast<const double2*>(r), rzPart, 0u, 0u, stop);
+}
+
+void Gnn::update_apply(hipStream_t s, const PcgUpdate& u, double* z, double* rzPart)
+{
+    hipLaunchKernelGGL(k_gnn_update_G, dim3(row_blocks(nV)), dim3(kBlock), 0, s, nV, dRowE, dEw,
+                       reinterpret_cast<const float4*>(dCinv), reinterpret_cast<const float4*>(dGo),
+                       reinterpret_cast<const float4*>(dGd), reinterpret_cast<const double2*>(u.p),
+                       reinterpret_cast<const double2*>(u.q), reinterpret_cast<const double2*>(u.rOld),
+                       reinterpret_cast<double2*>(u.x), reinterpret_cast<double2*>(u.rNew),
+                       reinterpret_cast<double2*>(dTmp), u.partS, u.nPartS, u.partU, u.ctrl);
+    apply_GT(s, u.rNew, z, rzPart, &u.ctrl->done);
 }
 
 void Gnn::zero_grad(hipStream_t s)
@@ -1109,7 +1218,7 @@ void Gnn::zero_grad(hipStream_t s)
 
 void Gnn::loss_grad(hipStream_t s, int nProbes, unsigned seed, double* dLoss)
 {
-    const int g = blocks_for(nV, kBlock);
+    const int g = row_blocks(nV);
     const float4* Ci = reinterpret_cast<const float4*>(dCinv);
     const float4* Go = reinterpret_cast<const float4*>(dGo);
     const float4* Gd = reinterpret_cast<const float4*>(dGd);

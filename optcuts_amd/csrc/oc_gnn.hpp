@@ -78,6 +78,8 @@ public:
     void apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop,
                const PcgStage* pcg = nullptr) override;
     int rz_records() const override;
+    int update_records() const override;
+    void update_apply(hipStream_t s, const PcgUpdate& u, double* z, double* rzPart) override;
 
     // Training (after forward): adds dL/dtheta to grads(), *dLoss (device) += L.
     void zero_grad(hipStream_t s);
@@ -92,6 +94,7 @@ public:
     const int* edge_slots() const { return dESlot; }
 
 private:
+    void apply_GT(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop);
     int nV = 0, E = 0;
     // parameters
     float *dTheta = nullptr, *dGrad = nullptr, *dAdamM = nullptr, *dAdamV = nullptr;

@@ -898,25 +898,6 @@ __device__ __forceinline__ double4 to_double4(const float4& v)
     return make_double4((double)v.x, (double)v.y, (double)v.z, (double)v.w);
 }
 
-// Workgroup sums of every thread's values, identical in every thread of every workgroup that sums the same values.
-template <int NV>
-__device__ __forceinline__ void all_sum(double (&acc)[NV])
-{
-    __shared__ double sh[kBlock / kWave][NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) acc[k] = wave_sum(acc[k]);
-    if (threadIdx.x % kWave == 0)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) sh[threadIdx.x / kWave][k] = acc[k];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        acc[k] = sh[0][k];
-#pragma unroll
-        for (int w = 1; w < kBlock / kWave; ++w) acc[k] += sh[w][k];
-    }
-}
-
 __device__ __forceinline__ void row_chunk(int nV, int& r0, int& r1)
 {
     const int chunk = (nV + (int)gridDim.x - 1) / (int)gridDim.x;
@@ -994,10 +975,10 @@ int pcg_grid_spmv(int nV)
 }
 
 void launch_pcg_init(hipStream_t s, int nV, const double* b, const double* Minv, double* x, double* r, double* z,
-                     double* partU, PcgCtrl* ctrl, const FirstStep& first)
+                     double* partU, int records, PcgCtrl* ctrl, const FirstStep& first)
 {
     const auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(pcg_grid_update(nV)), dim3(kBlock), 0, s, nV,
+        hipLaunchKernelGGL(kern, dim3(records), dim3(kBlock), 0, s, nV,
                            reinterpret_cast<const double2*>(b), Minv, first, reinterpret_cast<double2*>(x),
                            reinterpret_cast<double2*>(r), reinterpret_cast<double2*>(z), partU, ctrl);
     };

@@ -147,7 +147,7 @@ int pcg_grid_spmv(int nV);
 // first (without Minv): the external preconditioner's first step, computed
 // by init / update(i) from the residual they write.
 void launch_pcg_init(hipStream_t s, int nV, const double* b, const double* Minv, double* x, double* r, double* z,
-                     double* partU, PcgCtrl* ctrl, const FirstStep& first = {});
+                     double* partU, int records, PcgCtrl* ctrl, const FirstStep& first = {});
 // vals: double4 blocks, or float4 blocks when vals32 (FP64 arithmetic either way).
 void launch_pcg_spmv(hipStream_t s, int nV, const int* rowPtr, const int* colIdx, const void* vals,
                      int vals32, const double* z, const double* pOld, double* pNew, double* q, const double* partRz,

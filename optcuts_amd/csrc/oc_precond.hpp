@@ -34,6 +34,17 @@ struct PcgStage {
     PcgCtrl* ctrl = nullptr;
 };
 
+// The PCG update of one iteration (alpha = rz / sum of the p.q records, x += alpha p, rNew = rOld - alpha q) with its
+// records (value 2b + 1 of partU: r.r), for a preconditioner that does it in its first kernel.
+struct PcgUpdate {
+    const double *p, *q, *rOld;
+    double *x, *rNew;
+    const double* partS;
+    int nPartS;
+    double* partU;
+    PcgCtrl* ctrl;
+};
+
 // Chebyshev parameters on [lmax/30, lmax], lmax = 1.1 * lambda estimate
 struct ChebP {
     double theta, delta, sigma;
@@ -60,6 +71,10 @@ struct Preconditioner {
                        const PcgStage* pcg = nullptr) = 0;
     virtual int rz_records() const = 0;
     virtual FirstStep first_step() const { return {}; }
+    // Records of an update made by update_apply(), which then stands for the
+    // PCG's update and apply(); 0: not offered.
+    virtual int update_records() const { return 0; }
+    virtual void update_apply(hipStream_t, const PcgUpdate&, double* /*z*/, double* /*rzPart*/) {}
     // Changes whenever the device buffers apply() launches on may have
     // changed (a new set-up); launches captured into a graph stay valid while
     // it holds.
