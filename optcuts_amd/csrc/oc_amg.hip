@@ -146,8 +146,8 @@ __device__ __forceinline__ double hash_unit(unsigned int i)
 }
 
 // lambda_max(D^-1 A) by Lanczos in the D inner product (D^-1 A is self-adjoint
-// there; D is the block diagonal with zero diagonal entries set to 1, as in
-// k_blockinv). Ritz values approach the extreme eigenvalues far faster than
+// there; D is the block diagonal with zero diagonal entries set to 1, in the
+// matrix too on the coarse levels). Ritz values approach the extreme eigenvalues far faster than
 // power iteration does when the top of the spectrum is clustered (large
 // meshes), and they never exceed lambda_max.
 //
@@ -729,7 +729,7 @@ __device__ __forceinline__ void lanczos_finish(const double* __restrict__ partIn
 // path is one chain of dependent loads and a reduction (6 us a step), here the recurrence's vectors and the diagonal
 // blocks stay in LDS and a step is one pass over the row blocks between two barriers. 32 nodes: 77 -> 40 us; at
 // 250 nodes the single workgroup's four passes a step take as long as the launches (88 against 77 us).
-// Same formulas as k_lanczos_start, k_lanczos and k_lanczos_finish.
+// Same formulas as k_lanczos_start, k_lanczos and lanczos_finish.
 constexpr int kLanczosSmallNodes = 128, kLanczosSmallThreads = 512;
 template <typename T>
 __global__ void __launch_bounds__(kLanczosSmallThreads) k_lanczos_small(int n, int safe, int nsteps, const int* __restrict__ rowPtr,
@@ -1447,7 +1447,7 @@ __global__ void __launch_bounds__(kBlock) k_cheb_post1(const int* __restrict__ s
 // without passing through the block index; with the XCD chunk order the residual rows of neighbouring nodes stay
 // in one L2. Gathering 48-byte P blocks from workgroups dealt round robin ran at 2 TB/s (1M faces, finest level:
 // 38 us, now 24; 200k faces 9.9, now 6.0).
-// PRE1: the next level's first pre-smoothing step (k_cheb_pre1) is row-local,
+// PRE1: the next level's first pre-smoothing step (d = Dinv r / theta) is row-local,
 // so it runs here on each restricted row instead of in a launch of its own.
 template <typename T, int BS, bool PRE1, int LN, int NT = kBlock>
 __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int* __restrict__ rPtr,

@@ -89,7 +89,7 @@ void launch_step_bound(hipStream_t s, const TriSet& T, const double* UV, const d
                        unsigned long long* ordMin, double cap, unsigned long long* ordMinAir = nullptr);
 
 constexpr int kLSCand = 8;
-// Outcome of the line-search rule applied on the device to one batch of candidates (k_ls_decide).
+// Outcome of the line-search rule applied on the device to one batch of candidates (ls_decide).
 struct LsDecision {
     double alphaCommit;  // step the UV moved by (status 0 and 2)
     double alpha;        // accepted step (0 when stopped)

@@ -8,7 +8,7 @@ namespace oc {
 // The iteration number lives here, not in launch arguments, so that every
 // iteration of one parity launches identical arguments (graph replay):
 // k_pcg_init sets itNext = 0; k_pcg_spmv reads itNext and records it in itCur
-// (and iter); k_pcg_update reads itCur and sets itNext = itCur + 1. Each field
+// (and iter); k_pcg_update (or update_apply()) reads itCur and sets itNext = itCur + 1. Each field
 // is written by one kernel and read only by the next.
 struct PcgCtrl {
     double bb, tol2, rr, pad0;
