@@ -1548,6 +1548,9 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const int* __restrict__ stop
 // between the smoothing steps that do read A, so only the saved launch counts there: up to kCorrectMaxFine rows.
 // Whole Newton step, this pass against prolongation + product: 25k rows 1546 / 1565 us, 51k 2020 / 2043, 100k 2988 /
 // 3016, 203k 4953 / 4809, 501k 9084 / 8977. kCorrectLanes lanes per fine row.
+// FP32 storage keeps the product from the corrected x on the finest level: the residual formed here does not see the
+// rounding of the stored x, which the post-smoothing then leaves in z (joint-mode run on 200k faces in the mixed form:
+// one safe-interval retry and three Jacobi solves in 58 steps, against none and one in 51).
 constexpr int kCorrectLanes = 8;
 constexpr int kCorrectMaxFine = 131072;
 template <typename T, int BS, int NT = kBlock>
@@ -2284,7 +2287,7 @@ void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, co
                        A.vals, r, A.x, A.r);
     restrict_to(s, 0, stop);
     vcycle(s, 1, stop);
-    if (A.n <= kCorrectMaxFine) {
+    if (std::is_same<T, double>::value && A.n <= kCorrectMaxFine) {
         hipLaunchKernelGGL((k_correct<T, 2>), dim3(correct_grid(A.n)), dim3(kBlock), 0, s, stop, A.n, A.dPPtr, A.dPCol,
                            A.P, A.dTPtr, A.dTCol, A.Tv, A.Dinv, A.lam, N.x, A.r, A.x, A.d);
     } else {
