@@ -39,8 +39,8 @@ int rows_grid(int n, int rowsPerPass)
 }
 
 // ---------------------------------------------------------------------------- numeric set-up kernels
-template <typename TI, typename T>
-__global__ void __launch_bounds__(kBlock) k_cvt(long n, const TI* __restrict__ in, T* out)
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_cvt(long n, const double* __restrict__ in, T* out)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) out[i] = (T)in[i];
@@ -1686,7 +1686,7 @@ struct Amg<T>::Level : AmgHostLevel {
         *dTCol = nullptr, *dTcPtr = nullptr, *dTcA = nullptr,
         *dTcP = nullptr, *dAcPtr = nullptr, *dAcP = nullptr, *dAcT = nullptr;
     unsigned char* dPIsTent = nullptr;
-    T* vals = nullptr;      // the level's blocks; finest level in double: the caller's (numeric()), not owned
+    T* vals = nullptr;      // the level's blocks; a smoothed finest level in double: the caller's (numeric()), only read
     T* ownVals = nullptr;   // the buffer behind vals where the level has its own
     T *Dinv = nullptr, *Pt = nullptr, *P = nullptr, *R = nullptr, *Tv = nullptr;
     T *b = nullptr, *x = nullptr, *r = nullptr, *d = nullptr;  // right-hand side, iterate, residual, direction
@@ -1860,8 +1860,10 @@ int Amg<T>::setup(hipStream_t s, int nV, const std::vector<int>& rowPtr, const s
         up(pool_, s, A.dRowPtr, A.rowPtr);
         up(pool_, s, A.dColIdx, A.colIdx);
         up(pool_, s, A.dDiagPos, A.diagPos);
-        // the double hierarchy reads the caller's matrix in place (numeric())
-        if (l > 0 || !std::is_same<T, double>::value) dalloc(pool_, A.ownVals, A.colIdx.size() * bs * bs);
+        // the double hierarchy reads the caller's matrix in place (numeric()); not where the finest level is the last
+        // one too, whose zero diagonal entries are replaced (k_blockinv)
+        if (l > 0 || L.size() == 1 || !std::is_same<T, double>::value)
+            dalloc(pool_, A.ownVals, A.colIdx.size() * bs * bs);
         A.vals = A.ownVals;
         dalloc(pool_, A.Dinv, (size_t)A.n * bs * bs);
         dalloc(pool_, A.b, (size_t)A.n * bs);
@@ -1929,30 +1931,22 @@ int Amg<T>::setup(hipStream_t s, int nV, const std::vector<int>& rowPtr, const s
 }
 
 template <typename T>
-void Amg<T>::numeric(hipStream_t s, const void* A0vals, int vals32, const double* UV, int safe)
+void Amg<T>::numeric(hipStream_t s, const double* A0vals, const double* UV, int safe)
 {
     for (size_t l = 0; l < L.size(); ++l) {
         Level& A = *L[l];
         const int bs = A.bs;
         const long nvals = (long)A.colIdx.size() * bs * bs;
         if (l == 0) {
-            if (std::is_same<T, double>::value && !vals32) {
+            if (A.ownVals) {
+                hipLaunchKernelGGL((k_cvt<T>), dim3(grid_for(nvals)), dim3(kBlock), 0, s, nvals, A0vals, A.vals);
+            } else if constexpr (std::is_same<T, double>::value) {
                 // the matrix itself: a copy would be one more pass (14 us at 200k faces), and the PCG's product and
                 // the V-cycle would each bring their own 25 MB into the same 32 MB of L2 (with one matrix the
                 // product falls from 12.2 to 9.7 us, k_cheb_first from 10.3 to 8.8, k_correct from 13.5 to 12.4)
-                T* const a0 = static_cast<T*>(const_cast<void*>(A0vals));
+                T* const a0 = const_cast<T*>(A0vals);
                 if (A.vals != a0) ++generation_;  // captured launches name the old one
                 A.vals = a0;
-            } else {
-                if (!A.ownVals) dalloc(pool_, A.ownVals, A.colIdx.size() * bs * bs);
-                if (A.vals != A.ownVals) ++generation_;
-                A.vals = A.ownVals;
-                if (vals32)
-                    hipLaunchKernelGGL((k_cvt<float, T>), dim3(grid_for(nvals)), dim3(kBlock), 0, s, nvals,
-                                       static_cast<const float*>(A0vals), A.vals);
-                else
-                    hipLaunchKernelGGL((k_cvt<double, T>), dim3(grid_for(nvals)), dim3(kBlock), 0, s, nvals,
-                                       static_cast<const double*>(A0vals), A.vals);
             }
         }
         if (std::is_same<T, float>::value) {  // keep the FP32-stored level positive definite
@@ -2267,7 +2261,7 @@ void Amg<T>::apply(hipStream_t s, const double* r, double* z, double* rzPart, co
     const int g = row_grid(A.n, 2);
     if (L.size() == 1) {
         // single level: the dense inverse is the whole preconditioner
-        hipLaunchKernelGGL((k_cvt<double, T>), dim3(grid_for((long)A.n * 2)), dim3(kBlock), 0, s, (long)A.n * 2, r, A.b);
+        hipLaunchKernelGGL((k_cvt<T>), dim3(grid_for((long)A.n * 2)), dim3(kBlock), 0, s, (long)A.n * 2, r, A.b);
         coarse_solve(s, stop);
         hipLaunchKernelGGL(k_finish_z<T>, dim3(g), dim3(kBlock), 0, s, stop, A.n * 2, A.x, r, z, rzPart);
         return;

@@ -45,7 +45,7 @@ public:
     // safe != 0: smoother interval and prolongator damping from the
     // Gershgorin bound of D^-1 A (guaranteed, slower convergence) instead of
     // the Lanczos estimate.
-    virtual void numeric(hipStream_t s, const void* A0vals, int vals32, const double* UV, int safe = 0) = 0;
+    virtual void numeric(hipStream_t s, const double* A0vals, const double* UV, int safe = 0) = 0;
     virtual int levels() const = 0;
     virtual long level_rows(int l) const = 0;
     virtual long level_blocks(int l) const = 0;
@@ -87,10 +87,10 @@ public:
               const std::vector<unsigned char>* late = nullptr) override;
 
     // Numeric hierarchy from the fine-level block values (same layout as the
-    // pattern; double, or float when vals32; the double hierarchy keeps
-    // reading them in place) and the current UV (for the rigid near-null
-    // space).
-    void numeric(hipStream_t s, const void* A0vals, int vals32, const double* UV, int safe = 0) override;
+    // pattern; a double hierarchy of more than one level keeps reading them
+    // in place and never writes them) and the current UV (for the rigid
+    // near-null space).
+    void numeric(hipStream_t s, const double* A0vals, const double* UV, int safe = 0) override;
 
     // z = M r (one V-cycle) for FP64 vectors of 2*nV; writes per-workgroup
     // partial records of r.z into rzPart (rz_records() of them). Every

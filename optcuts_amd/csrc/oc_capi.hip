@@ -677,14 +677,14 @@ int step_bound(oc_ctx* c, const TriSet& T, const double* dDir, double cap, doubl
 // guaranteed smoother interval).
 void amg_numeric(oc_ctx* c, int safe)
 {
-    const void* vals = c->sys.dVals.p;
+    const double* vals = c->sys.dVals.as<double>();
     if (c->amgOnOld) {
         oc::launch_remap_blocks(c->stream, c->amgPat.nV, c->dAmgOldRowPtr.as<int>(), c->dAmgMap.as<int>(),
                                 c->dAmgDropPtr.as<int>(), c->dAmgDrop.as<int>(), c->dAmgOldDiag.as<int>(),
                                 c->sys.dVals.as<double>(), c->dAmgVals.as<double>());
-        vals = c->dAmgVals.p;
+        vals = c->dAmgVals.as<double>();
     }
-    c->amg->numeric(c->stream, vals, c->sys.vals32, c->dUV.as<double>(), safe);
+    c->amg->numeric(c->stream, vals, c->dUV.as<double>(), safe);
 }
 
 int amg_structure(oc_ctx* c);
@@ -2031,7 +2031,7 @@ int oc_solver_factorize(oc_ctx* c)
             }
             c->solAmgStruct = true;
         }
-        c->amgSol.numeric(c->stream, c->sol.dVals.p, 0, c->dSolUV.as<double>());
+        c->amgSol.numeric(c->stream, c->sol.dVals.as<double>(), c->dSolUV.as<double>());
         OC_HIP(c, hipGetLastError());
     }
     if (c->solPrecond == OC_PRECOND_IC0) {
@@ -2083,7 +2083,7 @@ int oc_solver_solve(oc_ctx* c, const double* rhs, double* x)
         st = run_pcg(c, c->sol, c->dSolB.as<double>(), c->solTol, c->solMaxIter, it, rr, &c->amgSol);
         if (st == OC_ERR_BREAKDOWN) {
             int it2;
-            c->amgSol.numeric(c->stream, c->sol.dVals.p, 0, c->dSolUV.as<double>(), 1);
+            c->amgSol.numeric(c->stream, c->sol.dVals.as<double>(), c->dSolUV.as<double>(), 1);
             OC_HIP(c, hipGetLastError());
             c->solFallback = 1;
             st = run_pcg(c, c->sol, c->dSolB.as<double>(), c->solTol, c->solMaxIter, it2, rr, &c->amgSol);
@@ -2493,7 +2493,7 @@ int oc_tutte(oc_ctx* c, int layout, int precond, double relTol, int maxIter, dou
         // rigid-motion near-null space at the boundary-initialised positions,
         // staged in the solution buffer (the solve starts from zero after it)
         OC_HIP(c, hipMemcpyAsync(c->dX.p, bc.data(), sizeof(double) * bc.size(), hipMemcpyHostToDevice, c->stream));
-        c->amgTut.numeric(c->stream, P.dVals.p, 0, c->dX.as<double>());
+        c->amgTut.numeric(c->stream, P.dVals.as<double>(), c->dX.as<double>());
         pre = &c->amgTut;
     }
     OC_HIP(c, hipGetLastError());
