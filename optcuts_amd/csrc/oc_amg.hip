@@ -1240,10 +1240,12 @@ __global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ st
 // (post-smoothing): x += d + d'; 2 (the finest level's last step): z = x + d +
 // d' in FP64 and partial records of rFinal.z per workgroup. d is read for the
 // neighbours and not written. Launch with row_grid workgroups.
-// Whether the PCG's residual is within its tolerance (then its control record is set as k_pcg_spmv sets it), from the
-// threads' shares of the r.r records: every workgroup sums them itself, in the same order. bb, the right-hand side's norm, is what the first
-// residual's records hold; k_pcg_spmv keeps it from then on.
-__device__ __forceinline__ bool pcg_converged(const PcgStage& st, double (&acc)[1])
+// Whether the PCG is over: its done flag, as this thread found it when the kernel began, or the residual within the
+// tolerance (then its control record is set as k_pcg_spmv sets it), from the threads' shares of the r.r records. Every
+// workgroup sums them itself, in the same order. bb, the right-hand side's norm, is what the first residual's records
+// hold; k_pcg_spmv keeps it from then on. Workgroup 0 sets the flag while other workgroups may not have begun, so their
+// waves can find it differently: it is acted on only behind the barriers, where all of them find the same sum.
+__device__ __forceinline__ bool pcg_over(const PcgStage& st, int done, double (&acc)[1])
 {
     const int it = st.ctrl->itNext;
     const double bbKept = st.ctrl->bb, tol2 = st.ctrl->tol2;
@@ -1252,6 +1254,7 @@ __device__ __forceinline__ bool pcg_converged(const PcgStage& st, double (&acc)[
     if (threadIdx.x == 0) sh = acc[0];
     __syncthreads();
     const double rr = sh, bb = it == 0 ? rr : bbKept;
+    if (done) return true;
     if (bb != 0.0 && !(rr <= tol2 * bb)) return false;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (it == 0) st.ctrl->bb = bb;
@@ -1282,9 +1285,9 @@ __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int*
         rp.begin(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr);
         double rr[1];
         if (CHECK && p == 0) sum_records<1>(st.partRr, st.nRr, st.sRr, rr);
-        if (p == 0 && stopped(stop, rp.kb[0])) return;
+        if (!CHECK && p == 0 && stopped(stop, rp.kb[0])) return;
         rp.blocks(colIdx, vals, lane);
-        if (CHECK && p == 0 && pcg_converged(st, rr)) return;
+        if (CHECK && p == 0 && pcg_over(st, stop, rr)) return;
         rp.gather(d);
         double Dm[UNROLL][BS * BS], dd[UNROLL][BS], xo[UNROLL][BS], rf[UNROLL][BS];
 #pragma unroll

@@ -887,9 +887,10 @@ void launch_ls_commit(hipStream_t s, const LsDecision* dec, long n, const double
 // alone and the caller applies M between update(i) and spmv(i+1), handing
 // its own r.z partial records to spmv; a multigrid's row-local first step is
 // computed where the residual is written (FirstStep).
-// Scalars shared across kernels (rz_i, bb, done) are written by block 0 only,
-// into slots that no other block of the same kernel reads. No atomics and no
-// device-scope fences: kernel boundaries order everything.
+// Scalars shared across kernels (rz_i, bb) are written by block 0 only, into
+// slots whose value no other block of the same kernel uses; done, which it may
+// set as well, is acted on only behind the record sums (PcgCtrl). No atomics
+// and no device-scope fences: kernel boundaries order everything.
 // Rows are split into one contiguous chunk per workgroup, so the neighbour
 // gathers of a chunk stay in the L2 of the XCD that runs it.
 __device__ __forceinline__ double4 to_double4(const double4& v) { return v; }

@@ -8,8 +8,10 @@ namespace oc {
 // The iteration number lives here, not in launch arguments, so that every
 // iteration of one parity launches identical arguments (graph replay):
 // k_pcg_init sets itNext = 0; k_pcg_spmv reads itNext and records it in itCur
-// (and iter); k_pcg_update (or update_apply()) reads itCur and sets itNext = itCur + 1. Each field
-// is written by one kernel and read only by the next.
+// (and iter); k_pcg_update (or update_apply()) reads itCur and sets itNext = itCur + 1. A field is
+// written by workgroup 0 alone and read by later kernels; only done is read in the launch that may set it
+// (k_pcg_spmv, k_pcg_update, update_apply(), a multigrid's first kernel): there each thread reads it first and acts on
+// it behind the record sums, from which every workgroup takes the same decision as the one that set it.
 struct PcgCtrl {
     double bb, tol2, rr, pad0;
     double rzSlot[2];
