@@ -63,6 +63,7 @@ struct DevBuf {
 struct BlockPattern : oc::HostPattern {
     DevBuf dRowPtr, dColIdx, dDiagPos, dVals, dMinv;
     int vals32 = 0;  // dVals holds float blocks (room for double blocks is always allocated)
+    bool pcgSmall = false;  // Jacobi-PCG runs in one workgroup (pcg_small_fits)
 };
 
 }  // namespace
@@ -403,6 +404,7 @@ int upload_pattern(oc_ctx* c, BlockPattern& P)
     if (upload(c, P.dDiagPos, P.diagPos)) return OC_ERR_HIP;
     OC_HIP(c, P.dVals.ensure(sizeof(double) * 4 * (size_t)std::max<long>(1, P.nnzb())));
     OC_HIP(c, P.dMinv.ensure(sizeof(double) * 4 * (size_t)std::max(1, P.nV)));
+    P.pcgSmall = oc::pcg_small_fits(P.nV, P.rowPtr.data());
     return OC_OK;
 }
 
@@ -455,8 +457,9 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
         }
         return OC_OK;
     };
-    if (!amg && nV <= oc::kPcgSmallRows) {
-        constexpr int kSpan = 1024;  // iterations per launch, which bounds its length (2.5-6 ms)
+    if (!amg && P.pcgSmall) {
+        // iterations per launch, which bounds its length: 2.5-6 ms with rows of at most 8 blocks, 13 at the rule's limit
+        constexpr int kSpan = 1024;
         for (int it = 0; !h.done; it += kSpan) {
             oc::launch_pcg_small(c->stream, nV, P.dRowPtr.as<int>(), P.dColIdx.as<int>(), V, V32, b,
                                  P.dMinv.as<double>(), c->dX.as<double>(), c->dR.as<double>(), c->dP0.as<double>(),

@@ -1240,7 +1240,8 @@ void launch_pcg_update(hipStream_t s, int nV, const double* pNew, const double* 
 // (2.5 us: 128 registers are the limit of 16 waves, and it spills). A thread owns rows t, t + 1024, ...: its
 // first row's blocks stay in registers for the whole solve (kPcgSmallSlots of them; 64 registers in double), the second
 // row's come from the slot-major copy of k_pcg_small_pack (coalesced, from the L2 that one CU reads at 64 B a clock)
-// and p and x are in LDS. Blocks past kPcgSmallSlots of a row (a vertex of more than 7 neighbours) are read in place.
+// and p and x are in LDS. Blocks past kPcgSmallSlots of a row (a vertex of more than 7 neighbours) are read in place, one
+// after another, which pcg_small_fits bounds.
 // Iterations [it0, itEnd) of the same rule as k_pcg_spmv + k_pcg_update, state in x, r, p and ctrl between launches.
 constexpr int kPcgSmallThreads = 1024, kPcgSmallSlots = 8;
 
@@ -1431,6 +1432,18 @@ __global__ void __launch_bounds__(kPcgSmallThreads) k_pcg_small(int nV, const in
         ctrl->iter = it;
         ctrl->done = done;
     }
+}
+
+bool pcg_small_fits(int nV, const int* rowPtr)
+{
+    if (nV > kPcgSmallRows) return false;
+    long longest = 0, over = 0;
+    for (int v = 0; v < nV; ++v) {
+        const long len = rowPtr[v + 1] - rowPtr[v];
+        longest = std::max(longest, len);
+        over += std::max(0L, len - kPcgSmallSlots);
+    }
+    return longest * kPcgSmallOver + over * kPcgSmallLongest <= (long)kPcgSmallLongest * kPcgSmallOver;
 }
 
 size_t pcg_small_bytes(int nV)

@@ -160,6 +160,14 @@ void launch_pcg_update(hipStream_t s, int nV, const double* pNew, const double* 
 // 1.19 ms at 100 rows, 1.40 and 4.8 at 1,024, 4.7 and 7.4 at 2,025; with four rows a thread 15.6 and 10.6 at 3,844,
 // hence the limit of two.
 constexpr int kPcgSmallRows = 2048;
+// Whether it is the faster form for a pattern (host row pointers). One thread walks a row's blocks past the eighth, 0.11
+// us each, and one CU reads all of them: us an iteration by it and by two launches, with one long row of 50, 66, 98 and
+// 258 blocks at 1,024 rows 6.3 and 10.4, 8.0 and 11.6, 11.4 and 14.7, 29 and 26, at 2,048 rows 9.5 and 10.9, 11.4 and
+// 12.3, 15.4 and 14.7, 34 and 28; with every row of 9, 13, 17 and 65 blocks (1, 5, 9, 57 such blocks a row) at 1,024
+// rows 2.8 and 8.1, 5.6 and 8.4, 8.1 and 8.7, 51 and 11, at 2,048 rows 6.9 and 8.0, 12.5 and 8.3, 18 and 8.6, 254 and
+// 12. Hence the limits of 64 blocks for the longest row and 4,096 blocks past the eighth, shared where both occur.
+constexpr int kPcgSmallLongest = 64, kPcgSmallOver = 4096;
+bool pcg_small_fits(int nV, const int* rowPtr);
 size_t pcg_small_bytes(int nV);
 void launch_pcg_small(hipStream_t s, int nV, const int* rowPtr, const int* colIdx, const void* vals, int vals32,
                       const double* b, const double* Minv, double* x, double* r, double* p, void* work, int it0,
