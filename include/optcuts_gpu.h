@@ -296,6 +296,8 @@ int oc_newton_rebuild(oc_ctx* ctx, double* E);
  * set of buffers) or launched kernel by kernel (0). The results are identical either way. No reference
  * counterpart. */
 int oc_pcg_graphs(oc_ctx* ctx, int enable);
+/* Graphs captured so far for PCG iterations on this context. No reference counterpart (diagnostics and tests). */
+int oc_pcg_graph_builds(oc_ctx* ctx, long long* n);
 /* Selects OC_PRECISION_FP64 (default) or OC_PRECISION_MIXED for the next oc_newton_init. No reference
  * counterpart (the reference is FP64 throughout). */
 int oc_newton_set_precision(oc_ctx* ctx, int precision);

@@ -76,6 +76,7 @@ _SIGS = {
     "oc_check_inversion": (C.c_int, [_ctx, C.POINTER(C.c_int)]),
     "oc_div_grad_per_vert": (C.c_int, [_ctx, _dp]),
     "oc_pcg_graphs": (C.c_int, [_ctx, C.c_int]),
+    "oc_pcg_graph_builds": (C.c_int, [_ctx, C.POINTER(C.c_longlong)]),
     "oc_seam_sparsity": (C.c_int, [_ctx, C.c_int, _ip, C.c_double, C.c_int, C.POINTER(C.c_double)]),
     "oc_split_candidates": (C.c_int, [_ctx, C.c_int, C.c_double, _vp, C.c_int, _ip, C.POINTER(C.c_int),
                                       C.POINTER(C.c_int)]),
@@ -326,6 +327,12 @@ class Context:
     def pcg_graphs(self, enable):
         """PCG iterations from captured HIP graphs (True, the default) or launched one by one."""
         self._chk(self.L.oc_pcg_graphs(self.h, int(bool(enable))))
+
+    def pcg_graph_builds(self):
+        """Graphs captured so far for PCG iterations on this context."""
+        n = C.c_longlong()
+        self._chk(self.L.oc_pcg_graph_builds(self.h, C.byref(n)))
+        return n.value
 
     def div_grad_per_vert(self):
         """SymDirichletEnergy::computeDivGradPerVert at the current UV: (nV,)."""

@@ -1947,9 +1947,9 @@ void Amg<T>::numeric(hipStream_t s, const double* A0vals, const double* UV, int 
                 // the matrix itself: a copy would be one more pass (14 us at 200k faces), and the PCG's product and
                 // the V-cycle would each bring their own 25 MB into the same 32 MB of L2 (with one matrix the
                 // product falls from 12.2 to 9.7 us, k_cheb_first from 10.3 to 8.8, k_correct from 13.5 to 12.4)
-                T* const a0 = const_cast<T*>(A0vals);
-                if (A.vals != a0) ++generation_;  // captured launches name the old one
-                A.vals = a0;
+                A.vals = const_cast<T*>(A0vals);
+                if (namedVals_ != A0vals) ++generation_;  // captured launches name the old one
+                namedVals_ = A0vals;
             }
         }
         if (std::is_same<T, float>::value) {  // keep the FP32-stored level positive definite

@@ -135,6 +135,7 @@ private:
     // structure build writes into it instead of fresh allocations.
     std::vector<AmgHostLevel> spare_;
     bool ready_ = false;
+    const void* namedVals_ = nullptr;  // the caller's matrix that launches since the last generation change name
     int tailMax_ = -1, tailPending_ = -1;  // set_tail_max (-1: the built-in limit), active since the last setup()
     void release();
     void vcycle(hipStream_t s, int l, const int* stop);

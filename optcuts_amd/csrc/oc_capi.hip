@@ -212,6 +212,7 @@ struct oc_ctx {
     bool pcgGraphs = true;
     std::vector<uintptr_t> pcgSig;
     hipGraphExec_t pcgG[4] = {nullptr, nullptr, nullptr, nullptr};
+    long long pcgGraphBuilds = 0;
     void clear_pcg_graphs()
     {
         for (auto& g : pcgG)
@@ -546,6 +547,7 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
         (void)hipGraphDestroy(g);
         if (e != hipSuccess) return nullptr;
         c->pcgG[kind] = ex;
+        ++c->pcgGraphBuilds;
         return ex;
     };
     // Queues iterations [it, it + n): replayed graphs, or launches one by one
@@ -1465,6 +1467,14 @@ int oc_pcg_graphs(oc_ctx* c, int enable)
     OC_HIP(c, hipStreamSynchronize(c->stream));
     c->clear_pcg_graphs();
     c->pcgGraphs = enable != 0;
+    return OC_OK;
+}
+
+int oc_pcg_graph_builds(oc_ctx* c, long long* n)
+{
+    if (!c) return OC_ERR_ARG;
+    OC_ARG(c, n, "oc_pcg_graph_builds: no result pointer");
+    *n = c->pcgGraphBuilds;
     return OC_OK;
 }
 
