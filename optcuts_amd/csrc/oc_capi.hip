@@ -414,7 +414,6 @@ int ensure_pcg(oc_ctx* c, int nV)
     const size_t b = sizeof(double) * 2 * (size_t)std::max(1, nV);
     OC_HIP(c, c->dX.ensure(b));
     OC_HIP(c, c->dR.ensure(b));
-    OC_HIP(c, c->dR1.ensure(b));
     OC_HIP(c, c->dZ.ensure(b));
     OC_HIP(c, c->dP0.ensure(b));
     OC_HIP(c, c->dP1.ensure(b));
@@ -809,6 +808,7 @@ int build_system(oc_ctx* c, bool airOnly = false)
             return OC_ERR_HIP;
         }
         c->learned->rowPtr.clear();  // the network's pattern now belongs to this context
+        OC_HIP(c, c->dR1.ensure(sizeof(double) * 2 * (size_t)std::max(1, nVt)));  // its update alternates residuals
         if (c->learned->net.rz_records() > kRzRecords) {
             c->err = "learned preconditioner: too many partial records";
             return OC_ERR_STATE;
