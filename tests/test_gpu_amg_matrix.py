@@ -1,6 +1,6 @@
 """The multigrid only reads the matrix it is handed: a zero diagonal entry (a vertex that no triangle or triplet
 touches) is replaced in the hierarchy and not in the matrix that PCG and oc_solver_multiply use, on hierarchies of one
-level (the coarsest solve alone: a dense inverse, or diagonal blocks where every vertex is isolated).
+level (the coarsest solve alone: a dense inverse, or diagonal blocks where every vertex is isolated) and of more.
 
 Products: each row adds at most 5 blocks, rounded 10 times: 2^-49 of the sum of magnitudes; bitwise the same before and
 after the set-up. Solutions: condition at most 2 x 8 / 0.1 (Gershgorin and the diagonal excess), so a residual of 1e-12
@@ -45,7 +45,7 @@ def _grid_laplacian(m, isolated, seed):
     return n, ptr, nbr, I, J, V, (U + U.T - sp.diags(U.diagonal())).tocsr(), diag
 
 
-@pytest.mark.parametrize("m,isolated", [(3, 1), (1, 100)])
+@pytest.mark.parametrize("m,isolated", [(3, 1), (1, 100), (20, 7)])
 def test_factorize_leaves_the_matrix_as_it_was(m, isolated):
     n, ptr, nbr, I, J, V, A, diag = _grid_laplacian(m, isolated, m)
     rng = np.random.default_rng(1)
