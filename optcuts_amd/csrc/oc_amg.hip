@@ -348,7 +348,7 @@ struct RowPass {
 #pragma unroll
                 for (int q = 0; q < BS; ++q) y[i] += (Y)ak[i * BS + q] * gk[q];
         }
-    group_sum<LANES, BS>(y);
+        group_sum<LANES, BS>(y);
     }
 };
 
@@ -493,7 +493,7 @@ __global__ void __launch_bounds__(kBlock) k_lanczos(int j, int nsteps, int n, co
 #pragma unroll
                     for (int q = 0; q < BS; ++q) y[i] += ak[i * BS + q] * gk[q];
             }
-    group_sum<LANES, BS>(y);
+            group_sum<LANES, BS>(y);
             if (lane == 0 && u[r] < r1) {  // y = (A W_{j-1})_u
                 double m[BS][BS], mi[BS][BS];
 #pragma unroll
@@ -1235,11 +1235,6 @@ __global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ st
     }
 }
 
-// Second Chebyshev step, d the first step's direction: r = theta d - D^-1 A d,
-// d' = rho1 rho0 d + 2 rho1/delta r; KIND 0 (pre-smoothing): x = d + d'; 1
-// (post-smoothing): x += d + d'; 2 (the finest level's last step): z = x + d +
-// d' in FP64 and partial records of rFinal.z per workgroup. d is read for the
-// neighbours and not written. Launch with row_grid workgroups.
 // Whether the PCG is over: its done flag, as this thread found it when the kernel began, or the residual within the
 // tolerance (then its control record is set as k_pcg_spmv sets it), from the threads' shares of the r.r records. Every
 // workgroup sums them itself, in the same order. bb, the right-hand side's norm, is what the first residual's records
@@ -1265,6 +1260,11 @@ __device__ __forceinline__ bool pcg_over(const PcgStage& st, int done, double (&
     return true;
 }
 
+// Second Chebyshev step, d the first step's direction: r = theta d - D^-1 A d,
+// d' = rho1 rho0 d + 2 rho1/delta r; KIND 0 (pre-smoothing): x = d + d'; 1
+// (post-smoothing): x += d + d'; 2 (the finest level's last step): z = x + d +
+// d' in FP64 and partial records of rFinal.z per workgroup. d is read for the
+// neighbours and not written. Launch with row_grid workgroups.
 template <typename T, int BS, int KIND, bool CHECK = false, int NT = kBlock>
 __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int* __restrict__ rowPtr,
                                                const int* __restrict__ colIdx, const T* __restrict__ vals,
@@ -1476,7 +1476,7 @@ __device__ __forceinline__ void restrict_rows(int blk, int G, int nc, const int*
 #pragma unroll
                 for (int i = 0; i < NS; ++i) s[i] += (double)p[l * NS + i] * (double)ru[l];
         }
-    group_sum<LN, NS>(s);
+        group_sum<LN, NS>(s);
         if (lane == 0) {
             T bt[NS];
 #pragma unroll
@@ -1549,11 +1549,18 @@ __global__ void __launch_bounds__(kBlock) k_prolong(const int* __restrict__ stop
 // coarse levels fewer bytes (6 blocks a row in T against 13 in A; 1M faces, level 1: 21.3 -> 15.0 us, 200k faces
 // 8.8 -> 5.4). On the finest level T is as large as A (273 against 256 bytes a row) and evicts it from the caches
 // between the smoothing steps that do read A, so only the saved launch counts there: up to kCorrectMaxFine rows.
-// Whole Newton step, this pass against prolongation + product: 25k rows 1546 / 1565 us, 51k 2020 / 2043, 100k 2988 /
-// 3016, 203k 4953 / 4809, 501k 9084 / 8977. kCorrectLanes lanes per fine row.
-// FP32 storage keeps the product from the corrected x on the finest level: the residual formed here does not see the
-// rounding of the stored x, which the post-smoothing then leaves in z (joint-mode run on 200k faces in the mixed form:
-// one safe-interval retry and three Jacobi solves in 58 steps, against none and one in 51).
+// Whole Newton step, this pass against prolongation + product: 5k rows 909 / 933 us, 25k 1309 / 1308, 51k 1718 / 1736,
+// 76k 2003 / 1996, 100k 2454 / 2450, 116k 2567 / 2537, 130k 2548 / 2549, 152k 3240 / 3263, 176k 3673 / 3626, 203k 4124 /
+// 4003, 303k 5892 / 5743, 501k 8030 / 7845: worth it on small levels, no difference from 25k to 152k rows (the runs of
+// one side differ by 1%), a loss beyond. kCorrectLanes lanes per fine row.
+// The residual formed here does not see the rounding of the x stored beside it; in FP32 storage the post-smoothing
+// leaves that rounding in x, so there the finest level, whose x is z, forms its residual from the stored x. On the
+// coarse levels the next finer level's smoothing sees it as any other error of the correction, and no precision is
+// lost: against the FP64 V-cycle, one V-cycle's relative error in the A-norm is the same to three digits whether they
+// take this pass or the product (2e-3 to 2e-2, the FP32 matrix's own, on discs and spheres of 2.5k to 100k rows), and so
+// are the PCG iterations to 1e-3 and 1e-8. Three fused tori (200k faces, joint mode, mixed form), 100 runs from
+// maps moved by two units in the last place: Jacobi solves a run 0.78 as it is, 0.88 with the product on every level, 0.85
+// with this pass on every level (each +-0.1), steps 52.6, 52.8 and 52.2 (+-0.4).
 constexpr int kCorrectLanes = 8;
 constexpr int kCorrectMaxFine = 131072;
 template <typename T, int BS, int NT = kBlock>

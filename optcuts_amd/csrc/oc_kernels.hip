@@ -629,7 +629,7 @@ void launch_step_bound(hipStream_t s, const TriSet& T, const double* UV, const d
 // The candidates' energies of one 256-triangle tile into Es[k][thread] and the inversion counts added to
 // cnt[k][wave]. A kernel with all candidates' code and reductions unrolled is 27-38 KB of straight-line code, and
 // fetching it took most of its time (k_linesearch 37 us, its finisher 28 us at 200k faces); the candidates are a
-// loop, and their sums go through LDS so that each wave reduces whole candidates (lsWaveSums).
+// loop, and their sums go through LDS so that each wave reduces whole candidates (kLsPerWave).
 template <typename EP>
 __device__ __forceinline__ void ls_tile(const TriSet& T, const double2* __restrict__ UV,
                                         const double2* __restrict__ dir, int t, bool on, bool isMesh, double alpha,
