@@ -45,67 +45,119 @@ __device__ __forceinline__ float read_lane(float x, int i)
 }
 
 // x of another lane of the same 16-lane row, chosen by a DPP control: a move inside the vector unit (30 clocks with
-// the FP64 addition that follows, against 90 for a shuffle through LDS).
-template <int CTRL>
-__device__ __forceinline__ float lane_swap(float x)
+// the FP64 addition that follows, against 90 for a shuffle through LDS). BANKS: the groups of four lanes that take it,
+// the others keep `old`.
+template <int CTRL, int BANKS>
+__device__ __forceinline__ float lane_move(float old, float x)
 {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), CTRL, 0xf, BANKS, true));
 }
-template <int CTRL>
-__device__ __forceinline__ double lane_swap(double x)
+template <int CTRL, int BANKS>
+__device__ __forceinline__ double lane_move(double old, double x)
 {
-    const long long b = __double_as_longlong(x);
-    const unsigned int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
-    const unsigned int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    const long long o = __double_as_longlong(old), b = __double_as_longlong(x);
+    const unsigned int lo = __builtin_amdgcn_update_dpp((int)o, (int)b, CTRL, 0xf, BANKS, true);
+    const unsigned int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(b >> 32), CTRL, 0xf, BANKS, true);
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
-template <int CTRL>
-__device__ __forceinline__ CSum lane_swap(CSum x)
+template <int CTRL, int BANKS>
+__device__ __forceinline__ CSum lane_move(CSum old, CSum x)
 {
-    return CSum{lane_swap<CTRL>(x.s), lane_swap<CTRL>(x.c)};
+    return CSum{lane_move<CTRL, BANKS>(old.s, x.s), lane_move<CTRL, BANKS>(old.c, x.c)};
 }
-__device__ __forceinline__ CSum read_lane(CSum x, int i) { return CSum{read_lane(x.s, i), read_lane(x.c, i)}; }
 
-// All-reduce of a commutative operation over aligned groups of LANES (up to 16) lanes; every lane of the group takes
-// part and ends with the same value: lanes 1 apart, 2 apart (quad permutes), then the mirror images within 8 and 16
-// lanes, whose partners hold the other half's value.
-template <int LANES, typename X, typename Op>
-__device__ __forceinline__ X row_reduce(X x, Op op)
+// x of the lane whose number differs in bit OFF (1, 2, 4 or 8). PERIODIC (OFF 4): x repeats every eight lanes of a
+// row, where a rotation does it in one move.
+template <int OFF, bool PERIODIC, typename X>
+__device__ __forceinline__ X lane_xor(X x)
 {
-    static_assert(LANES >= 1 && LANES <= 16, "within a row of 16 lanes");
-    if (LANES >= 2) x = op(x, lane_swap<0xB1>(x));
-    if (LANES >= 4) x = op(x, lane_swap<0x4E>(x));
-    if (LANES >= 8) x = op(x, lane_swap<0x141>(x));
-    if (LANES >= 16) x = op(x, lane_swap<0x140>(x));
-    return x;
+    static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8, "within a row of 16 lanes");
+    if constexpr (OFF == 1) return lane_move<0xB1, 0xf>(x, x);            // quad permute 1, 0, 3, 2
+    else if constexpr (OFF == 2) return lane_move<0x4E, 0xf>(x, x);       // quad permute 2, 3, 0, 1
+    else if constexpr (OFF == 8) return lane_move<0x128, 0xf>(x, x);      // rotation by 8
+    else if constexpr (PERIODIC) return lane_move<0x124, 0xf>(x, x);      // rotation by 4
+    else return lane_move<0x114, 0xA>(lane_move<0x104, 0x5>(x, x), x);    // shifts by 4, each for half of the quads
 }
-// The same over a whole wave (every lane active): the four rows' values are read as scalars.
-template <typename X, typename Op>
-__device__ __forceinline__ X wave_reduce(X x, Op op)
+
+// x of the lane 16 or 32 apart, as a pair {the even rows', the odd rows'} (or lower, upper half's) value, the same for
+// both lanes of the pair.
+template <int OFF>
+__device__ __forceinline__ void half_pair(unsigned int x, unsigned int& a, unsigned int& b)
 {
-    x = row_reduce<16>(x, op);
-    return op(op(read_lane(x, 0), read_lane(x, 16)), op(read_lane(x, 32), read_lane(x, 48)));
+    if constexpr (OFF == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        a = r[0], b = r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        a = r[0], b = r[1];
+    }
+}
+template <int OFF>
+__device__ __forceinline__ void half_pair(float x, float& a, float& b)
+{
+    unsigned int u, v;
+    half_pair<OFF>((unsigned int)__float_as_int(x), u, v);
+    a = __int_as_float((int)u), b = __int_as_float((int)v);
+}
+template <int OFF>
+__device__ __forceinline__ void half_pair(double x, double& a, double& b)
+{
+    const unsigned long long q = (unsigned long long)__double_as_longlong(x);
+    unsigned int al, bl, ah, bh;
+    half_pair<OFF>((unsigned int)q, al, bl);
+    half_pair<OFF>((unsigned int)(q >> 32), ah, bh);
+    a = __longlong_as_double((long long)(((unsigned long long)ah << 32) | al));
+    b = __longlong_as_double((long long)(((unsigned long long)bh << 32) | bl));
+}
+template <int OFF>
+__device__ __forceinline__ void half_pair(CSum x, CSum& a, CSum& b)
+{
+    half_pair<OFF>(x.s, a.s, b.s);
+    half_pair<OFF>(x.c, a.c, b.c);
+}
+
+// All-reduce of a commutative operation over aligned groups of LANES lanes (a power of two); every lane of the group
+// takes part and ends with the same value: the butterfly that starts with the lanes LANES / 2 apart and ends with
+// neighbours, so that the order of a sum is that of the same loop over __shfl_xor.
+template <int LANES, typename X, typename Op>
+__device__ __forceinline__ X group_reduce(X x, Op op)
+{
+    static_assert(LANES >= 1 && LANES <= 64 && (LANES & (LANES - 1)) == 0, "a part of a wave");
+    X a, b;
+    if constexpr (LANES >= 64) {
+        half_pair<32>(x, a, b);
+        x = op(a, b);
+    }
+    if constexpr (LANES >= 32) {
+        half_pair<16>(x, a, b);
+        x = op(a, b);
+    }
+    if constexpr (LANES >= 16) x = op(x, lane_xor<8, false>(x));
+    if constexpr (LANES >= 8) x = op(x, lane_xor<4, (LANES >= 16)>(x));
+    if constexpr (LANES >= 4) x = op(x, lane_xor<2, false>(x));
+    if constexpr (LANES >= 2) x = op(x, lane_xor<1, false>(x));
+    return x;
 }
 
 __device__ __forceinline__ CSum wave_csum(CSum v)
 {
-    return wave_reduce(v, [](CSum a, CSum b) { return csum_add(a, b); });
+    return group_reduce<kWave>(v, [](CSum a, CSum b) { return csum_add(a, b); });
 }
 __device__ __forceinline__ double wave_sum(double v)
 {
-    return wave_reduce(v, [](double a, double b) { return a + b; });
+    return group_reduce<kWave>(v, [](double a, double b) { return a + b; });
 }
 __device__ __forceinline__ float wave_sumf(float v)
 {
-    return wave_reduce(v, [](float a, float b) { return a + b; });
+    return group_reduce<kWave>(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ double wave_max(double v)
 {
-    return wave_reduce(v, [](double a, double b) { return fmax(a, b); });
+    return group_reduce<kWave>(v, [](double a, double b) { return fmax(a, b); });
 }
 __device__ __forceinline__ double wave_min(double v)
 {
-    return wave_reduce(v, [](double a, double b) { return fmin(a, b); });
+    return group_reduce<kWave>(v, [](double a, double b) { return fmin(a, b); });
 }
 
 // Sums over aligned groups of LANES lanes, in every lane of the group (all of them active).
@@ -113,11 +165,7 @@ template <int LANES, int NV>
 __device__ __forceinline__ void group_sum(double (&v)[NV])
 {
 #pragma unroll
-    for (int i = 0; i < NV; ++i) v[i] = row_reduce<(LANES < 16 ? LANES : 16)>(v[i], [](double a, double b) { return a + b; });
-#pragma unroll
-    for (int off = 16; off < LANES; off <<= 1)
-#pragma unroll
-        for (int i = 0; i < NV; ++i) v[i] += __shfl_xor(v[i], off, LANES);
+    for (int i = 0; i < NV; ++i) v[i] = group_reduce<LANES>(v[i], [](double a, double b) { return a + b; });
 }
 
 // This thread's share of the sum of n records' NV values (value k of record b at part[b * stride + k]), for workgroups
@@ -189,16 +237,19 @@ __device__ __forceinline__ void block_sum(double (&v)[NV])
     __syncthreads();
 }
 
-// Workgroup sums of every thread's values, identical in every thread of every workgroup that sums the same values.
+// Sums of the first kBlock threads' values, in every thread of the workgroup and identical in every workgroup that sums
+// the same values.
 template <int NV>
 __device__ __forceinline__ void all_sum(double (&acc)[NV])
 {
     __shared__ double sh[kBlock / kWave][NV];
+    if (threadIdx.x < kBlock) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) acc[k] = wave_sum(acc[k]);
-    if (threadIdx.x % kWave == 0)
+        for (int k = 0; k < NV; ++k) acc[k] = wave_sum(acc[k]);
+        if (threadIdx.x % kWave == 0)
 #pragma unroll
-        for (int k = 0; k < NV; ++k) sh[threadIdx.x / kWave][k] = acc[k];
+            for (int k = 0; k < NV; ++k) sh[threadIdx.x / kWave][k] = acc[k];
+    }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NV; ++k) {

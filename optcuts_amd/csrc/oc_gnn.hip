@@ -358,11 +358,11 @@ __global__ void __launch_bounds__(kBlock) k_gnn_heads_node(int nV, const float* 
 // ---------------------------------------------------------------------------- factor products (FP64 arithmetic)
 __device__ __forceinline__ double2 bmv(float4 B, double2 v)
 {
-    return make_double2((double)B.x * v.x + (double)B.y * v.y, (double)B.z * v.x + (double)B.w * v.y);
+    return make_double2(fma((double)B.x, v.x, (double)B.y * v.y), fma((double)B.z, v.x, (double)B.w * v.y));
 }
 __device__ __forceinline__ double2 bmtv(float4 B, double2 v)
 {
-    return make_double2((double)B.x * v.x + (double)B.z * v.y, (double)B.y * v.x + (double)B.w * v.y);
+    return make_double2(fma((double)B.x, v.x, (double)B.z * v.y), fma((double)B.y, v.x, (double)B.w * v.y));
 }
 
 __device__ __forceinline__ unsigned int probe_hash(unsigned int i, unsigned int seed, unsigned int j)
@@ -381,44 +381,31 @@ __device__ __forceinline__ double2 probe(int u, unsigned int seed, unsigned int 
                         (probe_hash(2u * u + 1u, seed, j) & 1u) ? 1.0 : -1.0);
 }
 
-// The factor products: kRowLanes lanes per row with kRowEdges edges each in flight, the rest in a loop (a thread per
-// row walked its 6 edges one after another with a wave per SIMD of 99 CUs at 50k faces: G 4.7 us, G^T 6.2 us). With
-// k_gnn_update_G (5.6 us, G^T 4.6) a learned Newton step took 8.3 -> 7.1 ms at 50k faces and 21.4 -> 17.5 at 79k; four lanes of two
-// edges 6.9 and 19.7, eight of one 8.0 and 21.7 (more passes of the at most kGnnMaxGrid workgroups, each on a
-// contiguous chunk of rows).
-constexpr int kRowLanes = 2, kRowEdges = 4;
-int row_blocks(int nV) { return blocks_for((long)nV * kRowLanes, kBlock); }
+// The factor products: one row per thread, its edges into lower (G) or upper (G^T) neighbours (rowM: where the upper ones
+// begin) in batches of kRowEdges whose loads are in flight together, their terms added in edge order and with the
+// products' rounding written out (the PCG's path depends on both, see k_pcg_spmv). Learned Newton step, one edge after
+// another with G and the update in launches of their own / two lanes a row over all its edges / this: 10.0 / 6.9 / 6.5
+// ms at 50k faces, 7.5 / 5.5 / 5.0 at 79k, 33.4 / 27.4 / 25.4 at 200k.
+constexpr int kRowEdges = 4;
 
-// Sum over row u's edges into lower (LOWER: w < u) or upper neighbours, in every lane of the row: body(e, w) gives the
-// edge's term.
-template <bool LOWER, typename Body>
-__device__ __forceinline__ double2 edge_sum(const int* __restrict__ ew, int u, int e0, int e1, int lane,
-                                            const Body& body)
+// o += the terms body(e, w) of the edges [e0, e1), in order
+template <typename Body>
+__device__ __forceinline__ void add_edges(const int* __restrict__ ew, int e0, int e1, const Body& body, double2& o)
 {
-    double y[2] = {0.0, 0.0};
-    int w[kRowEdges];
+    for (int e = e0; e < e1; e += kRowEdges) {
+        int w[kRowEdges];
+        double2 t[kRowEdges];
 #pragma unroll
-    for (int k = 0; k < kRowEdges; ++k) {
-        const int e = e0 + lane + k * kRowLanes;
-        w[k] = e < e1 ? ew[e] : u;
-    }
+        for (int k = 0; k < kRowEdges; ++k) w[k] = ew[min(e + k, e1 - 1)];
 #pragma unroll
-    for (int k = 0; k < kRowEdges; ++k)
-        if (LOWER ? w[k] < u : w[k] > u) {
-            const double2 t = body(e0 + lane + k * kRowLanes, w[k]);
-            y[0] += t.x;
-            y[1] += t.y;
-        }
-    for (int e = e0 + lane + kRowEdges * kRowLanes; e < e1; e += kRowLanes) {
-        const int v = ew[e];
-        if (LOWER ? v < u : v > u) {
-            const double2 t = body(e, v);
-            y[0] += t.x;
-            y[1] += t.y;
-        }
+        for (int k = 0; k < kRowEdges; ++k) t[k] = body(min(e + k, e1 - 1), w[k]);
+#pragma unroll
+        for (int k = 0; k < kRowEdges; ++k)
+            if (e + k < e1) {
+                o.x += t[k].x;
+                o.y += t[k].y;
+            }
     }
-    group_sum<kRowLanes, 2>(y);
-    return make_double2(y[0], y[1]);
 }
 
 enum { kApplyPrecond = 0, kApplyLoss = 1 };
@@ -426,6 +413,7 @@ enum { kApplyPrecond = 0, kApplyLoss = 1 };
 // out = G^ s, s_x = C^-1 in_x (precond) or in_x (loss: then out = 2 norm (G^ t - w), loss records)
 template <int MODE>
 __global__ void __launch_bounds__(kBlock) k_gnn_apply_G(int nV, const int* __restrict__ rowE,
+                                                        const int* __restrict__ rowM,
                                                         const int* __restrict__ ew, const float4* __restrict__ Cinv,
                                                         const float4* __restrict__ Go, const float4* __restrict__ Gd,
                                                         const double2* __restrict__ in, double2* out, double norm,
@@ -435,28 +423,25 @@ __global__ void __launch_bounds__(kBlock) k_gnn_apply_G(int nV, const int* __res
     if (stop && *stop) return;
     long r0, r1;
     chunk(nV, r0, r1);
-    const int sub = threadIdx.x / kRowLanes, lane = threadIdx.x % kRowLanes;
     double acc[1] = {0.0};
-    for (int u = (int)r0 + sub; u < r1; u += kBlock / kRowLanes) {
+    for (int u = (int)r0 + threadIdx.x; u < r1; u += kBlock) {
         double2 su = in[u];
         if (MODE == kApplyPrecond) su = bmv(Cinv[u], su);
         double2 o = bmv(Gd[u], su);
-        const double2 t = edge_sum<true>(ew, u, rowE[u], rowE[u + 1], lane, [&](int e, int w) {
+        add_edges(ew, rowE[u], rowM[u], [&](int e, int w) {
             double2 sw = in[w];
             if (MODE == kApplyPrecond) sw = bmv(Cinv[w], sw);
             return bmv(Go[e], sw);
-        });
-        o.x += t.x;
-        o.y += t.y;
+        }, o);
         if (MODE == kApplyLoss) {
             const double2 wv = probe(u, seed, pj);
             o.x -= wv.x;
             o.y -= wv.y;
-            if (lane == 0) acc[0] += o.x * o.x + o.y * o.y;
+            acc[0] += o.x * o.x + o.y * o.y;
             o.x *= 2.0 * norm;
             o.y *= 2.0 * norm;
         }
-        if (lane == 0) out[u] = o;
+        out[u] = o;
     }
     if (MODE == kApplyLoss) {
         block_sum<1>(acc);
@@ -467,6 +452,7 @@ __global__ void __launch_bounds__(kBlock) k_gnn_apply_G(int nV, const int* __res
 // A PCG update with the product by G^ on the new residual in the same launch (a launch less of four an iteration): a
 // gathered residual is formed as r_w - alpha q_w again, so the new one goes to another buffer.
 __global__ void __launch_bounds__(kBlock) k_gnn_update_G(int nV, const int* __restrict__ rowE,
+                                                         const int* __restrict__ rowM,
                                                          const int* __restrict__ ew, const float4* __restrict__ Cinv,
                                                          const float4* __restrict__ Go, const float4* __restrict__ Gd,
                                                          const double2* __restrict__ p, const double2* __restrict__ q,
@@ -478,7 +464,6 @@ __global__ void __launch_bounds__(kBlock) k_gnn_update_G(int nV, const int* __re
     const double rzCur = ctrl->rzSlot[it & 1];
     long r0, r1;
     chunk(nV, r0, r1);
-    const int sub = threadIdx.x / kRowLanes, lane = threadIdx.x % kRowLanes;
     double pq[1];
     sum_records<1>(partS, nPartS, 1, pq);
     all_sum<1>(pq);
@@ -493,25 +478,23 @@ __global__ void __launch_bounds__(kBlock) k_gnn_update_G(int nV, const int* __re
     const auto residual = [&](int w) {
         double2 r = rOld[w];
         const double2 qw = q[w];
-        r.x -= alpha * qw.x;
-        r.y -= alpha * qw.y;
+        r.x = fma(-alpha, qw.x, r.x);
+        r.y = fma(-alpha, qw.y, r.y);
         return r;
     };
-    for (int u = (int)r0 + sub; u < r1; u += kBlock / kRowLanes) {
+    for (int u = (int)r0 + threadIdx.x; u < r1; u += kBlock) {
         const double2 ru = residual(u);
         double2 o = bmv(Gd[u], bmv(Cinv[u], ru));
-        const double2 t = edge_sum<true>(ew, u, rowE[u], rowE[u + 1], lane,
-                                         [&](int e, int w) { return bmv(Go[e], bmv(Cinv[w], residual(w))); });
-        if (lane == 0) {
-            const double2 pu = p[u];
-            double2 xu = x[u];
-            xu.x += alpha * pu.x;
-            xu.y += alpha * pu.y;
-            x[u] = xu;
-            rNew[u] = ru;
-            out[u] = make_double2(o.x + t.x, o.y + t.y);
-            acc[1] += ru.x * ru.x + ru.y * ru.y;
-        }
+        const double2 pu = p[u];
+        double2 xu = x[u];
+        add_edges(ew, rowE[u], rowM[u],
+                  [&](int e, int w) { return bmv(Go[e], bmv(Cinv[w], residual(w))); }, o);
+        xu.x += alpha * pu.x;
+        xu.y += alpha * pu.y;
+        x[u] = xu;
+        rNew[u] = ru;
+        out[u] = o;
+        acc[1] += ru.x * ru.x + ru.y * ru.y;
     }
     block_sum<2>(acc);
     if (threadIdx.x == 0) {
@@ -525,6 +508,7 @@ enum { kGTPrecond = 0, kGTProbe = 1, kGTPlain = 2 };
 // y = G^T in (in = probe when MODE == kGTProbe); precond: z = C^-T y and r.z records
 template <int MODE>
 __global__ void __launch_bounds__(kBlock) k_gnn_apply_GT(int nV, const int* __restrict__ rowE,
+                                                         const int* __restrict__ rowM,
                                                          const int* __restrict__ ew, const int* __restrict__ rev,
                                                          const float4* __restrict__ Cinv,
                                                          const float4* __restrict__ Go, const float4* __restrict__ Gd,
@@ -535,23 +519,20 @@ __global__ void __launch_bounds__(kBlock) k_gnn_apply_GT(int nV, const int* __re
     if (stop && *stop) return;
     long r0, r1;
     chunk(nV, r0, r1);
-    const int sub = threadIdx.x / kRowLanes, lane = threadIdx.x % kRowLanes;
     double acc[1] = {0.0};
-    for (int u = (int)r0 + sub; u < r1; u += kBlock / kRowLanes) {
+    for (int u = (int)r0 + threadIdx.x; u < r1; u += kBlock) {
         const double2 iu = MODE == kGTProbe ? probe(u, seed, pj) : in[u];
         double2 y = bmtv(Gd[u], iu);
-        const double2 t = edge_sum<false>(ew, u, rowE[u], rowE[u + 1], lane, [&](int e, int w) {
+        add_edges(ew, rowM[u], rowE[u + 1], [&](int e, int w) {
             const double2 iw = MODE == kGTProbe ? probe(w, seed, pj) : in[w];
             return bmtv(Go[rev[e]], iw);
-        });
-        y.x += t.x;
-        y.y += t.y;
+        }, y);
         if (MODE == kGTPrecond) {
             y = bmtv(Cinv[u], y);
             const double2 rv = r[u];
-            if (lane == 0) acc[0] += rv.x * y.x + rv.y * y.y;
+            acc[0] += fma(rv.x, y.x, rv.y * y.y);
         }
-        if (lane == 0) out[u] = y;
+        out[u] = y;
     }
     if (MODE == kGTPrecond) {
         block_sum<1>(acc);
@@ -1053,7 +1034,7 @@ int Gnn::init(std::string& err)
 
 void Gnn::release_pattern()
 {
-    for (int** p : {&dRowE, &dEu, &dEw, &dRev, &dESlot, &dDiagPos}) dfree(*p);
+    for (int** p : {&dRowE, &dRowM, &dEu, &dEw, &dRev, &dESlot, &dDiagPos}) dfree(*p);
     dfree(dFixed);
     for (float** p : {&dCinv, &dLogTr, &dX, &dAhat, &dEf, &dGo, &dGd, &dDGo, &dDGd, &dDh, &dDa, &dDXe, &dPart}) dfree(*p);
     for (int l = 0; l <= kGnnLayers; ++l) dfree(dH[l]);
@@ -1112,6 +1093,9 @@ int Gnn::set_pattern(hipStream_t s, int nVin, const std::vector<int>& rowPtr, co
         }
         rev[e] = lo;
     }
+    std::vector<int> rowM(n);  // a row's edges into lower neighbours come first (found above: rows are sorted)
+    for (int u = 0; u < n; ++u)
+        rowM[u] = (int)(std::lower_bound(ew.begin() + rowE[u], ew.begin() + rowE[u + 1], u) - ew.begin());
     nV = n;
     E = nE;
     auto up = [&](int*& d, const std::vector<int>& h) -> int {
@@ -1120,7 +1104,7 @@ int Gnn::set_pattern(hipStream_t s, int nVin, const std::vector<int>& rowPtr, co
             return -1;
         return 0;
     };
-    int bad = up(dRowE, rowE) | up(dEu, eu) | up(dEw, ew) | up(dRev, rev) | up(dESlot, eslot) | up(dDiagPos, diagPos);
+    int bad = up(dRowE, rowE) | up(dRowM, rowM) | up(dEu, eu) | up(dEw, ew) | up(dRev, rev) | up(dESlot, eslot) | up(dDiagPos, diagPos);
     bad |= dalloc(dFixed, n);
     if (!bad) bad |= hipMemcpyAsync(dFixed, fixedMask.data(), n, hipMemcpyHostToDevice, s) != hipSuccess;
     const size_t nh = (size_t)n * kGnnH, mh = (size_t)std::max(nE, 1) * kGnnH;
@@ -1179,12 +1163,12 @@ void Gnn::forward(hipStream_t s, const void* vals, int vals32)
                        dTheta, dFixed, reinterpret_cast<float4*>(dGd));
 }
 
-int Gnn::rz_records() const { return row_blocks(nV); }
-int Gnn::update_records() const { return row_blocks(nV); }
+int Gnn::rz_records() const { return blocks_for(nV, kBlock); }
+int Gnn::update_records() const { return blocks_for(nV, kBlock); }
 
 void Gnn::apply(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop, const PcgStage*)
 {
-    hipLaunchKernelGGL(k_gnn_apply_G<kApplyPrecond>, dim3(row_blocks(nV)), dim3(kBlock), 0, s, nV, dRowE, dEw,
+    hipLaunchKernelGGL(k_gnn_apply_G<kApplyPrecond>, dim3(blocks_for(nV, kBlock)), dim3(kBlock), 0, s, nV, dRowE, dRowM, dEw,
                        reinterpret_cast<const float4*>(dCinv), reinterpret_cast<const float4*>(dGo),
                        reinterpret_cast<const float4*>(dGd), reinterpret_cast<const double2*>(r),
                        reinterpret_cast<double2*>(dTmp), 0.0, 0u, 0u, nullptr, stop);
@@ -1193,7 +1177,7 @@ void Gnn::apply(hipStream_t s, const double* r, double* z, double* rzPart, const
 
 void Gnn::apply_GT(hipStream_t s, const double* r, double* z, double* rzPart, const int* stop)
 {
-    hipLaunchKernelGGL(k_gnn_apply_GT<kGTPrecond>, dim3(row_blocks(nV)), dim3(kBlock), 0, s, nV, dRowE, dEw, dRev,
+    hipLaunchKernelGGL(k_gnn_apply_GT<kGTPrecond>, dim3(blocks_for(nV, kBlock)), dim3(kBlock), 0, s, nV, dRowE, dRowM, dEw, dRev,
                        reinterpret_cast<const float4*>(dCinv), reinterpret_cast<const float4*>(dGo),
                        reinterpret_cast<const float4*>(dGd), reinterpret_cast<const double2*>(dTmp),
                        reinterpret_cast<double2*>(z), reinterpret_cast<const double2*>(r), rzPart, 0u, 0u, stop);
@@ -1201,7 +1185,7 @@ void Gnn::apply_GT(hipStream_t s, const double* r, double* z, double* rzPart, co
 
 void Gnn::update_apply(hipStream_t s, const PcgUpdate& u, double* z, double* rzPart)
 {
-    hipLaunchKernelGGL(k_gnn_update_G, dim3(row_blocks(nV)), dim3(kBlock), 0, s, nV, dRowE, dEw,
+    hipLaunchKernelGGL(k_gnn_update_G, dim3(blocks_for(nV, kBlock)), dim3(kBlock), 0, s, nV, dRowE, dRowM, dEw,
                        reinterpret_cast<const float4*>(dCinv), reinterpret_cast<const float4*>(dGo),
                        reinterpret_cast<const float4*>(dGd), reinterpret_cast<const double2*>(u.p),
                        reinterpret_cast<const double2*>(u.q), reinterpret_cast<const double2*>(u.rOld),
@@ -1218,7 +1202,7 @@ void Gnn::zero_grad(hipStream_t s)
 
 void Gnn::loss_grad(hipStream_t s, int nProbes, unsigned seed, double* dLoss)
 {
-    const int g = row_blocks(nV);
+    const int g = blocks_for(nV, kBlock);
     const float4* Ci = reinterpret_cast<const float4*>(dCinv);
     const float4* Go = reinterpret_cast<const float4*>(dGo);
     const float4* Gd = reinterpret_cast<const float4*>(dGd);
@@ -1234,13 +1218,13 @@ void Gnn::loss_grad(hipStream_t s, int nProbes, unsigned seed, double* dLoss)
     hipLaunchKernelGGL(k_gnn_fill, dim3((4L * nV + kBlock - 1) / kBlock), dim3(kBlock), 0, s, 4L * nV, dDGd);
     const double norm = 1.0 / ((double)nProbes * 2.0 * nV);
     for (int j = 0; j < nProbes; ++j) {
-        hipLaunchKernelGGL(k_gnn_apply_GT<kGTProbe>, dim3(g), dim3(kBlock), 0, s, nV, dRowE, dEw, dRev, Ci, Go, Gd,
+        hipLaunchKernelGGL(k_gnn_apply_GT<kGTProbe>, dim3(g), dim3(kBlock), 0, s, nV, dRowE, dRowM, dEw, dRev, Ci, Go, Gd,
                            nullptr, y, nullptr, nullptr, seed, (unsigned)j, nullptr);
         hipLaunchKernelGGL(k_gnn_ahat, dim3(gv), dim3(kBlock), 0, s, nV, dRowE, dEw, Ah, y, t);
-        hipLaunchKernelGGL(k_gnn_apply_G<kApplyLoss>, dim3(g), dim3(kBlock), 0, s, nV, dRowE, dEw, Ci, Go, Gd, t, gs,
+        hipLaunchKernelGGL(k_gnn_apply_G<kApplyLoss>, dim3(g), dim3(kBlock), 0, s, nV, dRowE, dRowM, dEw, Ci, Go, Gd, t, gs,
                            norm, seed, (unsigned)j, dPartD, nullptr);
         hipLaunchKernelGGL(k_gnn_sum_to, dim3(1), dim3(kBlock), 0, s, dPartD, g, dLoss);
-        hipLaunchKernelGGL(k_gnn_apply_GT<kGTPlain>, dim3(g), dim3(kBlock), 0, s, nV, dRowE, dEw, dRev, Ci, Go, Gd, gs,
+        hipLaunchKernelGGL(k_gnn_apply_GT<kGTPlain>, dim3(g), dim3(kBlock), 0, s, nV, dRowE, dRowM, dEw, dRev, Ci, Go, Gd, gs,
                            tmp, nullptr, nullptr, 0u, 0u, nullptr);
         hipLaunchKernelGGL(k_gnn_ahat, dim3(gv), dim3(kBlock), 0, s, nV, dRowE, dEw, Ah, tmp, q);
         hipLaunchKernelGGL(k_gnn_dG, dim3(((long)E + nV + kBlock - 1) / kBlock), dim3(kBlock), 0, s, E, nV, dEu, dEw,

@@ -99,7 +99,8 @@ private:
     // parameters
     float *dTheta = nullptr, *dGrad = nullptr, *dAdamM = nullptr, *dAdamV = nullptr;
     // pattern maps
-    int *dRowE = nullptr, *dEu = nullptr, *dEw = nullptr, *dRev = nullptr, *dESlot = nullptr, *dDiagPos = nullptr;
+    int *dRowE = nullptr, *dRowM = nullptr;  // a row's first edge, and its first into an upper neighbour
+    int *dEu = nullptr, *dEw = nullptr, *dRev = nullptr, *dESlot = nullptr, *dDiagPos = nullptr;
     unsigned char* dFixed = nullptr;
     // features
     float *dCinv = nullptr, *dLogTr = nullptr, *dX = nullptr, *dAhat = nullptr, *dEf = nullptr;

@@ -965,12 +965,11 @@ __global__ void __launch_bounds__(kBlock) k_pcg_init(int nV, const double2* __re
 }
 
 int pcg_grid_update(int nV) { return std::max(1, std::min((nV + kBlock - 1) / kBlock, kPcgMaxGrid)); }
-// Workgroups of the PCG product: one row per kPcgLanes-lane group, at most kPcgMaxGrid, a multiple of 8 (XCD-contiguous
-// chunk order). Past the limit a workgroup makes several passes: up to 2,048 workgroups (one pass at 200k faces) cost
-// 6-9% there by their records, fewer with equal passes up to 2% more (405k faces).
+// Workgroups of the PCG product: one pass of kPcgRows rows per group, at most kPcgMaxGrid, a multiple of 8
+// (XCD-contiguous chunk order).
 int pcg_grid_spmv(int nV)
 {
-    constexpr int rows = kBlock / kPcgLanes;
+    constexpr int rows = (kBlock / kPcgLanes) * kPcgRows;
     const int g = std::max(1, std::min((nV + rows - 1) / rows, kPcgMaxGrid));
     return (g + 7) & ~7;
 }
@@ -1020,45 +1019,55 @@ __device__ __forceinline__ double2 row_apply(const int* __restrict__ rowPtr, con
 // records of p_new.q. beta needs the previous update's reductions, so the
 // row loads (blocks, gathered z and p_old) are issued first and the records
 // reduced while they are in flight; p_w = z_w + beta p_old_w is formed per
-// gathered entry. One row per kPcgLanes-lane group and pass, kPcgSlots blocks
-// per lane in flight (two rows a group with one block each, the second blocks
-// in a loop behind: 9.2 us an iteration at 2,116 rows and 10.1 at 100k faces
-// with the update, now 7.9 and 9.3; 8 lanes a row 7.8 and 10.0, 2 lanes of 4
-// blocks 8.2 and 9.6); workgroup b takes row chunk (b % 8) * (G / 8) + b / 8 so each XCD owns a contiguous eighth of
-// the rows (G = pcg_grid_spmv, a multiple of 8).
-template <typename V4>
-__global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restrict__ rowPtr,
-                                                     const int* __restrict__ colIdx,
-                                                     const V4* __restrict__ vals,
-                                                     const double2* __restrict__ z,
-                                                     const double2* __restrict__ pOld, double2* pNew, double2* q,
-                                                     const double* __restrict__ partRz, int nRz, int sRz,
-                                                     const double* __restrict__ partRr, int nRr, int sRr,
-                                                     double* partS, PcgCtrl* ctrl)
+// gathered entry. kPcgLanes lanes per row, kPcgSlots blocks per lane in flight;
+// workgroup b takes row chunk (b % 8) * (G / 8) + b / 8 so each XCD owns a
+// contiguous eighth of the rows (G = pcg_grid_spmv, a multiple of 8).
+// THREADS = 2 kBlock: one row per lane group and pass; kBlock: two. Both add
+// the same terms in the same order and rounding (fused products are written
+// out, the second half's p.q values go through LDS to the threads that add the
+// first half's): a solve of several hundred iterations stopped at a loose
+// tolerance ends elsewhere under any other rounding, by up to a few percent of
+// the map. Jacobi-PCG step, two rows / one row per group: 7.4 / 6.8 ms at 2,116
+// rows, 27.7 / 25.2 at 25k, 79.7 / 76.6 at 93k, 91.8 / 96.6 at 100k.
+template <typename V4, int THREADS>
+__global__ void __launch_bounds__(THREADS) k_pcg_spmv(int nV, const int* __restrict__ rowPtr,
+                                                      const int* __restrict__ colIdx,
+                                                      const V4* __restrict__ vals,
+                                                      const double2* __restrict__ z,
+                                                      const double2* __restrict__ pOld, double2* pNew, double2* q,
+                                                      const double* __restrict__ partRz, int nRz, int sRz,
+                                                      const double* __restrict__ partRr, int nRr, int sRr,
+                                                      double* partS, PcgCtrl* ctrl)
 {
     // The control record, the row pointers and the previous kernel's records are loaded together; the blocks follow
     // and are in flight while the records are reduced, the gathers come last: three dependent round trips in all. A
     // finished PCG is seen with the records (the loads before it are harmless, nothing is written).
     const int done = ctrl->done, it = ctrl->itNext, maxit = ctrl->maxit;
     const double bbKept = ctrl->bb, tol2 = ctrl->tol2, rzOld = ctrl->rzSlot[(it + 1) & 1];
-    constexpr int LANES = kPcgLanes, SLOTS = kPcgSlots, RPP = kBlock / LANES;
+    constexpr int LANES = kPcgLanes, SLOTS = kPcgSlots, RPP = kBlock / LANES, ROWS = kPcgRows * kBlock / THREADS;
+    static_assert(THREADS == kBlock || THREADS == kPcgRows * kBlock, "a pass is kPcgRows x RPP rows");
+    __shared__ double upper[2][THREADS > kBlock ? kBlock : 1];  // the second half's values of p.q, by the pass's parity
     const int G = gridDim.x;
     const int c = (nV + G - 1) / G;
     const int r0 = ((int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3)) * c, r1 = min(nV, r0 + c);
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
-    const int passes = max(1, (c + RPP - 1) / RPP);
-    const bool first = it == 0;
+    const int passes = max(1, (c + kPcgRows * RPP - 1) / (kPcgRows * RPP));
+    const bool first = it == 0, low = threadIdx.x < kBlock;
     double beta = 0.0;
     double acc[1] = {0.0};
     for (int pass = 0; pass < passes; ++pass) {
-        int w[SLOTS];
-        double4 a[SLOTS];
-        double2 gz[SLOTS], gp[SLOTS], oz, op;
-        double rec[2];
-        const int u = r0 + sub + pass * RPP;
-        const bool valid = u < r1;
-        const int kb = valid ? rowPtr[u] : 0, ke = valid ? rowPtr[u + 1] : 0;
-        if (pass == 0) {
+        int u[ROWS], kb[ROWS], ke[ROWS], w[ROWS][SLOTS];
+        double4 a[ROWS][SLOTS];
+        double2 gz[ROWS][SLOTS], gp[ROWS][SLOTS], oz[ROWS], op[ROWS];
+        double rec[2] = {0.0, 0.0};
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            u[r] = r0 + sub + (pass * kPcgRows + r) * RPP;
+            const bool valid = u[r] < r1;
+            kb[r] = valid ? rowPtr[u[r]] : 0;
+            ke[r] = valid ? rowPtr[u[r] + 1] : 0;
+        }
+        if (pass == 0 && low) {
             double one[1];
             sum_records<1>(partRz, nRz, sRz, one);
             rec[0] = one[0];
@@ -1066,14 +1075,16 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
             rec[1] = one[0];
         }
 #pragma unroll
-        for (int r = 0; r < SLOTS; ++r) {
-            const int k = kb + lane + r * LANES;
-            const bool has = k < ke;
-            const int kk = has ? k : 0;
-            const double4 av = to_double4(vals[kk]);
-            a[r] = has ? av : make_double4(0.0, 0.0, 0.0, 0.0);
-            w[r] = has ? colIdx[kk] : 0;
-        }
+        for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+            for (int i = 0; i < SLOTS; ++i) {
+                const int k = kb[r] + lane + i * LANES;
+                const bool has = k < ke[r];
+                const int kk = has ? k : 0;
+                const double4 av = to_double4(vals[kk]);
+                a[r][i] = has ? av : make_double4(0.0, 0.0, 0.0, 0.0);
+                w[r][i] = has ? colIdx[kk] : 0;
+            }
         if (pass == 0) {
             all_sum<2>(rec);
             const double rz = rec[0], rr = rec[1];
@@ -1095,45 +1106,67 @@ __global__ void __launch_bounds__(kBlock) k_pcg_spmv(int nV, const int* __restri
             if (conv || capped || indef) return;
             beta = first ? 0.0 : rz / rzOld;
         }
-        oz = op = make_double2(0.0, 0.0);
 #pragma unroll
-        for (int r = 0; r < SLOTS; ++r) {
-            gz[r] = z[w[r]];
-            gp[r] = first ? make_double2(0.0, 0.0) : pOld[w[r]];
-        }
-        if (lane == 0 && valid) {
-            oz = z[u];
-            if (!first) op = pOld[u];
-        }
-        double y[2] = {0.0, 0.0};
+        for (int r = 0; r < ROWS; ++r) {
+            oz[r] = op[r] = make_double2(0.0, 0.0);
 #pragma unroll
-        for (int r = 0; r < SLOTS; ++r) {
-            const double px = gz[r].x + beta * gp[r].x, py = gz[r].y + beta * gp[r].y;
-            y[0] += a[r].x * px + a[r].y * py;
-            y[1] += a[r].z * px + a[r].w * py;
-        }
-        for (int k = kb + lane + SLOTS * LANES; k < ke; k += LANES) {
-            const int wk = colIdx[k];
-            const double4 ak = to_double4(vals[k]);
-            const double2 zw = z[wk];
-            double px = zw.x, py = zw.y;
-            if (!first) {
-                const double2 pw = pOld[wk];
-                px += beta * pw.x;
-                py += beta * pw.y;
+            for (int i = 0; i < SLOTS; ++i) {
+                gz[r][i] = z[w[r][i]];
+                gp[r][i] = first ? make_double2(0.0, 0.0) : pOld[w[r][i]];
             }
-            y[0] += ak.x * px + ak.y * py;
-            y[1] += ak.z * px + ak.w * py;
+            if (lane == 0 && u[r] < r1) {
+                oz[r] = z[u[r]];
+                if (!first) op[r] = pOld[u[r]];
+            }
         }
-        group_sum<LANES, 2>(y);
-        if (lane == 0 && valid) {
-            const double2 pn = make_double2(oz.x + beta * op.x, oz.y + beta * op.y);
-            pNew[u] = pn;
-            q[u] = make_double2(y[0], y[1]);
-            acc[0] += pn.x * y[0] + pn.y * y[1];
+        double pq[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            double y[2];
+#pragma unroll
+            for (int i = 0; i < SLOTS; ++i) {
+                const double4& ai = a[r][i];
+                const double px = gz[r][i].x + beta * gp[r][i].x, py = gz[r][i].y + beta * gp[r][i].y;
+                if (i == 0) {
+                    y[0] = fma(ai.x, px, ai.y * py);
+                    y[1] = fma(ai.z, px, ai.w * py);
+                } else {
+                    y[0] += fma(ai.y, py, ai.x * px);
+                    y[1] += fma(ai.w, py, ai.z * px);
+                }
+            }
+            for (int k = kb[r] + lane + SLOTS * LANES; k < ke[r]; k += LANES) {
+                const int wk = colIdx[k];
+                const double4 ak = to_double4(vals[k]);
+                const double2 zw = z[wk];
+                double px = zw.x, py = zw.y;
+                if (!first) {
+                    const double2 pw = pOld[wk];
+                    px += beta * pw.x;
+                    py += beta * pw.y;
+                }
+                y[0] += fma(ak.y, py, ak.x * px);
+                y[1] += fma(ak.w, py, ak.z * px);
+            }
+            group_sum<LANES, 2>(y);
+            pq[r] = 0.0;
+            if (lane == 0 && u[r] < r1) {
+                const double2 pn = make_double2(oz[r].x + beta * op[r].x, oz[r].y + beta * op[r].y);
+                pNew[u[r]] = pn;
+                q[u[r]] = make_double2(y[0], y[1]);
+                pq[r] = fma(pn.x, y[0], pn.y * y[1]);
+            }
+        }
+        if constexpr (THREADS > kBlock) {
+            if (!low) upper[pass & 1][threadIdx.x - kBlock] = pq[0];
+            __syncthreads();
+            if (low) acc[0] = (acc[0] + pq[0]) + upper[pass & 1][threadIdx.x];
+        } else {
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) acc[0] += pq[r];
         }
     }
-    block_sum<1>(acc);
+    all_sum<1>(acc);
     if (threadIdx.x == 0) partS[blockIdx.x] = acc[0];
 }
 
@@ -1141,16 +1174,23 @@ void launch_pcg_spmv(hipStream_t s, int nV, const int* rowPtr, const int* colIdx
                      int vals32, const double* z, const double* pOld, double* pNew, double* q, const double* partRz,
                      int nRz, int sRz, const double* partRr, int nRr, int sRr, double* partS, PcgCtrl* ctrl)
 {
-    if (vals32)
-        hipLaunchKernelGGL(k_pcg_spmv<float4>, dim3(pcg_grid_spmv(nV)), dim3(kBlock), 0, s, nV, rowPtr, colIdx,
-                           reinterpret_cast<const float4*>(vals), reinterpret_cast<const double2*>(z),
-                           reinterpret_cast<const double2*>(pOld), reinterpret_cast<double2*>(pNew),
-                           reinterpret_cast<double2*>(q), partRz, nRz, sRz, partRr, nRr, sRr, partS, ctrl);
-    else
-        hipLaunchKernelGGL(k_pcg_spmv<double4>, dim3(pcg_grid_spmv(nV)), dim3(kBlock), 0, s, nV, rowPtr, colIdx,
-                           reinterpret_cast<const double4*>(vals), reinterpret_cast<const double2*>(z),
-                           reinterpret_cast<const double2*>(pOld), reinterpret_cast<double2*>(pNew),
-                           reinterpret_cast<double2*>(q), partRz, nRz, sRz, partRr, nRr, sRr, partS, ctrl);
+    const int G = pcg_grid_spmv(nV);
+    const auto launch = [&](auto kern, auto* v, int threads) {
+        hipLaunchKernelGGL(kern, dim3(G), dim3(threads), 0, s, nV, rowPtr, colIdx, v,
+                           reinterpret_cast<const double2*>(z), reinterpret_cast<const double2*>(pOld),
+                           reinterpret_cast<double2*>(pNew), reinterpret_cast<double2*>(q), partRz, nRz, sRz, partRr, nRr,
+                           sRr, partS, ctrl);
+    };
+    constexpr int wide = kPcgRows * kBlock;
+    const float4* v32 = reinterpret_cast<const float4*>(vals);
+    const double4* v64 = reinterpret_cast<const double4*>(vals);
+    if (G <= kPcgWideGrid) {
+        if (vals32) launch(k_pcg_spmv<float4, wide>, v32, wide);
+        else launch(k_pcg_spmv<double4, wide>, v64, wide);
+    } else {
+        if (vals32) launch(k_pcg_spmv<float4, kBlock>, v32, kBlock);
+        else launch(k_pcg_spmv<double4, kBlock>, v64, kBlock);
+    }
 }
 
 template <int MODE>

@@ -133,7 +133,12 @@ void launch_axpy_commit(hipStream_t s, long n, double alpha, const double* d, do
 // ---- PCG on the 2x2-block CSR ------------------------------------------------
 constexpr int kSpmvLanes = 8;     // lanes per block-row in the SpMV
 constexpr int kPcgLanes = 4;      // lanes per block-row in the PCG product
-constexpr int kPcgSlots = 2;      // blocks per lane in flight in the PCG product
+constexpr int kPcgRows = 2;       // passes of kBlock / kPcgLanes block rows that a workgroup of the PCG product makes at once
+constexpr int kPcgSlots = 2;      // blocks per lane and row in flight there
+// Workgroups up to which they are of 2 kBlock threads, one row per lane group: at 76 registers three of them fit a CU,
+// 768 the chip, and the rest would run as a second, nearly empty wave (792 workgroups: 96.6 ms a Jacobi step against 91.8
+// with kBlock threads; 728: 76.6 against 79.7). Of kBlock threads with two rows a group, 118 registers, four fit.
+constexpr int kPcgWideGrid = 768;
 constexpr int kPcgMaxGrid = 1024;  // workgroups of the PCG kernels (bounds the partial records)
 
 // Workgroups of the update/init kernels and of the SpMV kernel for nV rows.
