@@ -352,10 +352,6 @@ struct RowPass {
     }
 };
 
-// Whether a kernel is to return: `stop` (its flag's value) is set. first is the first value the kernel loads (a row
-// pointer, never negative), so that its load, and not only the flag's, comes before the branch: a kernel of a few
-// dependent round trips would otherwise spend one on the flag alone.
-__device__ __forceinline__ bool stopped(int stop, int first) { return (stop | (first & 0x80000000)) != 0; }
 __device__ __forceinline__ int stop_value(const int* __restrict__ stop) { return stop ? *stop : 0; }
 
 // Rows of this workgroup's chunk and the pass count (block-uniform).
@@ -1235,14 +1231,13 @@ __global__ void __launch_bounds__(kBlock) k_cheb_pre1(const int* __restrict__ st
     }
 }
 
-// Whether the PCG is over: its done flag, as this thread found it when the kernel began, or the residual within the
-// tolerance (then its control record is set as k_pcg_spmv sets it), from the threads' shares of the r.r records. Every
+// Whether the PCG is over: its done flag, as this thread found it when the kernel began (in a launch further on the
+// iteration number says so at once), or the residual within the tolerance (then its control record is set as k_pcg_spmv sets it), from the threads' shares of the r.r records. Every
 // workgroup sums them itself, in the same order. bb, the right-hand side's norm, is what the first residual's records
 // hold; k_pcg_spmv keeps it from then on. Workgroup 0 sets the flag while other workgroups may not have begun, so their
 // waves can find it differently: it is acted on only behind the barriers, where all of them find the same sum.
-__device__ __forceinline__ bool pcg_over(const PcgStage& st, int done, double (&acc)[1])
+__device__ __forceinline__ bool pcg_over(const PcgStage& st, int done, int it, double (&acc)[1])
 {
-    const int it = st.ctrl->itNext;
     const double bbKept = st.ctrl->bb, tol2 = st.ctrl->tol2;
     block_sum<1>(acc);
     __shared__ double sh;
@@ -1279,15 +1274,16 @@ __device__ __forceinline__ void cheb_step_rows(int blk, int G, int n, const int*
     const double c1 = rho1 * rho0, c2 = 2.0 * rho1 / cp.delta;
     const RowChunk rc = row_chunk<BS, NT>(n, blk, G);
     const int sub = threadIdx.x / LANES, lane = threadIdx.x % LANES;
+    const int it = CHECK ? st.ctrl->itNext : 0;
     double acc[1] = {0.0};
     for (int p = 0; p < rc.passes; ++p) {
         RowPass<T, BS, UNROLL> rp;
         rp.begin(rc.r0 + sub + p * UNROLL * RPP, RPP, rc.r1, rowPtr);
         double rr[1];
         if (CHECK && p == 0) sum_records<1>(st.partRr, st.nRr, st.sRr, rr);
-        if (!CHECK && p == 0 && stopped(stop, rp.kb[0])) return;
+        if (p == 0 && stopped(CHECK ? it < 0 : stop, rp.kb[0])) return;
         rp.blocks(colIdx, vals, lane);
-        if (CHECK && p == 0 && pcg_over(st, stop, rr)) return;
+        if (CHECK && p == 0 && pcg_over(st, stop, it, rr)) return;
         rp.gather(d);
         double Dm[UNROLL][BS * BS], dd[UNROLL][BS], xo[UNROLL][BS], rf[UNROLL][BS];
 #pragma unroll

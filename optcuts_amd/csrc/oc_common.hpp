@@ -191,6 +191,11 @@ __device__ __forceinline__ void sum_records(const double* __restrict__ part, int
     }
 }
 
+// Whether a kernel is to return: `stop` (its flag's value) is set. first is the first value the kernel loads (a row
+// pointer, never negative), so that its load, and not only the flag's, comes before the branch: a kernel of a few
+// dependent round trips would otherwise spend one on the flag alone.
+__device__ __forceinline__ bool stopped(int stop, int first) { return (stop | (first & 0x80000000)) != 0; }
+
 // Block reduction of NV independent compensated sums; result valid in thread 0.
 template <int NV>
 __device__ __forceinline__ void block_csum(CSum (&v)[NV])

@@ -460,20 +460,24 @@ __global__ void __launch_bounds__(kBlock) k_gnn_update_G(int nV, const int* __re
                                                          double2* out, const double* __restrict__ partS, int nPartS,
                                                          double* partU, PcgCtrl* ctrl)
 {
-    const int done = ctrl->done, it = ctrl->itCur;
+    const int it = ctrl->itCur;
     const double rzCur = ctrl->rzSlot[it & 1];
     long r0, r1;
     chunk(nV, r0, r1);
     double pq[1];
     sum_records<1>(partS, nPartS, 1, pq);
-    all_sum<1>(pq);
-    if (done) return;
-    if (!(pq[0] > 0.0)) {  // breakdown: A not positive definite along p
-        if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->done = 3;
+    if (it < 0) {  // over
+        if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->itNext = -1;
         return;
     }
+    all_sum<1>(pq);
+    const bool broke = !(pq[0] > 0.0);  // A not positive definite along p
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctrl->itNext = broke ? -1 : it + 1;
+        if (broke) ctrl->done = 3;
+    }
+    if (broke) return;
     const double alpha = rzCur / pq[0];
-    if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->itNext = it + 1;
     double acc[2] = {0.0, 0.0};
     const auto residual = [&](int w) {
         double2 r = rOld[w];

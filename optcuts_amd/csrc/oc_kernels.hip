@@ -1041,7 +1041,7 @@ __global__ void __launch_bounds__(THREADS) k_pcg_spmv(int nV, const int* __restr
 {
     // The control record, the row pointers and the previous kernel's records are loaded together; the blocks follow
     // and are in flight while the records are reduced, the gathers come last: three dependent round trips in all. A
-    // finished PCG is seen with the records (the loads before it are harmless, nothing is written).
+    // PCG that ended in an earlier iteration is seen with the row pointers, one that ended in this one with the records.
     const int done = ctrl->done, it = ctrl->itNext, maxit = ctrl->maxit;
     const double bbKept = ctrl->bb, tol2 = ctrl->tol2, rzOld = ctrl->rzSlot[(it + 1) & 1];
     constexpr int LANES = kPcgLanes, SLOTS = kPcgSlots, RPP = kBlock / LANES, ROWS = kPcgRows * kBlock / THREADS;
@@ -1074,6 +1074,10 @@ __global__ void __launch_bounds__(THREADS) k_pcg_spmv(int nV, const int* __restr
             sum_records<1>(partRr, nRr, sRr, one);
             rec[1] = one[0];
         }
+        if (pass == 0 && stopped(it < 0, kb[0])) {
+            if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->itCur = -1;
+            return;
+        }
 #pragma unroll
         for (int r = 0; r < ROWS; ++r)
 #pragma unroll
@@ -1092,18 +1096,19 @@ __global__ void __launch_bounds__(THREADS) k_pcg_spmv(int nV, const int* __restr
             const bool conv = (bb == 0.0) || (rr <= tol2 * bb);
             const bool capped = it >= maxit;
             const bool indef = !conv && !(rz > 0.0);  // preconditioner not positive definite on r
+            const bool over = done || conv || capped || indef;
+            if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->itCur = over ? -1 : it;
             if (done) return;
             if (blockIdx.x == 0 && threadIdx.x == 0) {
                 if (first) ctrl->bb = bb;
                 ctrl->rzSlot[it & 1] = rz;
                 ctrl->rr = rr;
                 ctrl->iter = it;
-                ctrl->itCur = it;
                 if (conv) ctrl->done = 1;
                 else if (indef) ctrl->done = 3;
                 else if (capped) ctrl->done = 2;
             }
-            if (conv || capped || indef) return;
+            if (over) return;
             beta = first ? 0.0 : rz / rzOld;
         }
 #pragma unroll
@@ -1203,7 +1208,7 @@ __global__ void __launch_bounds__(kBlock) k_pcg_update(int nV, const double2* __
 {
     constexpr bool APPLY_M = MODE == kPcgApplyM;
     // the thread's first row is loaded together with the records, before either is used
-    const int done = ctrl->done, it = ctrl->itCur;
+    const int it = ctrl->itCur;
     const double rzCur = ctrl->rzSlot[it & 1];
     const double theta = MODE >= kPcgFirst64 ? cheb_params(*first.lam).theta : 0.0;
     int r0, r1;
@@ -1220,14 +1225,18 @@ __global__ void __launch_bounds__(kBlock) k_pcg_update(int nV, const double2* __
     }
     double pq[1];
     sum_records<1>(partS, nPartS, 1, pq);
-    all_sum<1>(pq);
-    if (done) return;
-    if (!(pq[0] > 0.0)) {  // breakdown: A not positive definite along p
-        if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->done = 3;
+    if (it < 0) {  // over
+        if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->itNext = -1;
         return;
     }
+    all_sum<1>(pq);
+    const bool broke = !(pq[0] > 0.0);  // A not positive definite along p
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctrl->itNext = broke ? -1 : it + 1;
+        if (broke) ctrl->done = 3;
+    }
+    if (broke) return;
     const double alpha = rzCur / pq[0];
-    if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->itNext = it + 1;
     double acc[2] = {0.0, 0.0};
     while (v < r1) {
         xv.x += alpha * pv.x;

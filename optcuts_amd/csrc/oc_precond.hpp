@@ -10,8 +10,10 @@ namespace oc {
 // k_pcg_init sets itNext = 0; k_pcg_spmv reads itNext and records it in itCur
 // (and iter); k_pcg_update (or update_apply()) reads itCur and sets itNext = itCur + 1. A field is
 // written by workgroup 0 alone and read by later kernels; only done is read in the launch that may set it
-// (k_pcg_spmv, k_pcg_update, update_apply(), a multigrid's first kernel): there each thread reads it first and acts on
-// it behind the record sums, from which every workgroup takes the same decision as the one that set it.
+// (k_pcg_spmv, a multigrid's first kernel): there each thread reads it first and acts on it behind the record sums, from
+// which every workgroup takes the same decision as the one that set it. Once the PCG is over, k_pcg_spmv leaves -1 in
+// itCur and the update -1 in itNext, each written by one kernel and read by the other: launches queued past the end
+// return on it at once (behind the sums, such an iteration of Jacobi-PCG at 200k faces took 9 us instead of 5).
 struct PcgCtrl {
     double bb, tol2, rr, pad0;
     double rzSlot[2];
