@@ -94,11 +94,11 @@ def cheb_levels(ctx, reps=50):
 # same counters read the known size of a plain 512 MiB device copy. Summaries with commands:
 # profiles/pmc_traffic_200k.md (disc) and profiles/pmc_traffic_tori_200k.md (fused tori).
 TRAFFIC = {
-    ("disc_200k", "k_lanczos_fine"): (2.0 * 17072.8 + 3188.8) * 1024,
-    ("disc_200k", "k_pcg_spmv"): (2.0 * 14334.2 + 3209.3) * 1024,
+    ("disc_200k", "k_lanczos_fine"): (2.0 * 16672.9 + 3189.9) * 1024,
+    ("disc_200k", "k_pcg_spmv"): (2.0 * 14121.9 + 3165.4) * 1024,
     # three fused tori, chosen form: mean over multigrid levels 1-3 of the Chebyshev step; the PCG product
-    ("tori_200k", "k_cheb_step3"): ((2.0 * 6745.6 + 840.5) + (2.0 * 654.8 + 50.4) + (2.0 * 60.7 + 2.3)) / 3.0 * 1024,
-    ("tori_200k", "k_pcg_spmv"): (2.0 * 21640.6 + 3458.0) * 1024,
+    ("tori_200k", "k_cheb_step3"): ((2.0 * 6611.6 + 280.2) + (2.0 * 637.7 + 16.8) + (2.0 * 67.2 + 0.8)) / 3.0 * 1024,
+    ("tori_200k", "k_pcg_spmv"): (2.0 * 17713.7 + 3458.0) * 1024,
 }
 
 FALLBACK_NAMES = {1: "retry_safe_amg", 2: "jacobi", 3: "truncated", 4: "retry_fp64_elements", 5: "jacobi_direct",
@@ -518,7 +518,7 @@ def headline(ctx, args, targets, fast):
     # the dominant kernel of the chosen form on this workload: the V-cycle's Chebyshev step on the coarse
     # (3x3-block) levels; per level and over those levels (each launched twice per V-cycle)
     per_level, agg = cheb_levels(ctx)
-    roofline = {"bound": "hbm", "kernel": "k_cheb_step<double,3,false> (V-cycle Chebyshev step, coarse levels; "
+    roofline = {"bound": "hbm", "kernel": "k_cheb_step<double,3,1> (V-cycle Chebyshev step, coarse levels; "
                                           "aggregate over the levels, which the V-cycle launches equally often)",
                 "achieved": agg["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": agg["achieved"] / HBM_PEAK_GBS, "traffic": TRAFFIC.get((args.workload, "k_cheb_step3")),
@@ -526,6 +526,56 @@ def headline(ctx, args, targets, fast):
                 "avg_launch_ms": agg["avg_launch_ms"], "per_level": per_level, "pcg_spmv": spmv,
                 "element_pass": element, "assembly": assembly}
     return head, w, roofline
+
+
+def brief(x):
+    """A number to five significant digits."""
+    return float("%.5g" % x) if isinstance(x, float) else x
+
+
+def form_summary(r):
+    """The figures of one form that its readers compare: rate, step time, PCG iterations, fallbacks that occurred and
+    the time to the target energy."""
+    if not isinstance(r, dict):
+        return r
+    out = {k: brief(r[k]) for k in ("newton_iters_per_s", "step_ms_median", "pcg_iters_median", "pcg_iters_per_newton")
+           if r.get(k) is not None}
+    out["fallbacks"] = {k: v for k, v in r.get("pcg_fallbacks", {}).items() if v}
+    t = r.get("time_to_E_SD_1e-6")
+    if t:
+        out["s_to_target"] = brief(t.get("time_to_target_s", t.get("seconds")))
+        out["its_to_target"] = t.get("iterations_to_target", t.get("newton_iterations"))
+    return out
+
+
+def workload_summary(w):
+    return {k: form_summary(r) for k, r in w["forms"].items()} if isinstance(w, dict) and "forms" in w else None
+
+
+def roofline_summary(r):
+    keep = ("bound", "kernel", "achieved", "peak", "unit", "frac", "traffic", "algorithmic_bytes_per_launch",
+            "avg_launch_ms")
+    out = {k: brief(r[k]) for k in keep if k in r}
+    for k in ("pcg_spmv", "element_pass", "assembly"):
+        if k in r:
+            out[k] = {q: brief(r[k][q]) for q in ("achieved", "frac", "avg_launch_ms")}
+    return out
+
+
+def report(out):
+    """The whole result as one line on stderr, and on stdout the JSON line: the same figures without the per-phase and
+    per-level ones, short enough to be kept whole wherever the output's end is."""
+    print("bench: detail " + json.dumps(out), file=sys.stderr, flush=True)
+    line = dict(out)
+    line["headline"] = workload_summary(out["headline"])
+    line["secondary"] = {k: workload_summary(w) for k, w in out["secondary"].items()
+                         if workload_summary(w) is not None}
+    charts = out["secondary"].get("batched_charts")
+    if charts:
+        line["secondary"]["batched_charts"] = {k: brief(v) for k, v in charts.items() if isinstance(v, (int, float))}
+    if out.get("roofline"):
+        line["roofline"] = roofline_summary(out["roofline"])
+    print(json.dumps(line), flush=True)
 
 
 def main():
@@ -658,8 +708,8 @@ def main():
         net.close()
     ctx.close()
     if head is None or "chosen" not in head["forms"]:
-        print(json.dumps({"metric": METRIC, "value": None, "unit": "Newton iters/s", "n_gpus": 1,
-                          "headline": head, "secondary": secondary}), flush=True)
+        report({"metric": METRIC, "value": None, "unit": "Newton iters/s", "n_gpus": 1, "headline": head,
+                "secondary": secondary})
         return
     chosen = head["forms"]["chosen"]
     out = {
@@ -689,7 +739,7 @@ def main():
     if not args.no_cpu_baseline:
         print("bench: cpu baseline", file=sys.stderr, flush=True)
         out["cpu_baseline"] = cpu_baseline_closed(w)
-    print(json.dumps(out), flush=True)
+    report(out)
 
 
 if __name__ == "__main__":
