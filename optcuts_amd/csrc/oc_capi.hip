@@ -601,6 +601,8 @@ int run_pcg(oc_ctx* c, BlockPattern& P, const double* b, double relTol, int maxI
             h = c->pcgMail[slot ^ 1];
         }
     }
+    // what was queued past the end is over before the caller goes on: it may free or capture anew what those launches name
+    if (h.done) OC_HIP(c, hipStreamSynchronize(c->stream));
     while (!h.done) {
         OC_HIP(c, queue(it, batch));
         it += batch;

@@ -3,13 +3,16 @@ previous solve's count; launches past the end must cost little, and a long batch
 at 5e-3 on the 200k-face disc: 1,013 iterations on the first step, 4 on the second, whose time then is that of the
 launches past the end. Time of the second step over that of the first: 0.55 where all 1,014 iterations were queued and
 each launch summed the records before it saw the end, 0.24 where it saw the end first, 0.09 with the batch in parts.
-The iterate does not depend on how many are queued: the same from single launches."""
+The iterate does not depend on how many are queued: the same from single launches.
+A solve that breaks down early in such a batch goes on with another preconditioner in the same step, whose graphs take
+the place of those just queued: FP32 element terms at 0.99 (0.9999) of the first inversion sum to an indefinite matrix,
+after some 50 to 150 iterations of the 400 to 550 that the step before gives as the batch."""
 import time
 
 import numpy as np
 import pytest
 
-from optcuts_amd import capi
+from optcuts_amd import capi, learned
 from optcuts_amd.meshgen import height_field_disc
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +43,37 @@ def test_iterations_past_the_end_are_cheap():
             c.close()
     assert best < 0.18
     assert all(np.array_equal(m, maps[0]) for m in maps[1:])
+
+
+@pytest.mark.parametrize("precond,push", [(capi.PRECOND_LEARNED, 0.99), (capi.PRECOND_LEARNED, 0.9999),
+                                          (capi.PRECOND_IC0, 0.9999)])
+def test_breakdown_early_in_a_long_batch(precond, push):
+    V, F, UV = height_field_disc(80, seed=1)
+    d = np.random.default_rng(5).standard_normal(UV.shape)
+    d[0] = 0.0
+    maps = []
+    for graphs in (True, False):
+        c, net = capi.Context(0), None
+        try:
+            c.pcg_graphs(graphs)
+            c.set_mesh(V, F, fixed=(0,))
+            c.set_uv(UV)
+            if precond == capi.PRECOND_LEARNED:
+                net = capi.Gnn(0)
+                net.set_params(np.load(learned.DEFAULT_WEIGHTS))
+                c.set_learned(net)
+            c.newton_init(a0=1.0, rel_gl2_tol=1e-30, allow_edec_rel_tol=False, precond=precond, pcg_rel_tol=1e-8,
+                          pcg_max_iter=20000, precision=capi.PRECISION_MIXED)
+            first, _ = c.newton_step()
+            c.set_uv(c.get_uv() + push * c.init_step_size(d, 1e9) * d)
+            second, _ = c.newton_step()
+            print(graphs, first["pcg_iters"], second["pcg_iters_first"], second["pcg_iters"], second["pcg_fallback"],
+                  flush=True)
+            assert first["pcg_fallback"] == 0 and second["pcg_fallback"] != 0
+            assert second["pcg_iters_first"] < first["pcg_iters"] / 2
+            maps.append(c.get_uv())
+        finally:
+            c.close()
+            if net is not None:
+                net.close()
+    assert np.array_equal(maps[0], maps[1])
